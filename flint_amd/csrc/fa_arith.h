@@ -24,6 +24,30 @@ FA_DEV double fa_mulmod(double a, double b, double n, double ninv)
     return __builtin_fma(-q, n, h) + l;
 }
 
+// Global memory at a uniform base plus a 32-bit byte offset per lane.  The
+// base stays in scalar registers (the empty asm keeps it from being folded
+// into the lane offsets), so stepping it by a constant costs no vector
+// instruction; and a pointer read from memory is still known to be global
+// (a generic access would count as an LDS access too).
+typedef __attribute__((address_space(1))) char fa_gbyte;
+
+template <class T>
+FA_DEV T fa_ld(const void* base, uint32_t off)
+{
+    typedef __attribute__((address_space(1))) T gT;
+    const fa_gbyte* b = (const fa_gbyte*)base;
+    asm("" : "+s"(b));
+    return *(const gT*)(b + off);
+}
+
+FA_DEV void fa_st(double* base, uint32_t off, double v)
+{
+    typedef __attribute__((address_space(1))) double gT;
+    fa_gbyte* b = (fa_gbyte*)base;
+    asm("" : "+s"(b));
+    *(gT*)(b + off) = v;
+}
+
 // a mod n in [-n/2, n/2] (machine_vectors.h:646-651 reduce_to_pm1n)
 FA_DEV double fa_reduce_pm1n(double a, double n, double ninv)
 {

@@ -19,37 +19,92 @@
 
 #define PADX(p) ((p) + ((p) >> 4))
 
+// Value ranges of the column passes, in units of n.  A mulmod of operands
+// whose product is below P n^2 lands in 1/2 + P'/4, P' the power of two at or
+// above P (P <= 4, fa_mulmod_satisfies_bounds); twiddles are at most 1/2.
+//  - a radix-4 layer that reduces a0 takes values up to 6.4 (its largest
+//    product is (6.4 + 1.5) / 2 < 4) to at most 1/2 + 1.5 + 1.5 = 3.5;
+//  - one that does not takes 3.5 to 3.5 + 1 + 1.5 = 6, below 2^53.
+// So a radix-16 stage reduces in its first layer only, and its outputs, up to
+// 6, may enter the next stage or the row pass.
+// forward radix-4 without the reduction of a0
+FA_DEV void fa_fwd4_nr(double& a0, double& a1, double& a2, double& a3, double W2, double W,
+                       double IW, double n, double ninv)
+{
+    const double t2 = fa_mulmod(a2, W2, n, ninv);
+    const double t3 = fa_mulmod(a3, W2, n, ninv);
+    const double u0 = a0 + t2, u2 = a0 - t2;
+    const double v1 = fa_mulmod(a1 + t3, W, n, ninv);
+    const double v3 = fa_mulmod(a1 - t3, IW, n, ninv);
+    a0 = u0 + v1;
+    a1 = u0 - v1;
+    a2 = u2 + v3;
+    a3 = u2 - v3;
+}
+
+// forward radix-4 of block 0, whose roots are 1, 1 and I = w2[1] (one product
+// of the four is left).  HZ: a2 = a3 = 0 and a0, a1 up to 2.75 (imported
+// values): outputs up to 5.5.  Otherwise all four are reduced first: outputs
+// up to 2.
+template <bool HZ>
+FA_DEV void fa_fwd4_b0(double& a0, double& a1, double& a2, double& a3, double I, double n,
+                       double ninv)
+{
+    if (HZ) {
+        const double t = fa_mulmod(a1, I, n, ninv);
+        const double x = a0, y = a1;
+        a0 = x + y;
+        a1 = x - y;
+        a2 = x + t;
+        a3 = x - t;
+    } else {
+        const double x0 = fa_reduce_pm1n(a0, n, ninv), x1 = fa_reduce_pm1n(a1, n, ninv);
+        const double x2 = fa_reduce_pm1n(a2, n, ninv), x3 = fa_reduce_pm1n(a3, n, ninv);
+        const double t = fa_mulmod(x1 - x3, I, n, ninv);
+        const double s = x0 + x2, d = x0 - x2, e = x1 + x3;
+        a0 = s + e;
+        a1 = s - e;
+        a2 = d + t;
+        a3 = d - t;
+    }
+}
+
 // radix-16 = four levels from the block Q at level m0 (fft_small.h block
 // convention): t[0..2] = (w2[Q], w2[2Q], w2[2Q+1]), t[3+3j..5+3j] the same
-// for Q' = 4Q + j
+// for Q' = 4Q + j.  R2: the second layer reduces too (outputs up to 3).
+template <bool R2 = true>
 FA_DEV void fa_fwd16(double* x, const double* t, double n, double ninv)
 {
 #pragma unroll
     for (int k = 0; k < 4; k++) fa_fwd4(x[k], x[k + 4], x[k + 8], x[k + 12], t[0], t[1], t[2], n, ninv);
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-        fa_fwd4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3], t[3 + 3 * j], t[4 + 3 * j],
-                t[5 + 3 * j], n, ninv);
+    for (int j = 0; j < 4; j++) {
+        if (R2)
+            fa_fwd4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3], t[3 + 3 * j], t[4 + 3 * j],
+                    t[5 + 3 * j], n, ninv);
+        else
+            fa_fwd4_nr(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3], t[3 + 3 * j],
+                       t[4 + 3 * j], t[5 + 3 * j], n, ninv);
+    }
 }
 
-// fa_fwd16 for inputs whose upper half x[8..15] is zero: the first radix-4
-// layer needs only the products by x[k+4]
-FA_DEV void fa_fwd16_hz(double* x, const double* t, double n, double ninv)
+// the first four levels of a column (block 0, roots w2[0..7]) on imported
+// values (up to 2.75).  HZ: x[8..15] are zero.  17 products instead of 32;
+// outputs up to 6.25 (HZ: the block j = 1 sees 5.5 and reduces, the blocks 2
+// and 3 see 3.75 and give 3.75 + 1 + 1.5).
+template <bool HZ>
+FA_DEV void fa_fwd16_b0(double* x, const double* __restrict__ w, double n, double ninv)
 {
+    const double I = w[1];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const double a0 = fa_reduce_pm1n(x[k], n, ninv);
-        const double v1 = fa_mulmod(x[k + 4], t[1], n, ninv);
-        const double v3 = fa_mulmod(x[k + 4], t[2], n, ninv);
-        x[k] = a0 + v1;
-        x[k + 4] = a0 - v1;
-        x[k + 8] = a0 + v3;
-        x[k + 12] = a0 - v3;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-        fa_fwd4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3], t[3 + 3 * j], t[4 + 3 * j],
-                t[5 + 3 * j], n, ninv);
+    for (int k = 0; k < 4; k++) fa_fwd4_b0<HZ>(x[k], x[k + 4], x[k + 8], x[k + 12], I, n, ninv);
+    fa_fwd4_b0<false>(x[0], x[1], x[2], x[3], I, n, ninv);
+    if (HZ)
+        fa_fwd4(x[4], x[5], x[6], x[7], I, w[2], w[3], n, ninv);
+    else
+        fa_fwd4_nr(x[4], x[5], x[6], x[7], I, w[2], w[3], n, ninv);
+    fa_fwd4_nr(x[8], x[9], x[10], x[11], w[2], w[4], w[5], n, ninv);
+    fa_fwd4_nr(x[12], x[13], x[14], x[15], w[3], w[6], w[7], n, ninv);
 }
 
 FA_DEV void fa_inv16(double* x, const double* t, double n, double ninv)
@@ -62,15 +117,43 @@ FA_DEV void fa_inv16(double* x, const double* t, double n, double ninv)
     for (int k = 0; k < 4; k++) fa_inv4(x[k], x[k + 4], x[k + 8], x[k + 12], t[0], t[1], t[2], n, ninv);
 }
 
+// inverse radix-4 of block 0 (roots 1, 1 and IV = w2inv[1]) on values up to
+// 2.  LAST: the column's last levels, whose outputs (up to 8, below 2^53) are
+// reduced by whoever reads them; otherwise outputs stay below 2.
+template <bool LAST>
+FA_DEV void fa_inv4_b0(double& b0, double& b1, double& b2, double& b3, double IV, double n,
+                       double ninv)
+{
+    const double u = b0 + b1, v = b2 + b3;
+    const double s2 = fa_mulmod(b2 - b3, IV, n, ninv);
+    const double s1 = LAST ? b0 - b1 : fa_reduce_pm1n(b0 - b1, n, ninv);
+    b0 = LAST ? u + v : fa_reduce_pm1n(u + v, n, ninv);
+    b2 = LAST ? u - v : fa_reduce_pm1n(u - v, n, ninv);
+    b1 = s1 + s2;
+    b3 = s1 - s2;
+}
+
+// the last four inverse levels of a column (block 0)
+FA_DEV void fa_inv16_b0(double* x, const double* __restrict__ w, double n, double ninv)
+{
+    const double IV = w[1];
+    fa_inv4_b0<false>(x[0], x[1], x[2], x[3], IV, n, ninv);
+    fa_inv4(x[4], x[5], x[6], x[7], IV, w[2], w[3], n, ninv);
+    fa_inv4(x[8], x[9], x[10], x[11], w[2], w[4], w[5], n, ninv);
+    fa_inv4(x[12], x[13], x[14], x[15], w[3], w[6], w[7], n, ninv);
+#pragma unroll
+    for (int k = 0; k < 4; k++) fa_inv4_b0<true>(x[k], x[k + 4], x[k + 8], x[k + 12], IV, n, ninv);
+}
+
 // twiddles of block Q from a table indexed by global block number
-FA_DEV void fa_tw16(const double* __restrict__ w, uint64_t Q, double* t)
+FA_DEV void fa_tw16(const double* __restrict__ w, uint32_t Q, double* t)
 {
     t[0] = w[Q];
     t[1] = w[2 * Q];
     t[2] = w[2 * Q + 1];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        uint64_t Qp = 4 * Q + j;
+        uint32_t Qp = 4 * Q + j;
         t[3 + 3 * j] = w[Qp];
         t[4 + 3 * j] = w[2 * Qp];
         t[5 + 3 * j] = w[2 * Qp + 1];
@@ -323,7 +406,7 @@ FA_DEV void fa_row_conv_tile_lr(double* __restrict__ arow, const double* __restr
         const double* src = z ? arow : brow;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int k = 0; k < 16; k++) v[k] = src[t + 256 * k];
+        for (int k = 0; k < 16; k++) v[k] = fa_ld<double>(src + 256 * k, t * 8);
         fa_fwd16_rowtab(v, tab, 0, 0, n, ninv);
 #pragma unroll
         for (int k = 0; k < 16; k++) xch[PADX(t + 256 * k)] = v[k];
@@ -364,7 +447,7 @@ FA_DEV void fa_row_conv_tile_lr(double* __restrict__ arow, const double* __restr
     for (int k = 0; k < 16; k++) x[k] = xch[PADX(t + 256 * k)];
     fa_inv16_rowtab(x, tab, 0, 0, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) arow[t + 256 * k] = x[k];
+    for (int k = 0; k < 16; k++) fa_st(arow + 256 * k, t * 8, x[k]);
 }
 
 template <bool SQR>
@@ -486,12 +569,24 @@ __global__ void __launch_bounds__(256) fa_k_row_conv16(double* __restrict__ A,
 //     (b << (D1 - m0)) + i0 + (k << (D1 - m0 - 4)),  tc = b * 2^(D1-m0-4) + i0.
 // ---------------------------------------------------------------------------
 
+// A tile is CPW columns of NT threads together: 256 threads up to D1 = 8, so
+// that four tiles of at most 34.8 KB of LDS share a CU and one's loads and
+// stores run beside another's arithmetic, and a product of 2^13..2^20 points
+// gives four times the workgroups of a 1024-thread tile.  CPW never falls
+// below 16 columns (a 128-byte line) there; D1 = 9 keeps 16 with 512 threads,
+// D1 = 10 takes 8 (two tiles per CU), D1 = 11 eight with 1024 threads.
+// Measured against 1024-thread tiles whose import tested every chunk: the
+// column passes of a 65,536-limb square (2^17 points) 13.3 + 8.6 -> 7.8 +
+// 5.1 us; 64 batched fmpz products, 2^20 points, 913 + 389 -> 761 + 346 us (a
+// copy's rate, 5.3 TB/s, in the inverse pass; the forward pass waits on the
+// reads of its limb rows, without which it takes 363 us).
 template <int D1>
 struct col_geom {
     static constexpr int R = (D1 >= 4) ? (D1 % 4) : D1;   // levels of the partial stage
     static constexpr int NS = (D1 >= 4) ? (D1 / 4) : 0;   // radix-16 stages
     static constexpr int TPC = (D1 >= 4) ? (1 << (D1 - 4)) : 1;
-    static constexpr int CPW = 1024 / TPC;
+    static constexpr int CPW = D1 <= 8 ? 256 / TPC : D1 == 9 ? 16 : D1 <= 11 ? 8 : 4;
+    static constexpr int NT = CPW * TPC;                  // threads
     static constexpr int LEN = 1 << D1;
     static constexpr int PLEN = LEN + LEN / 16;
     static constexpr int NEL = (D1 >= 4) ? 16 : (1 << D1);  // elements per thread
@@ -512,82 +607,128 @@ struct col_geom {
         if (D1 < 4) return 0;
         return tc >> (D1 - m0(j) - 4);
     }
+    // LDS row of element k: PADX(pos(j, tc, k)) = PADX(pos(j, tc, 0)) + a
+    // constant (the bits of k do not meet those of pos(j, tc, 0))
+    static FA_DEV int lrow(int j, int tc, int k)
+    {
+        const int d = k << (D1 - m0(j) - 4);
+        return PADX(pos(j, tc, 0)) + PADX(d);
+    }
 };
 
-// the first r (< 4) levels of a radix-16 group, block Q: level 0 pairs
-// (k, k+8), level 1 (k, k+4), level 2 (k, k+2)
-FA_DEV void fa_fwd16_partial(double* x, int r, const double* __restrict__ w, uint64_t Q,
-                             double n, double ninv)
+// the first R (1..3) levels of a radix-16 group of a column (block 0, roots
+// w2[0..3]) on imported values: level 0 pairs (k, k+8), level 1 (k, k+4),
+// level 2 (k, k+2).  HZ: x[8..15] are zero.  Outputs up to 5.5.
+template <int R, bool HZ>
+FA_DEV void fa_fwd16_partial(double* x, const double* __restrict__ w, double n, double ninv)
 {
-    if (r == 1) {
-        const double W = w[Q];
+    if (R == 1) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) fa_fwd2(x[k], x[k + 8], W, n, ninv);
+        for (int k = 0; k < 8; k++) {
+            if (HZ) {
+                x[k + 8] = x[k];
+            } else {
+                const double a = fa_reduce_pm1n(x[k], n, ninv);
+                const double b = fa_reduce_pm1n(x[k + 8], n, ninv);
+                x[k] = a + b;
+                x[k + 8] = a - b;
+            }
+        }
         return;
     }
-    const double W2 = w[Q], W = w[2 * Q], IW = w[2 * Q + 1];
+    const double I = w[1];
 #pragma unroll
-    for (int k = 0; k < 4; k++) fa_fwd4(x[k], x[k + 4], x[k + 8], x[k + 12], W2, W, IW, n, ninv);
-    if (r == 3) {
+    for (int k = 0; k < 4; k++) fa_fwd4_b0<HZ>(x[k], x[k + 4], x[k + 8], x[k + 12], I, n, ninv);
+    if (R == 3) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const double Wj = w[4 * Q + j];
+        for (int i = 0; i < 2; i++) {
+            const double a = fa_reduce_pm1n(x[i], n, ninv), b = fa_reduce_pm1n(x[i + 2], n, ninv);
+            x[i] = a + b;
+            x[i + 2] = a - b;
+        }
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            const double Wj = w[j];
             fa_fwd2(x[4 * j], x[4 * j + 2], Wj, n, ninv);
             fa_fwd2(x[4 * j + 1], x[4 * j + 3], Wj, n, ninv);
         }
     }
 }
 
-FA_DEV void fa_inv16_partial(double* x, int r, const double* __restrict__ wi, uint64_t Q,
-                             double n, double ninv)
+// the last R levels of a column's inverse (block 0), on values up to 2;
+// outputs up to 8
+template <int R>
+FA_DEV void fa_inv16_partial(double* x, const double* __restrict__ wi, double n, double ninv)
 {
-    if (r == 1) {
-        const double V = wi[Q];
+    if (R == 1) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) fa_inv2(x[k], x[k + 8], V, n, ninv);
+        for (int k = 0; k < 8; k++) {
+            const double a = x[k], b = x[k + 8];
+            x[k] = a + b;
+            x[k + 8] = a - b;
+        }
         return;
     }
-    if (r == 3) {
+    if (R == 3) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const double Vj = wi[4 * Q + j];
+        for (int i = 0; i < 2; i++) {
+            const double a = x[i], b = x[i + 2];
+            x[i] = fa_reduce_pm1n(a + b, n, ninv);
+            x[i + 2] = fa_reduce_pm1n(a - b, n, ninv);
+        }
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            const double Vj = wi[j];
             fa_inv2(x[4 * j], x[4 * j + 2], Vj, n, ninv);
             fa_inv2(x[4 * j + 1], x[4 * j + 3], Vj, n, ninv);
         }
     }
-    const double V2 = wi[Q], V = wi[2 * Q], IV = wi[2 * Q + 1];
+    const double IV = wi[1];
 #pragma unroll
-    for (int k = 0; k < 4; k++) fa_inv4(x[k], x[k + 4], x[k + 8], x[k + 12], V2, V, IV, n, ninv);
+    for (int k = 0; k < 4; k++) fa_inv4_b0<true>(x[k], x[k + 4], x[k + 8], x[k + 12], IV, n, ninv);
 }
 
-// a whole column of 2^D1 <= 8 points in one thread (block 0 at level 0)
-template <int D1>
+// a whole column of 2^D1 <= 8 points in one thread.  HZ: the upper half of x
+// is zero
+template <int D1, bool HZ>
 FA_DEV void fa_fwd_small_col(double* x, const double* __restrict__ w, double n, double ninv)
 {
+    if constexpr (D1 == 1) {
+        const double a = x[0], b = HZ ? 0.0 : x[1];
+        x[0] = a + b;
+        x[1] = a - b;
+    } else if constexpr (D1 == 2) {
+        fa_fwd4_b0<HZ>(x[0], x[1], x[2], x[3], w[1], n, ninv);
+    } else {
+        const double I = w[1];
 #pragma unroll
-    for (int m = 0; m < D1; m++) {
-        const int half = 1 << (D1 - m - 1);
+        for (int i = 0; i < 2; i++) fa_fwd4_b0<HZ>(x[i], x[i + 2], x[i + 4], x[i + 6], I, n, ninv);
+        const double a = fa_reduce_pm1n(x[0], n, ninv), b = fa_reduce_pm1n(x[1], n, ninv);
+        x[0] = a + b;
+        x[1] = a - b;
 #pragma unroll
-        for (int q = 0; q < (1 << m); q++) {
-            const double W = w[q];
-#pragma unroll
-            for (int i = 0; i < half; i++) fa_fwd2(x[2 * half * q + i], x[2 * half * q + i + half], W, n, ninv);
-        }
+        for (int j = 1; j < 4; j++) fa_fwd2(x[2 * j], x[2 * j + 1], w[j], n, ninv);
     }
 }
 
 template <int D1>
 FA_DEV void fa_inv_small_col(double* x, const double* __restrict__ wi, double n, double ninv)
 {
+    if constexpr (D1 == 1) {
+        const double a = x[0], b = x[1];
+        x[0] = a + b;
+        x[1] = a - b;
+    } else if constexpr (D1 == 2) {
+        fa_inv4_b0<true>(x[0], x[1], x[2], x[3], wi[1], n, ninv);
+    } else {
+        const double a = x[0], b = x[1];
+        x[0] = fa_reduce_pm1n(a + b, n, ninv);
+        x[1] = fa_reduce_pm1n(a - b, n, ninv);
 #pragma unroll
-    for (int m = D1 - 1; m >= 0; m--) {
-        const int half = 1 << (D1 - m - 1);
+        for (int j = 1; j < 4; j++) fa_inv2(x[2 * j], x[2 * j + 1], wi[j], n, ninv);
 #pragma unroll
-        for (int q = 0; q < (1 << m); q++) {
-            const double V = wi[q];
-#pragma unroll
-            for (int i = 0; i < half; i++) fa_inv2(x[2 * half * q + i], x[2 * half * q + i + half], V, n, ninv);
-        }
+        for (int i = 0; i < 2; i++)
+            fa_inv4_b0<true>(x[i], x[i + 2], x[i + 4], x[i + 6], wi[1], n, ninv);
     }
 }
 
@@ -599,50 +740,64 @@ FA_DEV unsigned fa_xcd_linear()
     return (bid & 7) * (nb >> 3) + (bid >> 3);
 }
 
+// import and first stage (or, below 16 points, the whole column)
+template <int D1, int KIND, bool HZ>
+FA_DEV void fa_col_fwd_first(double* x, const fa_operand& op, uint32_t e0, double n, double ninv,
+                             const double* __restrict__ w2, const double* __restrict__ pow2)
+{
+    typedef col_geom<D1> G;
+    constexpr uint32_t step = 1u << (FA_ROW_LG + (D1 >= 4 ? D1 - 4 : 0));
+    fa_import_column<(HZ ? G::NEL / 2 : G::NEL), KIND>(x, op, e0, step, pow2, n, ninv);
+    if (HZ) {
+#pragma unroll
+        for (int k = G::NEL / 2; k < G::NEL; k++) x[k] = 0.0;
+    }
+    if constexpr (D1 < 4) fa_fwd_small_col<D1, HZ>(x, w2, n, ninv);
+    else if constexpr (G::R > 0) fa_fwd16_partial<G::R, HZ>(x, w2, n, ninv);
+    else fa_fwd16_b0<HZ>(x, w2, n, ninv);
+}
+
 // first D1 levels of column group g (CPW columns) of one residue array:
 // import, forward, store.  lds holds CPW * PLEN doubles.
 template <int D1, int KIND>
-FA_DEV void fa_col_fwd_tile(const fa_operand& op, double* __restrict__ dst, int d2, int g,
+FA_DEV void fa_col_fwd_tile(const fa_operand& op, double* __restrict__ dst, int g,
                             double n, double ninv, const double* __restrict__ w2,
                             const double* __restrict__ pow2, double* lds, int trows)
 {
     typedef col_geom<D1> G;
     const int c = threadIdx.x % G::CPW, tc = threadIdx.x / G::CPW;
-    const uint64_t col = (uint64_t)g * G::CPW + c;
+    const uint32_t col = (uint32_t)(g * G::CPW + c);
     double* my = lds + c;   // column c of the interleaved LDS rows
     double x[16], tw[15];
+    // the upper half of every column zero: the usual case of a product's
+    // operands, each at most half the transform length
+    const uint32_t e0 = ((uint32_t)G::pos(0, tc, 0) << FA_ROW_LG) + col;
+    if (fa_operand_fits(op, 1u << (D1 + FA_ROW_LG - 1)))
+        fa_col_fwd_first<D1, KIND, true>(x, op, e0, n, ninv, w2, pow2);
+    else
+        fa_col_fwd_first<D1, KIND, false>(x, op, e0, n, ninv, w2, pow2);
+    if constexpr (D1 >= 4) {
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++)
-        x[k] = fa_operand_value_k<KIND>(op, ((uint64_t)G::pos(0, tc, k) << d2) + col, pow2, n, ninv);
-    if (D1 < 4) {
-        fa_fwd_small_col<(D1 < 4 ? D1 : 1)>(x, w2, n, ninv);
-    } else {
+        for (int j = 1; j < G::NSTAGE; j++) {
+            // each position of a stage layout belongs to one thread: a
+            // single barrier separates stage j-1's stores from stage j's loads
 #pragma unroll
-        for (int j = 0; j < G::NSTAGE; j++) {
-            if (j > 0) {
-                // each position of a stage layout belongs to one thread: a
-                // single barrier separates stage j-1's stores from stage j's loads
+            for (int k = 0; k < 16; k++) my[G::lrow(j - 1, tc, k) * G::CPW] = x[k];
+            __syncthreads();
 #pragma unroll
-                for (int k = 0; k < 16; k++) my[PADX(G::pos(j - 1, tc, k)) * G::CPW] = x[k];
-                __syncthreads();
-#pragma unroll
-                for (int k = 0; k < 16; k++) x[k] = my[PADX(G::pos(j, tc, k)) * G::CPW];
-            }
-            if (G::R > 0 && j == 0) {
-                fa_fwd16_partial(x, G::R, w2, (uint64_t)G::block(0, tc), n, ninv);
-            } else {
-                fa_tw16(w2, (uint64_t)G::block(j, tc), tw);
-                fa_fwd16(x, tw, n, ninv);
-            }
+            for (int k = 0; k < 16; k++) x[k] = my[G::lrow(j, tc, k) * G::CPW];
+            fa_tw16(w2, (uint32_t)G::block(j, tc), tw);
+            fa_fwd16<false>(x, tw, n, ninv);
         }
     }
     const int jl = (D1 < 4) ? 0 : G::NSTAGE - 1;
     // rows at or past trows are not read by a truncated product
+    const int r0 = G::pos(jl, tc, 0);
+    const uint32_t at = ((uint32_t)r0 * FA_ROW_PITCH + col) * 8u;
+    // (the last stage of a column ends at level D1: consecutive rows)
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++) {
-        const int row = G::pos(jl, tc, k);
-        if (row < trows) dst[(uint64_t)row * FA_ROW_PITCH + col] = x[k];
-    }
+    for (int k = 0; k < G::NEL; k++)
+        if (r0 + k < trows) fa_st(dst + k * FA_ROW_PITCH, at, x[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -667,8 +822,8 @@ FA_DEV void fa_col_fwd_tile(const fa_operand& op, double* __restrict__ dst, int 
 // ---------------------------------------------------------------------------
 template <int D1>
 struct trunc_geom {
-    static constexpr int CPW = (D1 >= 4) ? (1024 >> (D1 - 4)) : 1024;
-    static constexpr int LG = (D1 >= 4) ? (14 - D1) : 10;   // log2 CPW
+    static constexpr int CPW = col_geom<D1>::CPW;
+    static constexpr int LG = __builtin_ctz(CPW);
     static constexpr int LDS = CPW << D1;
 };
 
@@ -759,69 +914,86 @@ FA_DEV void fa_col_inv_trunc_tile(double* __restrict__ dst, int g, int t, double
 }
 
 template <int D1>
-FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int d2, int g, double n, double ninv,
+FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int g, double n, double ninv,
                             const double* __restrict__ wi, double* lds)
 {
     typedef col_geom<D1> G;
     const int c = threadIdx.x % G::CPW, tc = threadIdx.x / G::CPW;
-    const uint64_t col = (uint64_t)g * G::CPW + c;
+    const uint32_t col = (uint32_t)(g * G::CPW + c);
     double* my = lds + c;   // column c of the interleaved LDS rows
     double x[16], tw[15];
     const int jl = (D1 < 4) ? 0 : G::NSTAGE - 1;
+    const uint32_t in = ((uint32_t)G::pos(jl, tc, 0) * FA_ROW_PITCH + col) * 8u;
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++) x[k] = dst[(uint64_t)G::pos(jl, tc, k) * FA_ROW_PITCH + col];
-    if (D1 < 4) {
-        fa_inv_small_col<(D1 < 4 ? D1 : 1)>(x, wi, n, ninv);
+    for (int k = 0; k < G::NEL; k++) x[k] = fa_ld<double>(dst + k * FA_ROW_PITCH, in);
+    if constexpr (D1 < 4) {
+        fa_inv_small_col<D1>(x, wi, n, ninv);
     } else {
 #pragma unroll
         for (int j = G::NSTAGE - 1; j >= 0; j--) {
             if (j < G::NSTAGE - 1) {
 #pragma unroll
-                for (int k = 0; k < 16; k++) my[PADX(G::pos(j + 1, tc, k)) * G::CPW] = x[k];
+                for (int k = 0; k < 16; k++) my[G::lrow(j + 1, tc, k) * G::CPW] = x[k];
                 __syncthreads();
 #pragma unroll
-                for (int k = 0; k < 16; k++) x[k] = my[PADX(G::pos(j, tc, k)) * G::CPW];
+                for (int k = 0; k < 16; k++) x[k] = my[G::lrow(j, tc, k) * G::CPW];
             }
-            if (G::R > 0 && j == 0) {
-                fa_inv16_partial(x, G::R, wi, (uint64_t)G::block(0, tc), n, ninv);
-            } else {
-                fa_tw16(wi, (uint64_t)G::block(j, tc), tw);
+            if (j > 0) {
+                fa_tw16(wi, (uint32_t)G::block(j, tc), tw);
                 fa_inv16(x, tw, n, ninv);
+            } else if constexpr (G::R > 0) {
+                fa_inv16_partial<G::R>(x, wi, n, ninv);
+            } else {
+                fa_inv16_b0(x, wi, n, ninv);
             }
         }
     }
+    const uint32_t out = ((uint32_t)G::pos(0, tc, 0) * FA_ROW_PITCH + col) * 8u;
+    constexpr uint32_t rs = (D1 < 4 ? 1u : 1u << (D1 - 4)) * FA_ROW_PITCH;
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++) dst[(uint64_t)G::pos(0, tc, k) * FA_ROW_PITCH + col] = x[k];
+    for (int k = 0; k < G::NEL; k++) fa_st(dst + k * rs, out, x[k]);
 }
 
-// work index L -> (prime i, column group g, operand z) with the two column
-// groups of one 128-byte line (g = 2h, 2h + 1) adjacent, then the primes,
-// then the line pairs: concurrent workgroups of an XCD share every line they
-// read or write, and the primes of one group follow each other (the limb
-// reads of the import are shared too).  ngroups is even.
+// Work order of the column passes: blocks of `lines` adjacent column groups
+// (512 columns), for each block the primes, then the next block, then the
+// other operand.  Concurrent workgroups of an XCD then read long runs of each
+// limb row (row starts are own * 4096 bytes apart, so a narrow block of
+// columns would fall on few HBM channels), and the primes of a block find its
+// limbs in L2.  64 batched fmpz products, 2^20 points, forward: 1015 us with
+// blocks of 64 columns, 906 with 512, 928 with 1024, 954 with all 4096.  At
+// 2^24 points one tile fills a CU and the limb rows of a block no longer fit
+// L2 beside the tiles, so the blocks there are 64 columns (the whole product
+// 2.33 ms; 2.48 with 512).
+#define FA_COL_BLOCK 512
+#ifndef FA_COLW_BLOCK
+#define FA_COLW_BLOCK 64
+#endif
+template <int CPW, int BLOCK>
+constexpr int fa_col_block() { return BLOCK / CPW < 2 ? 2 : BLOCK / CPW; }
+
+// work index L -> (prime i, column group g, operand z)
+template <int CPW, int BLOCK = FA_COL_BLOCK>
 FA_DEV void fa_col_split(unsigned L, int np, int ngroups, int* i, int* g, int* z)
 {
-    const int lo = L & 1;
-    const unsigned L2 = L >> 1;
+    constexpr unsigned GB = fa_col_block<CPW, BLOCK>();
+    const unsigned lo = L % GB, L2 = L / GB;
     *i = (int)(L2 % (unsigned)np);
     const unsigned rest = L2 / (unsigned)np;
-    const int half = ngroups >> 1;
-    *g = 2 * (int)(rest % (unsigned)half) + lo;
-    *z = (int)(rest / (unsigned)half);
+    const unsigned blocks = (unsigned)ngroups / GB;
+    *g = (int)(rest % blocks * GB + lo);
+    *z = (int)(rest / blocks);
 }
 
 template <int D1, int KIND>
-__global__ void __launch_bounds__(1024) fa_k_col_fwd16(fa_operand a, fa_operand b, int d2,
-                                                       double* __restrict__ A,
-                                                       double* __restrict__ B, uint64_t stride,
-                                                       fa_prime_set S, int np, int ngroups,
-                                                       int nops, int trows)
+__global__ void __launch_bounds__(col_geom<D1>::NT, 4)
+fa_k_col_fwd16(fa_operand a, fa_operand b, double* __restrict__ A, double* __restrict__ B,
+               uint64_t stride, fa_prime_set S, int np, int ngroups, int nops, int trows)
 {
     __shared__ double lds[col_geom<D1>::LDS];
     int i, g, z;
-    fa_col_split(fa_xcd_linear(), np, ngroups, &i, &g, &z);
+    fa_col_split<col_geom<D1>::CPW>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
     if (z >= nops) return;
-    fa_col_fwd_tile<D1, KIND>(z ? b : a, (z ? B : A) + (uint64_t)i * stride, d2, g, S.p[i],
+    fa_col_fwd_tile<D1, KIND>(z ? b : a, (z ? B : A) + (uint64_t)i * stride, g, S.p[i],
                               S.pinv[i], S.w2[i], S.pow2[i], lds, trows);
 }
 
@@ -834,19 +1006,19 @@ constexpr int fa_col_inv_lds()
 // trows < 2^D1: the truncated inverse (the tile groups of both kernels
 // cover the same 4096 columns: CPW columns per group)
 template <int D1>
-__global__ void __launch_bounds__(1024) fa_k_col_inv16(double* __restrict__ A, int d2,
-                                                       uint64_t stride, fa_prime_set S, int np,
-                                                       int ngroups, int trows)
+__global__ void __launch_bounds__(col_geom<D1>::NT, 4)
+fa_k_col_inv16(double* __restrict__ A, uint64_t stride, fa_prime_set S, int np, int ngroups,
+               int trows)
 {
     __shared__ double lds[fa_col_inv_lds<D1>()];
     int i, g, z;
-    fa_col_split(fa_xcd_linear(), np, ngroups, &i, &g, &z);
+    fa_col_split<col_geom<D1>::CPW>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
     if (z >= 1) return;
     if (trows < (1 << D1))
         fa_col_inv_trunc_tile<D1>(A + (uint64_t)i * stride, g, trows, S.p[i], S.pinv[i], S.w2[i],
                                   S.w2inv[i], lds);
     else
-        fa_col_inv_tile<D1>(A + (uint64_t)i * stride, d2, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
+        fa_col_inv_tile<D1>(A + (uint64_t)i * stride, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -885,7 +1057,7 @@ FA_DEV void fa_col_fwdw_rest(double* x0, double* x1, double* __restrict__ dst, i
                              double ninv, const double* __restrict__ w2, double* lds)
 {
     const int c = threadIdx.x & (C - 1), u = threadIdx.x / C;
-    const uint64_t col = (uint64_t)g * C + c;
+    const uint32_t col = (uint32_t)(g * C + c);
     double tw[15];
     // exchange 0 -> 1 in two halves
     double y0[16], y1[16];
@@ -906,10 +1078,10 @@ FA_DEV void fa_col_fwdw_rest(double* x0, double* x1, double* __restrict__ dst, i
         __syncthreads();
     }
     // stage 1: levels 4..7, block tc >> 4
-    fa_tw16(w2, (uint64_t)(u >> 4), tw);
-    fa_fwd16(y0, tw, n, ninv);
-    fa_tw16(w2, (uint64_t)((u + 128) >> 4), tw);
-    fa_fwd16(y1, tw, n, ninv);
+    fa_tw16(w2, (uint32_t)(u >> 4), tw);
+    fa_fwd16<false>(y0, tw, n, ninv);
+    fa_tw16(w2, (uint32_t)((u + 128) >> 4), tw);
+    fa_fwd16<false>(y1, tw, n, ninv);
     // exchange 1 -> 2, half H holds y_H entirely
 #pragma unroll
     for (int H = 0; H < 2; H++) {
@@ -926,111 +1098,73 @@ FA_DEV void fa_col_fwdw_rest(double* x0, double* x1, double* __restrict__ dst, i
         if (H == 0) __syncthreads();
     }
     // stage 2: levels 8..11, block tc
-    fa_tw16(w2, (uint64_t)u, tw);
-    fa_fwd16(x0, tw, n, ninv);
-    fa_tw16(w2, (uint64_t)(u + 128), tw);
-    fa_fwd16(x1, tw, n, ninv);
+    fa_tw16(w2, (uint32_t)u, tw);
+    fa_fwd16<false>(x0, tw, n, ninv);
+    fa_tw16(w2, (uint32_t)(u + 128), tw);
+    fa_fwd16<false>(x1, tw, n, ninv);
+    // one lane offset, the row steps in the (scalar) base
+    const uint32_t at = ((uint32_t)(16 * u) * FA_ROW_PITCH + col) * 8u;
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        dst[(uint64_t)(16 * u + k) * FA_ROW_PITCH + col] = x0[k];
-        dst[(uint64_t)(16 * (u + 128) + k) * FA_ROW_PITCH + col] = x1[k];
+        fa_st(dst + k * FA_ROW_PITCH, at, x0[k]);
+        fa_st(dst + (16 * 128 + k) * FA_ROW_PITCH, at, x1[k]);
     }
+}
+
+// import and levels 0..3 of the two groups of a thread
+template <int KIND, int OWN, bool HZ>
+FA_DEV void fa_col_fwdw_first(double* x0, double* x1, const fa_operand& op, uint32_t e0, double n,
+                              double ninv, const double* __restrict__ w2,
+                              const double* __restrict__ pow2)
+{
+    constexpr uint32_t step = 256u << FA_ROW_LG, half = 128u << FA_ROW_LG;
+    constexpr int NEL = HZ ? 8 : 16;
+    fa_import_column<NEL, KIND, OWN>(x0, op, e0, step, pow2, n, ninv);
+    fa_import_column<NEL, KIND, OWN>(x1, op, e0 + half, step, pow2, n, ninv);
+    if (HZ) {
+#pragma unroll
+        for (int k = 8; k < 16; k++) x0[k] = x1[k] = 0.0;
+    }
+    fa_fwd16_b0<HZ>(x0, w2, n, ninv);
+    fa_fwd16_b0<HZ>(x1, w2, n, ninv);
 }
 
 // OWN > 0: the chunk width in bytes of a byte-aligned import, fixed at
 // compile time (the import's word masks and partial sums fold away)
 template <int C, int KIND, int OWN = 0>
-FA_DEV void fa_col_fwdw_tile(const fa_operand& op, double* __restrict__ dst, int d2, int g,
-                             double n, double ninv, const double* __restrict__ w2,
+FA_DEV void fa_col_fwdw_tile(const fa_operand& op, double* __restrict__ dst, int g, double n,
+                             double ninv, const double* __restrict__ w2,
                              const double* __restrict__ pow2, double* lds)
 {
     const int c = threadIdx.x & (C - 1), u = threadIdx.x / C;
-    const uint64_t col = (uint64_t)g * C + c;
-    double x0[16], x1[16], tw[15];
-    // rows >= 2048 (elements >= 2^(d2+11)) all zero: the usual case of a
-    // product's operands, each at most half the transform length
-    const bool hz = fa_operand_len(op) <= (UINT64_C(1) << (d2 + 11));
-    fa_tw16(w2, 0, tw);
-    if constexpr (KIND == FA_PACK_MPN8) {
-        // byte-aligned chunks: when the last chunk a lane reads (row u + 128
-        // + 256 (nk - 1)) has its 32-byte window inside the limbs for every
-        // lane of the wave, all of the wave's chunks do; they are then read
-        // without per-chunk checks, at offsets stepping by 256 rows.  Each
-        // import path runs the rest of the tile on its own (no join of
-        // differently allocated registers).
-        const int own = OWN ? OWN : op.bits >> 3;
-        const uint64_t last = ((uint64_t)(u + 128 + 256 * (hz ? 7 : 15)) << d2) + col;
-        if (__all(((last * (uint64_t)own) & ~UINT64_C(3)) + 32 <= op.n * 8)) {
-            const char* base = (const char*)op.src;
-            const uint64_t B0 = (((uint64_t)u << d2) + col) * (uint64_t)own;
-            const uint64_t step = ((uint64_t)256 << d2) * (uint64_t)own;
-            const uint64_t half = ((uint64_t)128 << d2) * (uint64_t)own;
-            if (hz) {
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    x0[k] = fa_chunk_residue8_in(base, B0 + k * step, own, pow2, n, ninv);
-                    x1[k] = fa_chunk_residue8_in(base, B0 + half + k * step, own, pow2, n, ninv);
-                }
-#pragma unroll
-                for (int k = 8; k < 16; k++) x0[k] = x1[k] = 0.0;
-                fa_fwd16_hz(x0, tw, n, ninv);
-                fa_fwd16_hz(x1, tw, n, ninv);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 16; k++) {
-                    x0[k] = fa_chunk_residue8_in(base, B0 + k * step, own, pow2, n, ninv);
-                    x1[k] = fa_chunk_residue8_in(base, B0 + half + k * step, own, pow2, n, ninv);
-                }
-                fa_fwd16(x0, tw, n, ninv);
-                fa_fwd16(x1, tw, n, ninv);
-            }
-            fa_col_fwdw_rest<C>(x0, x1, dst, g, n, ninv, w2, lds);
-            return;
-        }
-    }
-    if (hz) {
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            x0[k] = fa_operand_value_k<KIND>(op, ((uint64_t)(u + 256 * k) << d2) + col, pow2, n,
-                                             ninv);
-            x1[k] = fa_operand_value_k<KIND>(op, ((uint64_t)(u + 128 + 256 * k) << d2) + col,
-                                             pow2, n, ninv);
-        }
-#pragma unroll
-        for (int k = 8; k < 16; k++) x0[k] = x1[k] = 0.0;
-        // stage 0: levels 0..3, block 0
-        fa_fwd16_hz(x0, tw, n, ninv);
-        fa_fwd16_hz(x1, tw, n, ninv);
-    } else {
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-            x0[k] = fa_operand_value_k<KIND>(op, ((uint64_t)(u + 256 * k) << d2) + col, pow2, n,
-                                             ninv);
-            x1[k] = fa_operand_value_k<KIND>(op, ((uint64_t)(u + 128 + 256 * k) << d2) + col,
-                                             pow2, n, ninv);
-        }
-        fa_fwd16(x0, tw, n, ninv);
-        fa_fwd16(x1, tw, n, ninv);
-    }
+    const uint32_t e0 = ((uint32_t)u << FA_ROW_LG) + (uint32_t)(g * C + c);
+    double x0[16], x1[16];
+    // rows >= 2048 (elements >= 2^23) all zero: the usual case of a product's
+    // operands, each at most half the transform length
+    if (fa_operand_fits(op, 1u << (FA_ROW_LG + 11)))
+        fa_col_fwdw_first<KIND, OWN, true>(x0, x1, op, e0, n, ninv, w2, pow2);
+    else
+        fa_col_fwdw_first<KIND, OWN, false>(x0, x1, op, e0, n, ninv, w2, pow2);
     fa_col_fwdw_rest<C>(x0, x1, dst, g, n, ninv, w2, lds);
 }
 
 template <int C>
-FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int d2, int g, double n, double ninv,
+FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int g, double n, double ninv,
                              const double* __restrict__ wi, double* lds)
 {
     const int c = threadIdx.x & (C - 1), u = threadIdx.x / C;
-    const uint64_t col = (uint64_t)g * C + c;
+    const uint32_t col = (uint32_t)(g * C + c);
     double x0[16], x1[16], tw[15];
+    const uint32_t in = ((uint32_t)(16 * u) * FA_ROW_PITCH + col) * 8u;
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        x0[k] = dst[(uint64_t)(16 * u + k) * FA_ROW_PITCH + col];
-        x1[k] = dst[(uint64_t)(16 * (u + 128) + k) * FA_ROW_PITCH + col];
+        x0[k] = fa_ld<double>(dst + k * FA_ROW_PITCH, in);
+        x1[k] = fa_ld<double>(dst + (16 * 128 + k) * FA_ROW_PITCH, in);
     }
     // stage 2 (levels 11..8), block tc
-    fa_tw16(wi, (uint64_t)u, tw);
+    fa_tw16(wi, (uint32_t)u, tw);
     fa_inv16(x0, tw, n, ninv);
-    fa_tw16(wi, (uint64_t)(u + 128), tw);
+    fa_tw16(wi, (uint32_t)(u + 128), tw);
     fa_inv16(x1, tw, n, ninv);
     // exchange 2 -> 1, half H holds x_H entirely
     double y0[16], y1[16];
@@ -1048,9 +1182,9 @@ FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int d2, int g, double n, 
         __syncthreads();
     }
     // stage 1 (levels 7..4), block tc >> 4
-    fa_tw16(wi, (uint64_t)(u >> 4), tw);
+    fa_tw16(wi, (uint32_t)(u >> 4), tw);
     fa_inv16(y0, tw, n, ninv);
-    fa_tw16(wi, (uint64_t)((u + 128) >> 4), tw);
+    fa_tw16(wi, (uint32_t)((u + 128) >> 4), tw);
     fa_inv16(y1, tw, n, ninv);
     // exchange 1 -> 0: half H receives stage-1 group 128H + u and returns
     // elements 8H .. 8H+7 of both stage-0 groups
@@ -1069,47 +1203,32 @@ FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int d2, int g, double n, 
         if (H == 0) __syncthreads();
     }
     // stage 0 (levels 3..0), block 0
-    fa_tw16(wi, 0, tw);
-    fa_inv16(x0, tw, n, ninv);
-    fa_inv16(x1, tw, n, ninv);
+    fa_inv16_b0(x0, wi, n, ninv);
+    fa_inv16_b0(x1, wi, n, ninv);
+    const uint32_t out = ((uint32_t)u * FA_ROW_PITCH + col) * 8u;
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        dst[(uint64_t)(u + 256 * k) * FA_ROW_PITCH + col] = x0[k];
-        dst[(uint64_t)(u + 128 + 256 * k) * FA_ROW_PITCH + col] = x1[k];
+        fa_st(dst + 256 * k * FA_ROW_PITCH, out, x0[k]);
+        fa_st(dst + (128 + 256 * k) * FA_ROW_PITCH, out, x1[k]);
     }
 }
 
 template <int KIND>
-FA_DEV void fa_col_fwd8_tile(const fa_operand& op, double* __restrict__ dst, int d2, int g,
+FA_DEV void fa_col_fwd8_tile(const fa_operand& op, double* __restrict__ dst, int g,
                              double n, double ninv, const double* __restrict__ w2,
                              const double* __restrict__ pow2, double* lds)
 {
-    fa_col_fwdw_tile<8, KIND>(op, dst, d2, g, n, ninv, w2, pow2, lds);
+    fa_col_fwdw_tile<8, KIND>(op, dst, g, n, ninv, w2, pow2, lds);
 }
 
-FA_DEV void fa_col_inv8_tile(double* __restrict__ dst, int d2, int g, double n, double ninv,
+FA_DEV void fa_col_inv8_tile(double* __restrict__ dst, int g, double n, double ninv,
                              const double* __restrict__ wi, double* lds)
 {
-    fa_col_invw_tile<8>(dst, d2, g, n, ninv, wi, lds);
-}
-
-// work index L -> (prime i, column group g, operand z) with the 16/C column
-// groups of one 128-byte line adjacent, as fa_col_split does for two
-template <int C>
-FA_DEV void fa_colw_split(unsigned L, int np, int ngroups, int* i, int* g, int* z)
-{
-    constexpr int LG = (C == 8) ? 1 : 2;   // log2(16 / C)
-    const int lo = L & ((1 << LG) - 1);
-    const unsigned L2 = L >> LG;
-    *i = (int)(L2 % (unsigned)np);
-    const unsigned rest = L2 / (unsigned)np;
-    const int lines = ngroups >> LG;
-    *g = ((int)(rest % (unsigned)lines) << LG) + lo;
-    *z = (int)(rest / (unsigned)lines);
+    fa_col_invw_tile<8>(dst, g, n, ninv, wi, lds);
 }
 
 template <int C, int KIND, int OWN = 0>
-__global__ void __launch_bounds__(128 * C) fa_k_col_fwd16w(fa_operand a, fa_operand b, int d2,
+__global__ void __launch_bounds__(128 * C) fa_k_col_fwd16w(fa_operand a, fa_operand b,
                                                            double* __restrict__ A,
                                                            double* __restrict__ B,
                                                            uint64_t stride, fa_prime_set S,
@@ -1117,22 +1236,22 @@ __global__ void __launch_bounds__(128 * C) fa_k_col_fwd16w(fa_operand a, fa_oper
 {
     __shared__ double lds[FA_CW_LDS(C)];
     int i, g, z;
-    fa_colw_split<C>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
+    fa_col_split<C, FA_COLW_BLOCK>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
     if (z >= nops) return;
-    fa_col_fwdw_tile<C, KIND, OWN>(z ? b : a, (z ? B : A) + (uint64_t)i * stride, d2, g, S.p[i],
-                              S.pinv[i], S.w2[i], S.pow2[i], lds);
+    fa_col_fwdw_tile<C, KIND, OWN>(z ? b : a, (z ? B : A) + (uint64_t)i * stride, g, S.p[i],
+                                    S.pinv[i], S.w2[i], S.pow2[i], lds);
 }
 
 template <int C>
-__global__ void __launch_bounds__(128 * C) fa_k_col_inv16w(double* __restrict__ A, int d2,
+__global__ void __launch_bounds__(128 * C) fa_k_col_inv16w(double* __restrict__ A,
                                                            uint64_t stride, fa_prime_set S,
                                                            int np, int ngroups)
 {
     __shared__ double lds[FA_CW_LDS(C)];
     int i, g, z;
-    fa_colw_split<C>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
+    fa_col_split<C, FA_COLW_BLOCK>(fa_xcd_linear(), np, ngroups, &i, &g, &z);
     if (z >= 1) return;
-    fa_col_invw_tile<C>(A + (uint64_t)i * stride, d2, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
+    fa_col_invw_tile<C>(A + (uint64_t)i * stride, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1164,10 +1283,14 @@ FA_DEV fa_operand fa_job_operand(const fa_bjob& j, int z)
     return o;
 }
 
+// threads of a batched column tile (D1 = 12: the 8-column tile)
+template <int D1>
+constexpr int fa_kb_nt() { return D1 == 12 ? 1024 : col_geom<D1>::NT; }
+
 template <int D1, int KIND>
-__global__ void __launch_bounds__(1024) fa_kb_col_fwd(const fa_bjob* __restrict__ J,
-                                                      const uint64_t* __restrict__ work,
-                                                      unsigned nwork, fa_prime_set S)
+__global__ void __launch_bounds__(fa_kb_nt<D1>(), 4)
+fa_kb_col_fwd(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, unsigned nwork,
+              fa_prime_set S)
 {
     __shared__ double lds[(D1 == 12) ? FA_C8_LDS : col_geom<D1>::LDS];
     const unsigned L = fa_xcd_linear();
@@ -1178,17 +1301,17 @@ __global__ void __launch_bounds__(1024) fa_kb_col_fwd(const fa_bjob* __restrict_
     const fa_operand op = fa_job_operand(j, w.op);
     double* dst = (w.op ? j.B : j.A) + (uint64_t)w.prime * j.stride;
     if constexpr (D1 == 12)
-        fa_col_fwd8_tile<KIND>(op, dst, FA_ROW_LG, w.tile, S.p[pi], S.pinv[pi], S.w2[pi],
+        fa_col_fwd8_tile<KIND>(op, dst, w.tile, S.p[pi], S.pinv[pi], S.w2[pi],
                                S.pow2[pi], lds);
     else
-        fa_col_fwd_tile<D1, KIND>(op, dst, FA_ROW_LG, w.tile, S.p[pi], S.pinv[pi], S.w2[pi],
-                                  S.pow2[pi], lds, j.trows);
+        fa_col_fwd_tile<D1, KIND>(op, dst, w.tile, S.p[pi], S.pinv[pi], S.w2[pi], S.pow2[pi], lds,
+                                  j.trows);
 }
 
 template <int D1>
-__global__ void __launch_bounds__(1024) fa_kb_col_inv(const fa_bjob* __restrict__ J,
-                                                      const uint64_t* __restrict__ work,
-                                                      unsigned nwork, fa_prime_set S)
+__global__ void __launch_bounds__(fa_kb_nt<D1>(), 4)
+fa_kb_col_inv(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, unsigned nwork,
+              fa_prime_set S)
 {
     __shared__ double lds[(D1 == 12) ? FA_C8_LDS : fa_col_inv_lds<D1>()];
     const unsigned L = fa_xcd_linear();
@@ -1198,12 +1321,12 @@ __global__ void __launch_bounds__(1024) fa_kb_col_inv(const fa_bjob* __restrict_
     const int pi = j.offset + w.prime;
     double* dst = j.A + (uint64_t)w.prime * j.stride;
     if constexpr (D1 == 12)
-        fa_col_inv8_tile(dst, FA_ROW_LG, w.tile, S.p[pi], S.pinv[pi], S.w2inv[pi], lds);
+        fa_col_inv8_tile(dst, w.tile, S.p[pi], S.pinv[pi], S.w2inv[pi], lds);
     else if (j.trows < (1 << D1))
         fa_col_inv_trunc_tile<D1>(dst, w.tile, j.trows, S.p[pi], S.pinv[pi], S.w2[pi],
                                   S.w2inv[pi], lds);
     else
-        fa_col_inv_tile<D1>(dst, FA_ROW_LG, w.tile, S.p[pi], S.pinv[pi], S.w2inv[pi], lds);
+        fa_col_inv_tile<D1>(dst, w.tile, S.p[pi], S.pinv[pi], S.w2inv[pi], lds);
 }
 
 __global__ void __launch_bounds__(256, 3) fa_kb_row_conv(const fa_bjob* __restrict__ J,
@@ -1261,12 +1384,30 @@ __global__ void __launch_bounds__(256) fa_kb_small_conv(const fa_bjob* __restric
 
 static unsigned grid8(unsigned n) { return (n + 7) & ~7u; }
 
-int fa_batch_col_groups(int depth)
+static int batch_col_cpw(int depth)
 {
-    const int d1 = depth - FA_ROW_LG;
-    if (d1 == 12) return 4096 / 8;
-    if (d1 >= 4) return 4096 / (1024 >> (d1 - 4));
-    return 4096 / 1024;
+    switch (depth - FA_ROW_LG) {
+    case 1: return col_geom<1>::CPW;
+    case 2: return col_geom<2>::CPW;
+    case 3: return col_geom<3>::CPW;
+    case 4: return col_geom<4>::CPW;
+    case 5: return col_geom<5>::CPW;
+    case 6: return col_geom<6>::CPW;
+    case 7: return col_geom<7>::CPW;
+    case 8: return col_geom<8>::CPW;
+    case 9: return col_geom<9>::CPW;
+    case 10: return col_geom<10>::CPW;
+    case 11: return col_geom<11>::CPW;
+    default: return 8;
+    }
+}
+
+int fa_batch_col_groups(int depth) { return 4096 / batch_col_cpw(depth); }
+
+int fa_batch_col_block(int depth)
+{
+    const int b = (depth == 24 ? FA_COLW_BLOCK : FA_COL_BLOCK) / batch_col_cpw(depth);
+    return b < 2 ? 2 : b;
 }
 
 int fa_batch_small_bin(int depth, int kind, const fa_bjob* J, const uint64_t* work,
@@ -1299,14 +1440,14 @@ static void batch_bin(const fa_bjob* J, const uint64_t* wf, unsigned nf, const u
                       hipStream_t s)
 {
     if (nf)
-        FA_LAUNCH("fa_kb_col_fwd", (fa_kb_col_fwd<D1, KIND>), dim3(grid8(nf)), dim3(1024), 0, s,
-                  J, wf, nf, S);
+        FA_LAUNCH("fa_kb_col_fwd", (fa_kb_col_fwd<D1, KIND>), dim3(grid8(nf)),
+                  dim3(fa_kb_nt<D1>()), 0, s, J, wf, nf, S);
     if (nr)
         FA_LAUNCH("fa_kb_row_conv", fa_kb_row_conv, dim3(grid8(nr)), dim3(256), 0, s, J, wr, nr,
                   S);
     if (ni)
-        FA_LAUNCH("fa_kb_col_inv", fa_kb_col_inv<D1>, dim3(grid8(ni)), dim3(1024), 0, s, J, wi,
-                  ni, S);
+        FA_LAUNCH("fa_kb_col_inv", fa_kb_col_inv<D1>, dim3(grid8(ni)),
+                  dim3(fa_kb_nt<D1>()), 0, s, J, wi, ni, S);
 }
 
 template <int D1>
@@ -1453,10 +1594,10 @@ static int launch_fast_pipe(const fa_operand& oa, const fa_operand& ob, int nops
         const unsigned gf = ((unsigned)(m * ngroups * nops) + 7) & ~7u;
         if (KIND == FA_PACK_MPN8 && oa.bits == 136 && ob.bits == 136)
             FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<8, KIND, 17>), dim3(gf), dim3(1024), 0,
-                      t, oa, ob, d2, Ag, Bg, stride, Sg, m, ngroups, nops);
+                      t, oa, ob, Ag, Bg, stride, Sg, m, ngroups, nops);
         else
             FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<8, KIND>), dim3(gf), dim3(1024), 0, t,
-                      oa, ob, d2, Ag, Bg, stride, Sg, m, ngroups, nops);
+                      oa, ob, Ag, Bg, stride, Sg, m, ngroups, nops);
         if (hipEventRecord(X->fwd[g], t) != hipSuccess)
             return fa_set_error(FA_E_HIP, "pipeline event");
         if (nops == 1)
@@ -1466,7 +1607,7 @@ static int launch_fast_pipe(const fa_operand& oa, const fa_operand& ob, int nops
             FA_LAUNCH("fa_k_row_conv16", fa_k_row_conv16lr<false>, dim3(1u << D1, m), dim3(256), 0,
                       t, Ag, Bg, stride, Sg);
         const unsigned gi = ((unsigned)(m * ngroups) + 7) & ~7u;
-        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(gi), dim3(1024), 0, t, Ag, d2, stride,
+        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(gi), dim3(1024), 0, t, Ag, stride,
                   Sg, m, ngroups);
         if (g && hipEventRecord(X->join[g - 1], t) != hipSuccess)
             return fa_set_error(FA_E_HIP, "pipeline join");
@@ -1507,16 +1648,16 @@ static int launch_fast(const fa_operand& oa, const fa_operand& ob, int nops, int
     unsigned grid = (total + 7) & ~7u;
     if (wide == 8 && KIND == FA_PACK_MPN8 && oa.bits == 136 && ob.bits == 136)
         FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<8, KIND, 17>), dim3(grid), dim3(1024), 0, s,
-                  oa, ob, d2, A, B, stride, S, np, ngroups, nops);
+                  oa, ob, A, B, stride, S, np, ngroups, nops);
     else if (wide == 8)
         FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<8, KIND>), dim3(grid), dim3(1024), 0, s, oa,
-                  ob, d2, A, B, stride, S, np, ngroups, nops);
+                  ob, A, B, stride, S, np, ngroups, nops);
     else if (wide == 4)
         FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<4, KIND>), dim3(grid), dim3(512), 0, s, oa,
-                  ob, d2, A, B, stride, S, np, ngroups, nops);
+                  ob, A, B, stride, S, np, ngroups, nops);
     else
-        FA_LAUNCH("fa_k_col_fwd16", (fa_k_col_fwd16<D1, KIND>), dim3(grid), dim3(1024), 0, s, oa, ob,
-                  d2, A, B, stride, S, np, ngroups, nops, trows);
+        FA_LAUNCH("fa_k_col_fwd16", (fa_k_col_fwd16<D1, KIND>), dim3(grid), dim3(G::NT), 0, s, oa,
+                  ob, A, B, stride, S, np, ngroups, nops, trows);
     const unsigned nrow = (unsigned)trows;
     if (fa_row_variant == 1 && nops == 1)
         FA_LAUNCH("fa_k_row_conv16", fa_k_row_conv16lr<true>, dim3(nrow, np), dim3(256), 0, s,
@@ -1530,14 +1671,14 @@ static int launch_fast(const fa_operand& oa, const fa_operand& ob, int nops, int
     unsigned total2 = (unsigned)(np * ngroups);
     unsigned grid2 = (total2 + 7) & ~7u;
     if (wide == 8)
-        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(grid2), dim3(1024), 0, s, A, d2,
+        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(grid2), dim3(1024), 0, s, A,
                   stride, S, np, ngroups);
     else if (wide == 4)
-        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<4>, dim3(grid2), dim3(512), 0, s, A, d2,
+        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<4>, dim3(grid2), dim3(512), 0, s, A,
                   stride, S, np, ngroups);
     else
-        FA_LAUNCH("fa_k_col_inv16", fa_k_col_inv16<D1>, dim3(grid2), dim3(1024), 0, s, A, d2, stride,
-                  S, np, ngroups, trows);
+        FA_LAUNCH("fa_k_col_inv16", fa_k_col_inv16<D1>, dim3(grid2), dim3(G::NT), 0, s, A, stride, S,
+                  np, ngroups, trows);
     return 1;
 }
 
@@ -1570,10 +1711,10 @@ static int launch_forward(const fa_operand& oa, int np, double* A, uint64_t stri
     const unsigned grid = ((unsigned)(np * ngroups) + 7) & ~7u;
     if (wide)
         FA_LAUNCH("fa_k_col_fwd16w", (fa_k_col_fwd16w<8, KIND>), dim3(grid), dim3(1024), 0, s, oa,
-                  oa, d2, A, A, stride, S, np, ngroups, 1);
+                  oa, A, A, stride, S, np, ngroups, 1);
     else
-        FA_LAUNCH("fa_k_col_fwd16", (fa_k_col_fwd16<D1, KIND>), dim3(grid), dim3(1024), 0, s, oa,
-                  oa, d2, A, A, stride, S, np, ngroups, 1, 1 << D1);
+        FA_LAUNCH("fa_k_col_fwd16", (fa_k_col_fwd16<D1, KIND>), dim3(grid), dim3(G::NT), 0, s, oa,
+                  oa, A, A, stride, S, np, ngroups, 1, 1 << D1);
     FA_LAUNCH("fa_k_row_fwd16", fa_k_row_fwd16, dim3(1u << D1, np), dim3(256), 0, s, A, stride, S);
     return 1;
 }
@@ -1589,11 +1730,11 @@ static int launch_inverse(int np, double* A, uint64_t stride, const fa_prime_set
     const unsigned grid = ((unsigned)(np * ngroups) + 7) & ~7u;
     FA_LAUNCH("fa_k_row_inv16", fa_k_row_inv16, dim3(1u << D1, np), dim3(256), 0, s, A, stride, S);
     if (wide)
-        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(grid), dim3(1024), 0, s, A, d2,
+        FA_LAUNCH("fa_k_col_inv16w", fa_k_col_inv16w<8>, dim3(grid), dim3(1024), 0, s, A,
                   stride, S, np, ngroups);
     else
-        FA_LAUNCH("fa_k_col_inv16", fa_k_col_inv16<D1>, dim3(grid), dim3(1024), 0, s, A, d2, stride,
-                  S, np, ngroups, 1 << D1);
+        FA_LAUNCH("fa_k_col_inv16", fa_k_col_inv16<D1>, dim3(grid), dim3(G::NT), 0, s, A, stride, S,
+                  np, ngroups, 1 << D1);
     return 1;
 }
 

@@ -281,6 +281,8 @@ int fa_batch_transform_bin(int depth, int kind, const fa_bjob* J, const uint64_t
                            hipStream_t s);
 // column groups per residue array in the batched column passes at depth D
 int fa_batch_col_groups(int depth);
+// adjacent column groups that come before the next prime in a work list
+int fa_batch_col_block(int depth);
 }
 
 // ---------------------------------------------------------------------------

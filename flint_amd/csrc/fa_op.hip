@@ -155,8 +155,13 @@ __global__ void __launch_bounds__(256) fa_k_op_point(int op, double* __restrict_
             r = fa_reduce_pm1n(op == OP_ADDMUL ? Z[at] + t : Z[at] - t, n, ninv);
             break;
         }
-        case OP_ADD: r = fa_reduce_pm1n(a + B[at], n, ninv); break;
-        case OP_SUB: r = fa_reduce_pm1n(a - B[at], n, ninv); break;
+        // coefficients after the inverse transform reach 8n: reduced before the sum
+        case OP_ADD:
+            r = fa_reduce_pm1n(fa_reduce_pm1n(a, n, ninv) + fa_reduce_pm1n(B[at], n, ninv), n, ninv);
+            break;
+        case OP_SUB:
+            r = fa_reduce_pm1n(fa_reduce_pm1n(a, n, ninv) - fa_reduce_pm1n(B[at], n, ninv), n, ninv);
+            break;
         default: r = -a; break;
         }
         Z[at] = r;

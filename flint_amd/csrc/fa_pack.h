@@ -121,41 +121,6 @@ FA_DEV double fa_chunk_residue8(const uint64_t* __restrict__ limbs, uint64_t nli
     return acc;
 }
 
-// fa_chunk_residue8 for a chunk whose 32-byte window [B & ~3, (B & ~3) + 32)
-// lies inside the limb array (no bounds checks)
-FA_DEV double fa_chunk_residue8_in(const char* __restrict__ base, uint64_t B, int own,
-                                   const double* __restrict__ pow2, double n, double ninv)
-{
-    const fa_u32x4_a4* q = (const fa_u32x4_a4*)(base + (B & ~UINT64_C(3)));
-    const fa_u32x4 lo4 = q[0], hi4 = q[1];
-    const uint32_t w[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-    const uint32_t s = (uint32_t)(B & 3);
-    uint32_t c[7];
-#pragma unroll
-    for (int m = 0; m < 7; m++) {
-        c[m] = __builtin_amdgcn_alignbyte(w[m + 1], w[m], s);
-        const int vb = own - 4 * m;
-        if (vb < 4) c[m] = (vb <= 0) ? 0u : (c[m] & ((1u << (8 * vb)) - 1u));
-    }
-    const double T16 = 65536.0, T32 = 4294967296.0;
-    double acc = __builtin_fma((double)(c[1] & 0xffffu), T32, (double)c[0]);
-    if (own > 6) {
-        const double p1 = __builtin_fma((double)c[2], T16, (double)(c[1] >> 16));
-        acc += fa_mulmod(p1, pow2[1], n, ninv);
-    }
-    if (own > 12) {
-        const double p2 = __builtin_fma((double)(c[4] & 0xffffu), T32, (double)c[3]);
-        acc += fa_mulmod(p2, pow2[2], n, ninv);
-    }
-    if (own > 18) {
-        const double p3 = __builtin_fma((double)c[5], T16, (double)(c[4] >> 16));
-        acc += fa_mulmod(p3, pow2[3], n, ninv);
-        if (own > 24) acc += fa_mulmod((double)c[6], pow2[4], n, ninv);
-        acc = fa_reduce_pm1n(acc, n, ninv);
-    }
-    return acc;
-}
-
 // ------------------------------------------------------------------------
 // operand import: the value of element x (coefficient index) of an operand
 // ------------------------------------------------------------------------
@@ -202,11 +167,12 @@ FA_DEV double fa_operand_value(const fa_operand& op, uint64_t x,
     return fa_coeff_residue_s(op.src + x * (uint64_t)op.width, op.width, pow2, n, ninv);
 }
 
-// number of elements of an operand (chunks of a limb array, coefficients)
-FA_DEV uint64_t fa_operand_len(const fa_operand& op)
+// whether an operand has at most len elements (chunks of a limb array,
+// coefficients), len a power of two below 2^25
+FA_DEV bool fa_operand_fits(const fa_operand& op, uint32_t len)
 {
-    if (op.kind == FA_PACK_MPN) return (64 * op.n + (uint64_t)op.bits - 1) / (uint64_t)op.bits;
-    return op.n;
+    if (op.kind == FA_PACK_MPN) return 64 * op.n <= (uint64_t)op.bits * len;
+    return op.n <= len;
 }
 
 // import specialized at compile time (KIND = FA_PACK_*), FA_PACK_ANY
@@ -230,6 +196,212 @@ FA_DEV double fa_operand_value_k(const fa_operand& op, uint64_t x,
         return fa_coeff_residue_s(op.src + x * (uint64_t)op.width, op.width, pow2, n, ninv);
     } else {
         return fa_operand_value(op, x, pow2, n, ninv);
+    }
+}
+
+// ------------------------------------------------------------------------
+// column import: elements e0 + k step (k < NB) of an operand, e < 2^24.  All
+// loads of a batch are issued before the arithmetic; a batch that lies inside
+// the operand for the whole wave is read without checks, one that lies past
+// its end for the whole wave is zero.  Values are below 2.75 n in size, which
+// the first stage of the column transforms allows for.
+// ------------------------------------------------------------------------
+
+// byte-aligned chunks: fa_chunk_residue8 for a batch.  A chunk of own bytes
+// is cut into ceil(own / 6) pieces of 48 bits; the width is uniform, so the
+// higher pieces are skipped by scalar branches.
+template <int NB, int OWN>
+FA_DEV void fa_import_mpn8(double* x, const fa_operand& op, uint32_t e0, uint32_t step,
+                           const double* __restrict__ pow2, double n, double ninv)
+{
+    const uint32_t own = OWN ? OWN : (uint32_t)op.bits >> 3;
+    const char* base = (const char*)op.src;
+    const uint32_t nbytes = op.n < (UINT64_C(1) << 29) ? (uint32_t)op.n * 8u : 0xfffffff8u;
+    const uint32_t B0 = e0 * own, bstep = step * own;
+    if (!__any(B0 < nbytes)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) x[i] = 0.0;
+        return;
+    }
+    // 32-byte windows at the enclosing 4-byte boundary.  Lanes past the end
+    // read the operand's last window instead and are cleared below; chunks
+    // that straddle the end (the last one or two of an operand) send their
+    // wave to word by word loads.
+    uint32_t c[NB][7];
+    const bool inside = __all(((B0 + (NB - 1) * bstep) & ~3u) + 32u <= nbytes);
+    bool edge = nbytes < 32u;
+    if (!inside) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const uint32_t B = B0 + i * bstep;
+            edge |= B < nbytes && (B & ~3u) + 32u > nbytes;
+        }
+    }
+    if (inside || !__any(edge)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const uint32_t B4 = (B0 + i * bstep) & ~3u;
+            const uint32_t at = B4 < nbytes - 32u ? B4 : nbytes - 32u;
+            const fa_u32x4 lo4 = fa_ld<fa_u32x4_a4>(base, at);
+            fa_u32x4 hi4 = {0, 0, 0, 0};
+            if (own > 13) hi4 = fa_ld<fa_u32x4_a4>(base + 16, at);
+            const uint32_t w[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+            const uint32_t s = (B0 + i * bstep) & 3u;
+#pragma unroll
+            for (int m = 0; m < 7; m++) c[i][m] = __builtin_amdgcn_alignbyte(w[m + 1], w[m], s);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const uint32_t B4 = (B0 + i * bstep) & ~3u;
+            uint32_t w[8];
+#pragma unroll
+            for (uint32_t m = 0; m < 8; m++) {
+                const uint32_t at = B4 + 4 * m;
+                const uint32_t v = fa_ld<uint32_t>(base, at < nbytes ? at : 0u);
+                w[m] = at < nbytes ? v : 0u;
+            }
+            const uint32_t s = (B0 + i * bstep) & 3u;
+#pragma unroll
+            for (int m = 0; m < 7; m++) c[i][m] = __builtin_amdgcn_alignbyte(w[m + 1], w[m], s);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 7; m++) {
+        // bytes of word m that belong to the chunk
+        const uint32_t mk = own >= 4u * m + 4 ? 0xffffffffu
+                            : own <= 4u * m ? 0u : (1u << (8 * (own - 4u * m))) - 1u;
+#pragma unroll
+        for (int i = 0; i < NB; i++) c[i][m] &= mk;
+    }
+    const double T16 = 65536.0, T32 = 4294967296.0;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+        x[i] = __builtin_fma((double)(c[i][1] & 0xffffu), T32, (double)c[i][0]);
+    if (own > 6) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const double p1 = __builtin_fma((double)c[i][2], T16, (double)(c[i][1] >> 16));
+            x[i] += fa_mulmod(p1, pow2[1], n, ninv);
+        }
+    }
+    if (own > 12) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const double p2 = __builtin_fma((double)(c[i][4] & 0xffffu), T32, (double)c[i][3]);
+            x[i] += fa_mulmod(p2, pow2[2], n, ninv);
+        }
+    }
+    if (own > 18) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const double p3 = __builtin_fma((double)c[i][5], T16, (double)(c[i][4] >> 16));
+            x[i] += fa_mulmod(p3, pow2[3], n, ninv);
+        }
+        if (own > 24) {
+#pragma unroll
+            for (int i = 0; i < NB; i++)
+                x[i] += fa_mulmod((double)c[i][6], pow2[4], n, ninv);
+        }
+    }
+    if (!inside) {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            if (B0 + i * bstep >= nbytes) x[i] = 0.0;
+    }
+}
+
+// u64 coefficients: v = lo + 2^32 hi as a double when the whole wave's values
+// are below 2^50, else lo + (2^32 hi mod n)
+template <int NB>
+FA_DEV void fa_import_u64(double* x, const fa_operand& op, uint32_t e0, uint32_t step,
+                          const double* __restrict__ pow2, double n, double ninv)
+{
+    const uint32_t len = op.n < (UINT64_C(1) << 31) ? (uint32_t)op.n : 1u << 31;
+    if (!__any(e0 < len)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) x[i] = 0.0;
+        return;
+    }
+    uint32_t lo[NB], hi[NB], top = 0;
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const uint32_t e = e0 + i * step;
+        const uint64_t v = fa_ld<uint64_t>(op.src, (e < len ? e : 0u) * 8u);
+        lo[i] = e < len ? (uint32_t)v : 0u;
+        hi[i] = e < len ? (uint32_t)(v >> 32) : 0u;
+        top |= hi[i];
+    }
+    if (__any(top >> 18)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            x[i] = fa_mulmod((double)hi[i], pow2[0], n, ninv) + (double)lo[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            x[i] = __builtin_fma((double)hi[i], 4294967296.0, (double)lo[i]);
+    }
+}
+
+// two's complement coefficients of w limbs: Horner over the 32-bit words from
+// the top one, which is read as signed
+template <int NB>
+FA_DEV void fa_import_s64w(double* x, const fa_operand& op, uint32_t e0, uint32_t step,
+                           const double* __restrict__ pow2, double n, double ninv)
+{
+    const uint32_t len = op.n < (UINT64_C(1) << 31) ? (uint32_t)op.n : 1u << 31;
+    const int w = op.width;
+    if (!__any(e0 < len)) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) x[i] = 0.0;
+        return;
+    }
+    const double c32 = pow2[0];
+    typedef __attribute__((address_space(1))) uint64_t gT;
+    const gT* p[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const uint32_t e = e0 + i * step;
+        p[i] = (const gT*)op.src + (uint64_t)(e < len ? e : 0u) * (uint64_t)w;
+        const uint64_t v = p[i][w - 1];
+        x[i] = fa_mulmod((double)(int32_t)(v >> 32), c32, n, ninv) + (double)(uint32_t)v;
+    }
+    for (int l = w - 2; l >= 0; l--) {
+        uint64_t v[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) v[i] = p[i][l];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            x[i] = fa_mulmod(x[i], c32, n, ninv) + (double)(uint32_t)(v[i] >> 32);
+            x[i] = fa_mulmod(x[i], c32, n, ninv) + (double)(uint32_t)v[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+        if (e0 + i * step >= len) x[i] = 0.0;
+}
+
+// elements e0 + k step, k < NEL (a multiple of the batch, or less than one)
+template <int NEL, int KIND, int OWN = 0>
+FA_DEV void fa_import_column(double* x, const fa_operand& op, uint32_t e0, uint32_t step,
+                             const double* __restrict__ pow2, double n, double ninv)
+{
+    if constexpr (KIND == FA_PACK_MPN8 || KIND == FA_PACK_U64 || KIND == FA_PACK_S64W) {
+        constexpr int NB = KIND == FA_PACK_U64 ? (NEL < 8 ? NEL : 8) : (NEL < 4 ? NEL : 4);
+#pragma unroll
+        for (int k = 0; k < NEL; k += NB) {
+            const uint32_t e = e0 + (uint32_t)k * step;
+            if constexpr (KIND == FA_PACK_MPN8)
+                fa_import_mpn8<NB, OWN>(x + k, op, e, step, pow2, n, ninv);
+            else if constexpr (KIND == FA_PACK_U64)
+                fa_import_u64<NB>(x + k, op, e, step, pow2, n, ninv);
+            else
+                fa_import_s64w<NB>(x + k, op, e, step, pow2, n, ninv);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NEL; k++)
+            x[k] = fa_operand_value(op, e0 + (uint32_t)k * step, pow2, n, ninv);
     }
 }
 

@@ -373,13 +373,13 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
 
     // ---- layout
     // two regions: the records, constants and work lists (uploaded), then the
-    // residue rows, staging and carry flags (no initial contents)
+    // residue rows, staging and carry aggregates (no initial contents)
     layout L, Lb, Lin, Lout;
     std::vector<fa_bjob> jobs;
     std::vector<fa_bmpn> mrec;
     std::vector<fa_bpoly> prec;
     std::vector<int> job_of((size_t)ntot, -1), rec_of((size_t)ntot, -1);
-    struct offs { size_t A, B, a, b, z, flags, agg; };
+    struct offs { size_t A, B, a, b, z, agg; };
     std::vector<offs> O((size_t)ntot);
     std::vector<size_t> ks_scratch(ksv.size());
     for (size_t k = 0; k < ksv.size(); k++) {
@@ -415,7 +415,6 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
                         : q.kind == FA_REQ_NMOD ? (size_t)p.cnt : (size_t)p.cnt * (size_t)q.zw;
         if (!dev && !p.virt) o.z = Lout.take(zwords * 8);
         if (q.kind == FA_REQ_MPN) {
-            o.flags = Lb.take((size_t)p.ngroups + 8);
             o.agg = Lb.take((size_t)p.nblk + 8);
         }
         if (q.kind != FA_REQ_MPN && p.np && !pconsts.count({p.np, p.offset}))
@@ -510,14 +509,13 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             m.stride = fa_res_stride(p.depth);
             m.zlen = p.zlen;
             m.zn = p.zn;
-            m.ngroups = p.ngroups;
             m.nblk = p.nblk;
             m.bits = p.bits;
             m.np = p.np;
             mrec.push_back(m);
             auto& w = crt_bins[p.np];
             for (uint64_t blk = 0; blk < p.nblk; blk++) w.push_back((uint64_t)mid | (blk << 32));
-            carry.push_back(mid);
+            if (p.nblk > 1) carry.push_back(mid);   // one workgroup resolves its own
         } else {
             const unsigned pid = (unsigned)prec.size();
             rec_of[(size_t)r] = (int)pid;
@@ -604,7 +602,7 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
         return fa_set_error(FA_E_NOMEM, "fa_batch_create: %zu bytes of device memory", B->dsize);
     }
     char* d = B->dmem;
-    char* db0 = d + big;   // residue rows and carry flags
+    char* db0 = d + big;   // residue rows and carry aggregates
     char* din = d + inb;   // staged operands (host-pointer batches)
     char* dout = d + outb; // staged outputs
 
@@ -677,7 +675,6 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             fa_bmpn& m = mrec[(size_t)rec_of[(size_t)r]];
             m.Q = (const double*)(db0 + o.A);
             m.z = dz;
-            m.flags = (uint8_t*)(db0 + o.flags);
             m.agg = (uint8_t*)(db0 + o.agg);
         } else {
             fa_bpoly& b = prec[(size_t)rec_of[(size_t)r]];

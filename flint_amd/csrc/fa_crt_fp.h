@@ -12,9 +12,11 @@
 // e_(i,d); every term u e < 2^48 and |v e| < 2^49 is an exact FMA, and a
 // column collects at most six primes' terms, 6 (2^48 + 2^49) < 2^53, before
 // it is carried into 24-bit digits (signed floor division).
-// k = rint(sum_i x_i / p_i) is k_true or k_true + 1 (the sum's rounding
-// error is far below 1/2), so c' = S - k M lies in [-M, M) and one
-// conditional + M fixes the sign.
+// k = floor(sum_i x_i / p_i + 2^-30) is floor(S / M) or one more (the sum's
+// rounding error is below 2^-45), so c' = S - k M lies in [-2^-30 M, M) and a
+// conditional + M, taken for values within 2^-30 M of M only, fixes the sign.
+// (Rounding to nearest instead made half of all values negative, and with
+// them almost every wave took the correction.)
 #pragma once
 
 #include "fa_internal.h"
@@ -24,7 +26,8 @@ template <int NP>
 struct fa_crt_fp_dims {
     static constexpr int ND = (50 * NP + 23) / 24;         // digits of M
     static constexpr int NDC = (50 * (NP - 1) + 23) / 24;  // digits of M / p_i
-    static constexpr int NL = (50 * NP + 63) / 64;         // 64-bit limbs of c < M
+    static constexpr int NW = (24 * ND + 31) / 32;         // 32-bit words of the digits
+    static constexpr int NB = (50 * NP + 7) / 8;           // bytes of c < M
 };
 
 // constants of the radix-2^24 CRT, filled on the host
@@ -55,15 +58,16 @@ FA_DEV double fa_crt_fp_carry(double* col)
     return carry;
 }
 
-// coefficient j -> its NL little-endian 64-bit limbs.  MODE 0: c in
+// coefficient j -> its NW little-endian 32-bit words.  MODE 0: c in
 // [0, M); for the centred lift c~ = c - M when c > M/2 (the signed exports,
 // export_signed.c:60-80), MODE 1 gives max(c~, 0) and MODE 2 max(-c~, 0).
 template <int NP, int MODE = 0>
-FA_DEV void fa_crt_fp_value(const double* __restrict__ Q, uint64_t stride, uint64_t j,
-                            const fa_crt_fp_consts& F, uint64_t* L)
+FA_DEV void fa_crt_fp_value(const double* __restrict__ Q, uint64_t stride, uint32_t j,
+                            const fa_crt_fp_consts& F, uint32_t* W)
 {
     typedef fa_crt_fp_dims<NP> D;
-    constexpr int ND = D::ND, NDC = D::NDC, NL = D::NL;
+    constexpr int ND = D::ND, NDC = D::NDC, NW = D::NW;
+    const uint32_t at = (uint32_t)fa_res_pos(j, stride) * 8u;
     const double B = 16777216.0, Binv = 1.0 / 16777216.0;
     double col[ND];
 #pragma unroll
@@ -78,7 +82,7 @@ FA_DEV void fa_crt_fp_value(const double* __restrict__ Q, uint64_t stride, uint6
             col[ND - 1] = __builtin_fma(top, B, col[ND - 1]);
         }
         const double n = F.p[i];
-        const double x = fa_reduce_pm1n(Q[(uint64_t)i * stride + fa_res_pos(j, stride)], n,
+        const double x = fa_reduce_pm1n(fa_ld<double>(Q + (uint64_t)i * stride, at), n,
                                         F.pinv[i]);   // [-n/2, n/2]
         qe = __builtin_fma(x, F.rp[i], qe);
         const double v = __builtin_floor(x * Binv);
@@ -89,7 +93,7 @@ FA_DEV void fa_crt_fp_value(const double* __restrict__ Q, uint64_t stride, uint6
             col[d + 1] = __builtin_fma(v, F.cof[i][d], col[d + 1]);
         }
     }
-    const double k = __builtin_rint(qe);
+    const double k = __builtin_floor(qe + 0x1p-30);
 #pragma unroll
     for (int m = 0; m < ND; m++) col[m] = __builtin_fma(-k, F.M[m], col[m]);
     const double top = fa_crt_fp_carry<ND>(col);
@@ -121,12 +125,12 @@ FA_DEV void fa_crt_fp_value(const double* __restrict__ Q, uint64_t stride, uint6
         }
     }
 #pragma unroll
-    for (int l = 0; l < NL; l++) L[l] = 0;
+    for (int l = 0; l < NW; l++) W[l] = 0;
 #pragma unroll
     for (int m = 0; m < ND; m++) {
-        const uint64_t dv = (uint64_t)(uint32_t)col[m];
+        const uint32_t dv = (uint32_t)col[m];
         const int pos = 24 * m;
-        if (pos / 64 < NL) L[pos / 64] |= dv << (pos % 64);
-        if (pos % 64 > 40 && pos / 64 + 1 < NL) L[pos / 64 + 1] |= dv >> (64 - pos % 64);
+        W[pos / 32] |= dv << (pos % 32);
+        if (pos % 32 > 8) W[pos / 32 + 1] |= dv >> (32 - pos % 32);
     }
 }

@@ -206,9 +206,8 @@ struct fa_bmpn {               // integer product
     uint64_t zlen;             // coefficients of the chunked product
     uint64_t* z;               // output limbs
     uint64_t zn;               // an + bn
-    uint64_t ngroups, nblk;    // CRT groups of 8 coefficients, CRT workgroups
-    uint8_t* flags;            // per group / per workgroup carry flags
-    uint8_t* agg;
+    uint64_t nblk;             // CRT workgroups
+    uint8_t* agg;              // their carry aggregates
     int bits, np;
 };
 struct fa_bpoly {              // nmod or fmpz polynomial product

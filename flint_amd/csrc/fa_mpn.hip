@@ -498,7 +498,6 @@ __global__ void __launch_bounds__(256) fa_k_crt_mpn16(const double* __restrict__
                                                       uint64_t zlen, int bits,
                                                       uint64_t* __restrict__ z, uint64_t zn,
                                                       uint64_t ngroups,
-                                                      uint8_t* __restrict__ flags,
                                                       uint8_t* __restrict__ agg)
 {
     constexpr int NL = fa_crt_limbs<NP>::N;
@@ -587,23 +586,27 @@ __global__ void __launch_bounds__(256) fa_k_crt_mpn16(const double* __restrict__
                 if (tt != ~UINT64_C(0)) prop = 0;
             }
             f = (uint8_t)(carry | (prop << 1));
-            flags[g] = f;
         }
         sF[t] = f;
     }
     __syncthreads();
     if (t == 0) {
-        // bit 0: carry out with no carry in, bit 1: every group propagates,
-        // bit 2: some group generates a carry
-        uint8_t gg = 0, pp = 1, any = 0;
+        // the carries between the workgroup's groups (bit 0 of the aggregate:
+        // carry out with no carry in, bit 1: every group propagates)
+        uint8_t gg = 0, pp = 1;
         for (int k = 1; k < FA_CRT16_GROUPS; k++) {
             uint8_t ft = sF[k];
+            if (gg) {
+                uint64_t* out = sOut + k * FA_OUT_STRIDE;
+                for (int l = 0; l < own; l++)
+                    if (++out[l]) break;
+            }
             gg = (uint8_t)((ft & 1) | (((ft >> 1) & 1) & gg));
             pp = (uint8_t)(pp & ((ft >> 1) & 1));
-            any = (uint8_t)(any | (ft & 1));
         }
-        agg[blockIdx.x] = (uint8_t)(gg | (pp << 1) | (any << 2));
+        agg[blockIdx.x] = (uint8_t)(gg | (pp << 1));
     }
+    __syncthreads();
     // contiguous write of the limbs of groups 1..31
     const uint64_t base = (uint64_t)(g0 + 1) * own;
     const int nl = (FA_CRT16_GROUPS - 1) * own;
@@ -613,46 +616,12 @@ __global__ void __launch_bounds__(256) fa_k_crt_mpn16(const double* __restrict__
     }
 }
 
-// carry-in of every group of a 31-group workgroup: scan of the group flags
-// seeded with the workgroup carry-in
-__global__ void __launch_bounds__(64) fa_k_carry_apply16(const uint8_t* __restrict__ flags,
-                                                         const uint8_t* __restrict__ cin,
-                                                         uint64_t* __restrict__ z, uint64_t zn,
-                                                         int own, uint64_t ngroups)
-{
-    __shared__ uint8_t sg[FA_CRT16_GROUPS], sp[FA_CRT16_GROUPS];
-    const int t = threadIdx.x;
-    const int64_t g = (int64_t)blockIdx.x * (FA_CRT16_GROUPS - 1) + t - 1;
-    const bool active = t >= 1 && t < FA_CRT16_GROUPS && g >= 0 && (uint64_t)g < ngroups;
-    if (t < FA_CRT16_GROUPS) {
-        uint8_t f = active ? flags[g] : 2;
-        if (t == 0) f = (uint8_t)(cin[blockIdx.x] & 1);
-        sg[t] = f & 1;
-        sp[t] = (f >> 1) & 1;
-    }
-    __syncthreads();
-    if (t != 0) return;
-    // serial inclusive scan over 32 entries, then apply
-    uint8_t gg = sg[0];
-    for (int k = 1; k < FA_CRT16_GROUPS; k++) {
-        int64_t gk = (int64_t)blockIdx.x * (FA_CRT16_GROUPS - 1) + k - 1;
-        if (gk < 0 || (uint64_t)gk >= ngroups) break;
-        if (gg) {
-            uint64_t zb = (uint64_t)gk * own;
-            for (int l = 0; l < own && zb + l < zn; l++) {
-                uint64_t v = z[zb + l] + 1;
-                z[zb + l] = v;
-                if (v != 0) break;
-            }
-        }
-        gg = sg[k] | (sp[k] & gg);
-    }
-}
-
 // adds 1 to the n limbs at p with carry (stops at the first limb that does
 // not wrap); eight loads in flight at a time
-FA_DEV void fa_add_one(uint64_t* __restrict__ p, int n)
+FA_DEV void fa_add_one(uint64_t* __restrict__ pz, int n)
 {
+    typedef __attribute__((address_space(1))) uint64_t gT;
+    gT* p = (gT*)pz;
     for (int l0 = 0; l0 < n; l0 += 8) {
         const int m = n - l0 < 8 ? n - l0 : 8;
         uint64_t v[8];
@@ -670,284 +639,273 @@ FA_DEV void fa_add_one(uint64_t* __restrict__ p, int n)
     }
 }
 
-FA_DEV uint8_t fa_gp_fold(uint8_t acc, uint8_t a)   // (generate, propagate) of acc then a
+// carries through 64 positions with generate and propagate masks G, P (no
+// position both): the carries into the positions for a carry c into the
+// first, and through cout the carry out of the last
+FA_DEV uint64_t fa_gp_carries(uint64_t G, uint64_t P, uint32_t c, uint32_t* cout)
 {
-    const uint8_t g = (uint8_t)((a & 1) | (((a >> 1) & 1) & acc));
-    const uint8_t p = (uint8_t)((acc >> 1) & (a >> 1) & 1);
-    return (uint8_t)(g | (p << 1));
+    const uint64_t X = G | P;
+    const uint64_t s1 = G + X;
+    const uint64_t s2 = s1 + c;
+    *cout = (uint32_t)(s1 < X) | (uint32_t)(s2 < s1);
+    return s2 ^ X ^ G;
 }
 
-// carries between CRT workgroups ("blocks" of FA_CRT16_GROUPS - 1 groups of
-// own limbs), by workgroup wg of nwg (1024 threads each) on its contiguous
-// range of blocks.  A block's aggregate holds bit 0: carry out with no
-// carry in, bit 1: every group propagates, bit 2: some group generates.
-//  1. the carry into the range: each thread folds a slice of the aggregates
-//     before it, the slices are combined in order in LDS;
-//  2. the carry into each block of the range: a scan over the range in
-//     tiles of 1024 blocks;
-//  3. one wave per block: lane k takes group k of the block, its carry-in
-//     composed from the flags of the groups before it, and a group with a
-//     carry-in adds it to its limbs.  A group's addition stays inside its
-//     own limbs except when they are all ones (then they become zeros and
-//     the carry passes on, which the flags already give the next group), so
-//     groups are independent once their carries-in are known.  Blocks that
-//     receive no carry and generate none inside are skipped.
-// No workgroup waits on another: each computes its own prefix.
-FA_DEV void fa_carry_resolve(const uint8_t* __restrict__ flags, const uint8_t* __restrict__ agg,
-                             uint64_t* __restrict__ z, uint64_t zn, int own, uint64_t ngroups,
-                             uint64_t nblk, unsigned wg, unsigned nwg)
+// carries between CRT workgroups ("blocks" of bl limbs), for the blocks
+// [b0, b1).  A block's aggregate holds bit 0: carry out with no carry in, bit
+// 1: all its limbs are ones.
+//  1. the carry into b0: the blocks before it, blockDim at a time from the
+//     nearest, until some block does not propagate (the first chunk, unless
+//     the product holds long runs of ones);
+//  2. tiles of blockDim blocks, one per thread: the carries into the blocks
+//     of a wave come from its ballots and the waves' masks in LDS;
+//  3. a block with a carry-in adds it to its limbs.  The addition leaves the
+//     block only if all its limbs are ones, which the propagate bit has
+//     already told the next block, so blocks are independent.
+// Latency bound: 25 -> 6 us for the 63,671 blocks of 2^24 x 2^24 limbs and 6
+// -> 1.5..2 us for a few blocks, against LDS scans of flag bytes by 1024
+// threads in 20 steps and one wave per block.
+FA_DEV void fa_carry_resolve(const uint8_t* __restrict__ agg, uint64_t* __restrict__ z,
+                             uint64_t zn, uint32_t bl, uint64_t nblk, uint64_t b0, uint64_t b1)
 {
-    __shared__ uint8_t sa[1024];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const uint64_t per = (nblk + nwg - 1) / nwg;
-    const uint64_t r0 = (uint64_t)wg * per < nblk ? (uint64_t)wg * per : nblk;
-    const uint64_t r1 = r0 + per < nblk ? r0 + per : nblk;
-    // 1. aggregate of blocks [0, r0), identity (no generate, propagate) = 2
-    {
-        const uint64_t sl = (r0 + 1023) / 1024;
-        const uint64_t s0 = (uint64_t)t * sl < r0 ? (uint64_t)t * sl : r0;
-        const uint64_t s1 = s0 + sl < r0 ? s0 + sl : r0;
-        uint8_t acc = 2;
-        for (uint64_t b = s0; b < s1; b++) acc = fa_gp_fold(acc, agg[b]);
-        sa[t] = acc;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            uint8_t v = 0;
-            const bool act = (t & (2 * off - 1)) == 0;
-            if (act) v = fa_gp_fold(sa[t], sa[t + off]);
-            __syncthreads();
-            if (act) sa[t] = v;
-            __syncthreads();
+    __shared__ uint64_t sG[16], sP[16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nt = blockDim.x, nw = nt >> 6;
+    uint32_t c = 0;
+    for (int64_t hi = (int64_t)b0; hi > 0; hi -= nt) {
+        const int64_t b = hi - nt + t;
+        const uint8_t a = b >= 0 ? agg[b] : 0;
+        const uint64_t G = __ballot(a & 1), P = __ballot(a & 2);
+        if (lane == 0) {
+            sG[wave] = G;
+            sP[wave] = P;
         }
+        __syncthreads();
+        uint64_t all = ~UINT64_C(0);
+        c = 0;
+        for (int w = 0; w < nw; w++) {
+            uint32_t o;
+            (void)fa_gp_carries(sG[w], sP[w], c, &o);
+            c = o;
+            all &= sP[w];
+        }
+        __syncthreads();
+        if (~all) break;     // the same for every thread
     }
-    uint8_t c = sa[0] & 1;          // carry into block r0
-    __syncthreads();
-    const uint64_t gper = FA_CRT16_GROUPS - 1;
-    for (uint64_t tb = r0; tb < r1; tb += 1024) {
-        // 2. inclusive scan of this tile's aggregates, seeded with c
+    for (uint64_t tb = b0; tb < b1; tb += nt) {
         const uint64_t b = tb + (uint64_t)t;
-        const uint8_t a = b < r1 ? agg[b] : 2;
-        sa[t] = a;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            uint8_t v = sa[t];
-            if (t >= off) v = fa_gp_fold(sa[t - off], v);
-            __syncthreads();
-            sa[t] = v;
-            __syncthreads();
+        const uint8_t a = b < b1 ? agg[b] : 0;
+        const uint64_t G = __ballot(a & 1), P = __ballot(a & 2);
+        if (lane == 0) {
+            sG[wave] = G;
+            sP[wave] = P;
         }
-        // carry into block b: fold of c with the tile's blocks before b
-        const uint8_t cin = t ? (uint8_t)(fa_gp_fold(c, sa[t - 1]) & 1) : c;
-        const uint8_t cout_tile = (uint8_t)(fa_gp_fold(c, sa[1023]) & 1);
         __syncthreads();
-        sa[t] = (uint8_t)(cin | (a & 4));
-        __syncthreads();
-        // 3. one wave per block of the tile
-        const uint64_t nb = r1 - tb < 1024 ? r1 - tb : 1024;
-        for (uint64_t k = (uint64_t)wave; k < nb; k += 16) {
-            const uint8_t s = sa[k];
-            if (!(s & 1) && !(s & 4)) continue;
-            const uint64_t gs = (tb + k) * gper;
-            const uint64_t ge = gs + gper < ngroups ? gs + gper : ngroups;
-            const uint64_t gi = gs + (uint64_t)lane;
-            const uint8_t f = gi < ge ? flags[gi] : 2;
-            uint8_t cg = s & 1;
-            // every lane takes part in every shuffle (the block test above
-            // is the same for the whole wave)
-            for (int j = 0; j < (int)gper; j++) {
-                const uint8_t fj = (uint8_t)__shfl((int)f, j);
-                if (j < lane) cg = (uint8_t)((fj & 1) | (((fj >> 1) & 1) & cg));
-            }
-            if (cg && gi < ge) {
-                const uint64_t zb = gi * (uint64_t)own;
-                const int n = zb + (uint64_t)own <= zn ? own : (int)(zn - zb);
-                fa_add_one(z + zb, n);
-            }
+        uint32_t cw = 0;
+        for (int w = 0; w < nw; w++) {
+            if (w == wave) cw = c;
+            uint32_t o;
+            (void)fa_gp_carries(sG[w], sP[w], c, &o);
+            c = o;
         }
-        c = cout_tile;
+        uint32_t o;
+        const uint64_t cin = fa_gp_carries(G, P, cw, &o);
+        const uint64_t zb = b * bl;
+        if (b < b1 && ((cin >> lane) & 1) && zb < zn)
+            fa_add_one(z + zb, zn - zb < bl ? (int)(zn - zb) : (int)bl);
         __syncthreads();
     }
 }
 
-__global__ void __launch_bounds__(1024) fa_k_carry_fused(const uint8_t* __restrict__ flags,
-                                                         const uint8_t* __restrict__ agg,
+__global__ void __launch_bounds__(1024) fa_k_carry_fused(const uint8_t* __restrict__ agg,
                                                          uint64_t* __restrict__ z, uint64_t zn,
-                                                         int own, uint64_t ngroups, uint64_t nblk)
+                                                         uint32_t bl, uint64_t nblk)
 {
-    fa_carry_resolve(flags, agg, z, zn, own, ngroups, nblk, blockIdx.x, gridDim.x);
+    const uint64_t b0 = (uint64_t)blockIdx.x * blockDim.x;
+    fa_carry_resolve(agg, z, zn, bl, nblk, b0, b0 + blockDim.x < nblk ? b0 + blockDim.x : nblk);
 }
 
-// workgroups of the carry kernel for nblk CRT workgroups: one per 32 blocks,
-// at most 256
-static unsigned carry_grid(uint64_t nblk)
+// one block per thread; a single block has no carry to receive
+static void launch_carry(const uint8_t* agg, uint64_t* z, uint64_t zn, int own, uint64_t nblk,
+                         hipStream_t s)
 {
-    const uint64_t g = nblk / 32;
-    return (unsigned)(g < 1 ? 1 : g > 256 ? 256 : g);
+    if (nblk < 2) return;
+    const unsigned nt = nblk < 1024 ? (unsigned)((nblk + 63) & ~UINT64_C(63)) : 1024u;
+    FA_LAUNCH("fa_k_carry_fused", fa_k_carry_fused, dim3((unsigned)((nblk + nt - 1) / nt)),
+              dim3(nt), 0, s, agg, z, zn, (uint32_t)(FA_CRT16_GROUPS - 1) * (uint32_t)own, nblk);
 }
 
 // ------------------------------------------------------------------------
-// CRT on the FP64 lanes (fa_crt_fp.h), 31 groups of 8 coefficients per
-// workgroup of 256 threads plus one halo group in front (its overhang
-// reaches the first group).
-//   1. thread t: coefficient 8 g0 + t -> NL limbs, shifted left by
-//      (bits * (t mod 8)) mod 64 into NLS = NL + 1 limbs in LDS;
-//   2. lanes (group gl, limb q), 32 lanes per group: the sum of the <= 8
-//      shifted coefficients overlapping limb q of the group, then the
-//      group's carries: limb q gets the carry count of limb q-1, and the
-//      single-bit overflows ripple through all-ones limbs, resolved at once
-//      from the wave's ballot masks (generate G, propagate P: the carries
-//      in are (G + (G|P)) ^ (G|P) ^ G);
-//   3. lanes (group gl >= 1, limb q < own): owned limb q plus limb own + q
-//      of the previous group (its overhang, which fits in own limbs), the
-//      same mask carry resolution, the store, and the group's flag
-//      (generate: carry out of the owned limbs, propagate: all ones).
+// CRT on the FP64 lanes (fa_crt_fp.h).  A workgroup of 256 threads takes 248
+// coefficients (31 groups of 8, whose 8 bits are whole limbs) and, in front
+// of them, a halo of the 8 before.  With chunks of own = bits / 8 bytes, a
+// coefficient of up to 50 NP / 8 bytes reaches into the chunks after its own:
+//   1. thread t: coefficient t -> its 32-bit words, as a row of LDS;
+//   2. thread t sums what falls on chunk t: bytes [p own, (p + 1) own) of row
+//      t - p.  The sum is s + k 2^bits, k < 7; k goes to chunk t + 1, and T =
+//      s + k stays below 2^bits + 7;
+//   3. T generates a carry when it reaches 2^bits, propagates when it is
+//      2^bits - 1: the carries of a wave come from its ballots, those between
+//      the four waves from their masks in LDS;
+//   4. the chunks go to LDS as one run of bytes and to z as limbs, coalesced.
+// All carries inside the workgroup are resolved; one aggregate byte tells
+// fa_carry_resolve the carry out (bit 0) and whether all limbs are ones.
+// The earlier form shifted each coefficient to limb boundaries and summed
+// limbs with 32 lanes per group (17 to 22 of them busy at 136 bits), with
+// single-bit flags per group for the carry kernel.
+// Measured before and now: 2^24 x 2^24 limbs (np = 6) 366 -> 283 us, where the
+// 1.08 GB it moves take 240 us at a copy's rate; a 65,536-limb square (np =
+// 3) 7.9 -> 5.1 us.
 // ------------------------------------------------------------------------
-#define FA_CRTFP_TL 32   // max limbs of a group's sum: 7*200/64 + 8 + 1
-
-FA_DEV uint32_t fa_seg_ballot(bool pred)
-{
-    const unsigned long long m = __ballot(pred);
-    return (uint32_t)(m >> (threadIdx.x & 32));
-}
-
 template <int NP, int MODE = 0>
 FA_DEV void fa_crt_fp_block(const double* __restrict__ Q, uint64_t stride,
                             const fa_crt_fp_consts& F, uint64_t zlen, int bits,
-                            uint64_t* __restrict__ z, uint64_t zn, uint64_t ngroups,
-                            uint8_t* __restrict__ flags, uint8_t* __restrict__ agg, uint64_t blk,
-                            uint64_t jlo = 0)
+                            uint64_t* __restrict__ z, uint64_t zn, uint8_t* __restrict__ agg,
+                            uint64_t blk, uint64_t jlo = 0)
 {
-    constexpr int NL = fa_crt_fp_dims<NP>::NL;
-    constexpr int NLS = NL + 1;
-    __shared__ uint64_t sC[256 * NLS];
-    __shared__ uint64_t sR[FA_CRT16_GROUPS][FA_CRTFP_TL];
-    __shared__ uint8_t sF[FA_CRT16_GROUPS];
-    const int t = threadIdx.x;
+    constexpr int NW = fa_crt_fp_dims<NP>::NW, NB = fa_crt_fp_dims<NP>::NB;
+    constexpr int RS = NW | 1;                 // odd row stride: no bank conflicts
+    constexpr int OWX = (25 * NP / 8) / 4 + 1; // words of a chunk and its overflow
+    __shared__ uint64_t sBuf[128 * RS];        // rows, later the output bytes
+    __shared__ uint32_t sK[256];
+    __shared__ uint64_t sG[4], sP[4];
+    uint32_t* sW = (uint32_t*)sBuf;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int own = bits >> 3;
-    const int TL = ((7 * bits) >> 6) + NLS;
-    const int ovh = TL - own;
-    const int64_t g0 = (int64_t)blk * (FA_CRT16_GROUPS - 1) - 1;
+    const int64_t j0 = (int64_t)blk * (8 * (FA_CRT16_GROUPS - 1)) - 8;
 
-    {   // 1. the coefficient of thread t, shifted to its bit offset in the group
-        //    (coefficients below jlo read as zero)
-        const int64_t j = g0 * 8 + t;
-        uint64_t L[NL];
+    {   // 1. (coefficients below jlo read as zero)
+        const int64_t j = j0 + t;
+        uint32_t W[NW];
         if (j >= (int64_t)jlo && (uint64_t)j < zlen) {
-            fa_crt_fp_value<NP, MODE>(Q, stride, (uint64_t)j, F, L);
+            fa_crt_fp_value<NP, MODE>(Q, stride, (uint32_t)j, F, W);
         } else {
 #pragma unroll
-            for (int l = 0; l < NL; l++) L[l] = 0;
+            for (int l = 0; l < NW; l++) W[l] = 0;
         }
-        const int sh = (bits * (t & 7)) & 63;
-        uint64_t* o = sC + t * NLS;
-        uint64_t prev = 0;
 #pragma unroll
-        for (int l = 0; l < NL; l++) {
-            o[l] = (L[l] << sh) | (sh ? (prev >> (64 - sh)) : 0);
-            prev = L[l];
-        }
-        o[NL] = sh ? (prev >> (64 - sh)) : 0;
+        for (int l = 0; l < NW; l++) sW[t * RS + l] = W[l];
     }
-
-    // the coefficients k overlapping limb q: o_k <= q < o_k + NLS with
-    // o_k = (bits k) >> 6, k in [kmin, kmax] (at most 8 of them)
-    const int q = t & 31, seg = t >> 5;
-    const bool qin = q < TL;
-    int kmax = (64 * q + 63) / bits;
-    if (kmax > 7) kmax = 7;
-    int kmin = 0;
-    if (q >= NLS) kmin = (64 * (q - NLS + 1) + bits - 1) / bits;
-    int offs[8];
+    // word m of a chunk: its bits below 2^bits, and the index q and shift r of
+    // the bits above
+    uint32_t mk[OWX];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const int k = kmin + e;
-        offs[e] = k * NLS + q - ((bits * k) >> 6);
-    }
-    const int nk = qin ? kmax - kmin + 1 : 0;
-    // no limb overlaps more than (64 NLS - 1) / bits + 1 coefficients: a
-    // bound the whole workgroup shares, so the loop below stops there
-    const int emax = (64 * NLS - 1) / bits + 1;
+    for (int m = 0; m < OWX; m++)
+        mk[m] = own >= 4 * m + 4 ? 0xffffffffu
+                : own <= 4 * m ? 0u : (1u << (8 * (own - 4 * m))) - 1u;
+    const int q = own >> 2, r = 8 * (own & 3);
     __syncthreads();
 
-    // 2. group sums and the carries inside each group
+    // 2. the rows before the workgroup's first lie in the halo of no owned
+    // chunk (at most 7 parts, 8 halo rows)
+    uint32_t S[OWX];
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int gl = seg + 8 * it;
-        const uint64_t* base = sC + gl * 8 * NLS;
-        uint64_t lo = 0;
-        uint32_t hi = 0;
+    for (int m = 0; m < OWX; m++) S[m] = 0;
+    for (int p = 0, off = 0; off < NB; p++, off += own) {
+        const uint32_t* row = sW + (t > p ? t - p : 0) * RS;
+        const int w0 = off >> 2, sh = off & 3;
+        uint32_t v[OWX + 1];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            if (e >= emax) break;
-            if (e < nk) {
-                const uint64_t v = base[offs[e]];
-                lo += v;
-                hi += (lo < v);
-            }
+        for (int m = 0; m <= OWX; m++) v[m] = w0 + m < NW ? row[w0 + m] : 0u;
+        unsigned cy = 0;
+#pragma unroll
+        for (int m = 0; m < OWX; m++) {
+            const uint32_t x = __builtin_amdgcn_alignbyte(v[m + 1], v[m], sh) & mk[m];
+            S[m] = __builtin_addc(S[m], x, cy, &cy);
         }
-        uint32_t hprev = __shfl_up(hi, 1, 32);
-        if (q == 0) hprev = 0;
-        const uint64_t v = lo + hprev;
-        const uint32_t G = fa_seg_ballot(qin && v < lo);
-        const uint32_t P = fa_seg_ballot(qin && v == ~UINT64_C(0));
-        const uint64_t X = (uint64_t)(G | P);
-        const uint64_t cin = ((uint64_t)G + X) ^ X ^ (uint64_t)G;
-        if (qin) sR[gl][q] = v + ((cin >> q) & 1);
     }
+    uint32_t top = 0;
+#pragma unroll
+    for (int m = 0; m < OWX; m++)
+        if (m == q) top = S[m];
+    sK[t] = top >> r;
     __syncthreads();
 
-    // 3. the previous group's overhang into the owned limbs, store, flags
+    // 3.
+    {
+        unsigned cy = 0;
+        uint32_t k = t ? sK[t - 1] : 0;
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const int gl = seg + 8 * it;
-        const int64_t g = g0 + gl;
-        const bool valid = gl >= 1 && g >= 0 && (uint64_t)g < ngroups;
-        const uint64_t zi = (uint64_t)g * own + q;
-        const bool lin = valid && q < own && zi < zn;
-        uint64_t S = 0, add = 0;
-        if (lin) {
-            add = (q < ovh) ? sR[gl - 1][own + q] : 0;
-            S = sR[gl][q] + add;
+        for (int m = 0; m < OWX; m++) {
+            S[m] = __builtin_addc(S[m] & mk[m], k, cy, &cy);
+            k = 0;
         }
-        const uint32_t G = fa_seg_ballot(lin && S < add);
-        const uint32_t P = fa_seg_ballot(lin && S == ~UINT64_C(0));
-        const uint64_t X = (uint64_t)(G | P);
-        const uint64_t cin = ((uint64_t)G + X) ^ X ^ (uint64_t)G;
-        if (lin) z[zi] = S + ((cin >> q) & 1);
-        if (q == 0 && gl >= 1) {
-            uint8_t f = 2;   // identity of the carry operator: propagate, no generate
-            if (valid) {
-                const uint32_t full = (own >= 32) ? 0xffffffffu : ((1u << own) - 1);
-                f = (uint8_t)(((cin >> own) & 1) | ((P == full) ? 2 : 0));
-                flags[g] = f;
-            }
-            sF[gl] = f;
-        }
+    }
+    uint32_t ones = 0;
+    top = 0;
+#pragma unroll
+    for (int m = 0; m < OWX; m++) {
+        ones |= S[m] ^ mk[m];
+        if (m == q) top = S[m];
+    }
+    uint64_t G = __ballot((top >> r) != 0), P = __ballot(ones == 0);
+    const uint64_t ownm = wave ? ~UINT64_C(0) : ~UINT64_C(0xff);   // owned lanes
+    G &= ownm;
+    P &= ownm;
+    if (lane == 0) {
+        sG[wave] = G;
+        sP[wave] = P | ~ownm;
     }
     __syncthreads();
-    if (t == 0) {
-        // bit 0: carry out with no carry in, bit 1: every group propagates,
-        // bit 2: some group generates a carry
-        uint8_t gg = 0, pp = 1, any = 0;
-        for (int k = 1; k < FA_CRT16_GROUPS; k++) {
-            const uint8_t ft = sF[k];
-            gg = (uint8_t)((ft & 1) | (((ft >> 1) & 1) & gg));
-            pp = (uint8_t)(pp & ((ft >> 1) & 1));
-            any = (uint8_t)(any | (ft & 1));
-        }
-        agg[blk] = (uint8_t)(gg | (pp << 1) | (any << 2));
+    uint32_t c = 0, cw = 0;
+    uint64_t all = ~UINT64_C(0);
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        if (w == wave) cw = c;
+        uint32_t o;
+        // lanes 0..7 of wave 0 neither generate nor receive (c = 0 there)
+        (void)fa_gp_carries(sG[w], w ? sP[w] : sP[w] & ~UINT64_C(0xff), c, &o);
+        c = o;
+        all &= sP[w];
     }
+    if (t == 0) agg[blk] = (uint8_t)(c | (all == ~UINT64_C(0) ? 2u : 0u));
+    uint32_t o;
+    const uint64_t cin = fa_gp_carries(G, P, cw, &o);
+    {
+        unsigned cy = (unsigned)((cin >> lane) & 1);
+#pragma unroll
+        for (int m = 0; m < OWX; m++) S[m] = __builtin_addc(S[m], 0u, cy, &cy) & mk[m];
+    }
+
+    // 4. chunk t at bytes [8 - t) own of the output: shifted to the word grid,
+    // its first word joined with the end of the chunk before (a wave's first
+    // chunk starts on a word: 56 own and 64 own are multiples of 4)
+    const int B = (t - 8) * own, sh = B & 3, w0 = B >> 2;
+    uint32_t v[OWX + 1];
+    v[0] = S[0] << (8 * sh);
+#pragma unroll
+    for (int m = 1; m <= OWX; m++)
+        v[m] = sh ? __builtin_amdgcn_alignbyte(m < OWX ? S[m] : 0u, S[m - 1], 4 - sh)
+                  : (m < OWX ? S[m] : 0u);
+    // bytes [B, B + own) end in word (B + own) >> 2 unless that is a boundary
+    const int e = (B + own) >> 2;              // first word not wholly written here
+    uint32_t tail = 0;
+#pragma unroll
+    for (int m = 0; m <= OWX; m++)
+        if (w0 + m == e) tail = v[m];
+    const uint32_t before = __shfl_up(tail, 1);
+    if (sh) v[0] |= before;
+    if (t >= 8) {
+#pragma unroll
+        for (int m = 0; m <= OWX; m++)
+            if (w0 + m < e) sW[w0 + m] = v[m];
+    }
+    __syncthreads();
+    const uint64_t base = blk * (uint64_t)((FA_CRT16_GROUPS - 1) * own);
+    const int nl = (FA_CRT16_GROUPS - 1) * own;
+    const int lim = base >= zn ? 0 : zn - base < (uint64_t)nl ? (int)(zn - base) : nl;
+    // z and agg may come from a job record: still global memory
+    typedef __attribute__((address_space(1))) uint64_t gT;
+    gT* zg = (gT*)z + base;
+    for (int i = t; i < lim; i += 256) zg[i] = sBuf[i];
 }
 
 template <int NP, int MODE = 0>
 __global__ void __launch_bounds__(256) fa_k_crt_fp(const double* __restrict__ Q, uint64_t stride,
                                                    fa_crt_fp_consts F, uint64_t zlen, int bits,
                                                    uint64_t* __restrict__ z, uint64_t zn,
-                                                   uint64_t ngroups, uint8_t* __restrict__ flags,
                                                    uint8_t* __restrict__ agg, uint64_t jlo)
 {
-    fa_crt_fp_block<NP, MODE>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, blockIdx.x,
-                              jlo);
+    fa_crt_fp_block<NP, MODE>(Q, stride, F, zlen, bits, z, zn, agg, blockIdx.x, jlo);
 }
 
 // batched CRT of integer products: work item = job | block << 32
@@ -967,8 +925,7 @@ __global__ void __launch_bounds__(256) fa_kb_crt_fp(const fa_bmpn* __restrict__ 
     if (L >= nwork) return;
     const uint64_t w = work[L];
     const fa_bmpn& m = M[(unsigned)(w & 0xffffffffu)];
-    fa_crt_fp_block<NP>(m.Q, m.stride, *F, m.zlen, m.bits, m.z, m.zn, m.ngroups, m.flags, m.agg,
-                        w >> 32);
+    fa_crt_fp_block<NP>(m.Q, m.stride, *F, m.zlen, m.bits, m.z, m.zn, m.agg, w >> 32);
 }
 
 __global__ void __launch_bounds__(1024) fa_kb_carry(const fa_bmpn* __restrict__ M,
@@ -977,7 +934,8 @@ __global__ void __launch_bounds__(1024) fa_kb_carry(const fa_bmpn* __restrict__ 
 {
     if (blockIdx.x >= njobs) return;
     const fa_bmpn& m = M[jobs[blockIdx.x]];
-    fa_carry_resolve(m.flags, m.agg, m.z, m.zn, m.bits / 8, m.ngroups, m.nblk, 0, 1);
+    fa_carry_resolve(m.agg, m.z, m.zn, (uint32_t)(FA_CRT16_GROUPS - 1) * (uint32_t)(m.bits / 8),
+                     m.nblk, 0, m.nblk);
 }
 
 int fa_batch_crt_mpn(int np, const fa_bmpn* M, const uint64_t* work, unsigned nwork,
@@ -1011,66 +969,63 @@ extern "C" FA_API void fa_set_crt_variant(int v) { fa_crt_fp_enabled = v; }
 
 template <int NP>
 static void launch_crt_fp(const double* Q, uint64_t stride, const fa_crt_fp_consts& F,
-                          uint64_t zlen, int bits, uint64_t* z, uint64_t zn, uint64_t ngroups,
-                          uint8_t* flags, uint8_t* agg, uint64_t nblk, hipStream_t s,
+                          uint64_t zlen, int bits, uint64_t* z, uint64_t zn, uint8_t* agg,
+                          uint64_t nblk, hipStream_t s,
                           int mode = 0, uint64_t jlo = 0)
 {
     if (mode == 1)
         FA_LAUNCH("fa_k_crt_fp", (fa_k_crt_fp<NP, 1>), dim3((unsigned)nblk), dim3(256), 0, s, Q,
-                  stride, F, zlen, bits, z, zn, ngroups, flags, agg, jlo);
+                  stride, F, zlen, bits, z, zn, agg, jlo);
     else if (mode == 2)
         FA_LAUNCH("fa_k_crt_fp", (fa_k_crt_fp<NP, 2>), dim3((unsigned)nblk), dim3(256), 0, s, Q,
-                  stride, F, zlen, bits, z, zn, ngroups, flags, agg, jlo);
+                  stride, F, zlen, bits, z, zn, agg, jlo);
     else
         FA_LAUNCH("fa_k_crt_fp", fa_k_crt_fp<NP>, dim3((unsigned)nblk), dim3(256), 0, s, Q,
-                  stride, F, zlen, bits, z, zn, ngroups, flags, agg, jlo);
+                  stride, F, zlen, bits, z, zn, agg, jlo);
 }
 
 template <int NP>
 static void launch_crt16(const double* Q, uint64_t stride, const fa_crt_consts& C, uint64_t zlen,
-                         int bits, uint64_t* z, uint64_t zn, uint64_t ngroups, uint8_t* flags,
-                         uint8_t* agg, uint64_t nblk, hipStream_t s)
+                         int bits, uint64_t* z, uint64_t zn, uint64_t ngroups, uint8_t* agg,
+                         uint64_t nblk, hipStream_t s)
 {
     FA_LAUNCH("fa_k_crt_mpn16", fa_k_crt_mpn16<NP>, dim3((unsigned)nblk), dim3(256), 0, s, Q,
-              stride, C, zlen, bits, z, zn, ngroups, flags, agg);
+              stride, C, zlen, bits, z, zn, ngroups, agg);
 }
 
 // mode: 0 the CRT value c in [0, M); 1, 2 the positive and negated
 // negative parts of the centred value (FP64 route only)
 static int crt16(int np, const double* Q, uint64_t stride, const fa_crt_consts& C, uint64_t zlen,
-                 int bits, uint64_t* z, uint64_t zn, uint64_t ngroups, uint8_t* flags, uint8_t* agg,
-                 uint8_t* cin, uint64_t nblk, hipStream_t s, int mode = 0, uint64_t jlo = 0)
+                 int bits, uint64_t* z, uint64_t zn, uint64_t ngroups, uint8_t* agg,
+                 uint64_t nblk, hipStream_t s, int mode = 0, uint64_t jlo = 0)
 {
     if (fa_crt_fp_enabled || mode || jlo) {
         fa_crt_fp_consts F;
         fa_crt_fp_consts_init(&F, C);
         switch (np) {
-        case 2: launch_crt_fp<2>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 3: launch_crt_fp<3>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 4: launch_crt_fp<4>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 5: launch_crt_fp<5>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 6: launch_crt_fp<6>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 7: launch_crt_fp<7>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
-        case 8: launch_crt_fp<8>(Q, stride, F, zlen, bits, z, zn, ngroups, flags, agg, nblk, s, mode, jlo); break;
+        case 2: launch_crt_fp<2>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 3: launch_crt_fp<3>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 4: launch_crt_fp<4>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 5: launch_crt_fp<5>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 6: launch_crt_fp<6>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 7: launch_crt_fp<7>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
+        case 8: launch_crt_fp<8>(Q, stride, F, zlen, bits, z, zn, agg, nblk, s, mode, jlo); break;
         default: return fa_set_error(FA_E_ARG, "crt: np %d", np);
         }
-        FA_LAUNCH("fa_k_carry_fused", fa_k_carry_fused, dim3(carry_grid(nblk)), dim3(1024), 0, s,
-                  flags, agg, z, zn, bits / 8, ngroups, nblk);
+        launch_carry(agg, z, zn, bits / 8, nblk, s);
         return FA_OK;
     }
     switch (np) {
-    case 2: launch_crt16<2>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 3: launch_crt16<3>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 4: launch_crt16<4>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 5: launch_crt16<5>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 6: launch_crt16<6>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 7: launch_crt16<7>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
-    case 8: launch_crt16<8>(Q, stride, C, zlen, bits, z, zn, ngroups, flags, agg, nblk, s); break;
+    case 2: launch_crt16<2>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 3: launch_crt16<3>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 4: launch_crt16<4>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 5: launch_crt16<5>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 6: launch_crt16<6>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 7: launch_crt16<7>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
+    case 8: launch_crt16<8>(Q, stride, C, zlen, bits, z, zn, ngroups, agg, nblk, s); break;
     default: return fa_set_error(FA_E_ARG, "crt16: np %d", np);
     }
-    (void)cin;
-    FA_LAUNCH("fa_k_carry_fused", fa_k_carry_fused, dim3(carry_grid(nblk)), dim3(1024), 0, s,
-              flags, agg, z, zn, bits / 8, ngroups, nblk);
+    launch_carry(agg, z, zn, bits / 8, nblk, s);
     return FA_OK;
 }
 
@@ -1456,13 +1411,10 @@ int fa_crt_mpn_export(int np, const double* A, uint64_t stride, uint64_t zlen, i
     void* buf;
     int rc = fa_scratch_reserve(st, bytes, &buf, stream);
     if (rc) return rc;
-    uint8_t* flags = (uint8_t*)buf;
-    uint8_t* agg = flags + ((ngroups + 7) & ~UINT64_C(7));
-    uint8_t* cin = agg + ((nblk16 + 7) & ~UINT64_C(7));
+    uint8_t* agg = (uint8_t*)buf;
     fa_crt_consts C;
     fa_crt_consts_init(&C, np, 0);
-    rc = crt16(np, A, stride, C, zlen, bits, z, zn, ngroups, flags, agg, cin, nblk16, stream,
-               mode, jlo);
+    rc = crt16(np, A, stride, C, zlen, bits, z, zn, ngroups, agg, nblk16, stream, mode, jlo);
     if (rc) return rc;
     rc = fa_buffers_leave(st, stream);
     if (rc) return rc;
@@ -1482,8 +1434,6 @@ static int mpn_mul_run(uint64_t* z, const uint64_t* a, uint64_t an, const uint64
     W.A = (double*)buf;
     W.B = (double*)((char*)buf + tr);
     W.flags = (uint8_t*)((char*)buf + 2 * tr);
-    // aggregates start on an 8-byte boundary: the carry kernel reads them
-    // as 64-bit words
     W.agg = W.flags + ((ngroups + 7) & ~UINT64_C(7));
     W.cin = W.agg + (((ngroups + 29) / 30 + 7) & ~UINT64_C(7));
 
@@ -1497,8 +1447,7 @@ static int mpn_mul_run(uint64_t* z, const uint64_t* a, uint64_t an, const uint64
     const uint64_t stride = fa_res_stride(P.depth);
     if (fa_fast_enabled) {
         uint64_t nblk16 = (ngroups + (FA_CRT16_GROUPS - 2)) / (FA_CRT16_GROUPS - 1);
-        rc = crt16(P.np, W.A, stride, C, P.zlen, P.bits, z, zn, ngroups, W.flags, W.agg, W.cin,
-                   nblk16, stream);
+        rc = crt16(P.np, W.A, stride, C, P.zlen, P.bits, z, zn, ngroups, W.agg, nblk16, stream);
         if (rc) return rc;
         LAUNCH_CHECK();
         return FA_OK;

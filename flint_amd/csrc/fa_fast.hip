@@ -580,12 +580,16 @@ __global__ void __launch_bounds__(256) fa_k_row_conv16(double* __restrict__ A,
 // 5.1 us; 64 batched fmpz products, 2^20 points, 913 + 389 -> 761 + 346 us (a
 // copy's rate, 5.3 TB/s, in the inverse pass; the forward pass waits on the
 // reads of its limb rows, without which it takes 363 us).
-template <int D1>
+//
+// D2 < 12: shorter rows (the short-row path below).  A tile is then at least
+// one wave, 16 columns wide where that is more.
+template <int D1, int D2 = FA_ROW_LG>
 struct col_geom {
     static constexpr int R = (D1 >= 4) ? (D1 % 4) : D1;   // levels of the partial stage
     static constexpr int NS = (D1 >= 4) ? (D1 / 4) : 0;   // radix-16 stages
     static constexpr int TPC = (D1 >= 4) ? (1 << (D1 - 4)) : 1;
-    static constexpr int CPW = D1 <= 8 ? 256 / TPC : D1 == 9 ? 16 : D1 <= 11 ? 8 : 4;
+    static constexpr int CPW = D2 < FA_ROW_LG ? (TPC < 4 ? 64 / TPC : 16)
+                               : D1 <= 8 ? 256 / TPC : D1 == 9 ? 16 : D1 <= 11 ? 8 : 4;
     static constexpr int NT = CPW * TPC;                  // threads
     static constexpr int LEN = 1 << D1;
     static constexpr int PLEN = LEN + LEN / 16;
@@ -615,6 +619,15 @@ struct col_geom {
         return PADX(pos(j, tc, 0)) + PADX(d);
     }
 };
+
+// offset of row r of a residue array: rows of 4096 points at the pitch, or
+// 2^(12-D2) rows of 2^D2 points in each of them
+template <int D2>
+FA_DEV constexpr uint32_t fa_row_off(uint32_t r)
+{
+    constexpr int L = FA_ROW_LG - D2;
+    return (r >> L) * FA_ROW_PITCH + ((r & ((1u << L) - 1)) << D2);
+}
 
 // the first R (1..3) levels of a radix-16 group of a column (block 0, roots
 // w2[0..3]) on imported values: level 0 pairs (k, k+8), level 1 (k, k+4),
@@ -741,12 +754,12 @@ FA_DEV unsigned fa_xcd_linear()
 }
 
 // import and first stage (or, below 16 points, the whole column)
-template <int D1, int KIND, bool HZ>
+template <int D1, int KIND, bool HZ, int D2>
 FA_DEV void fa_col_fwd_first(double* x, const fa_operand& op, uint32_t e0, double n, double ninv,
                              const double* __restrict__ w2, const double* __restrict__ pow2)
 {
-    typedef col_geom<D1> G;
-    constexpr uint32_t step = 1u << (FA_ROW_LG + (D1 >= 4 ? D1 - 4 : 0));
+    typedef col_geom<D1, D2> G;
+    constexpr uint32_t step = 1u << (D2 + (D1 >= 4 ? D1 - 4 : 0));
     fa_import_column<(HZ ? G::NEL / 2 : G::NEL), KIND>(x, op, e0, step, pow2, n, ninv);
     if (HZ) {
 #pragma unroll
@@ -759,23 +772,23 @@ FA_DEV void fa_col_fwd_first(double* x, const fa_operand& op, uint32_t e0, doubl
 
 // first D1 levels of column group g (CPW columns) of one residue array:
 // import, forward, store.  lds holds CPW * PLEN doubles.
-template <int D1, int KIND>
+template <int D1, int KIND, int D2 = FA_ROW_LG>
 FA_DEV void fa_col_fwd_tile(const fa_operand& op, double* __restrict__ dst, int g,
                             double n, double ninv, const double* __restrict__ w2,
                             const double* __restrict__ pow2, double* lds, int trows)
 {
-    typedef col_geom<D1> G;
+    typedef col_geom<D1, D2> G;
     const int c = threadIdx.x % G::CPW, tc = threadIdx.x / G::CPW;
     const uint32_t col = (uint32_t)(g * G::CPW + c);
     double* my = lds + c;   // column c of the interleaved LDS rows
     double x[16], tw[15];
     // the upper half of every column zero: the usual case of a product's
     // operands, each at most half the transform length
-    const uint32_t e0 = ((uint32_t)G::pos(0, tc, 0) << FA_ROW_LG) + col;
-    if (fa_operand_fits(op, 1u << (D1 + FA_ROW_LG - 1)))
-        fa_col_fwd_first<D1, KIND, true>(x, op, e0, n, ninv, w2, pow2);
+    const uint32_t e0 = ((uint32_t)G::pos(0, tc, 0) << D2) + col;
+    if (fa_operand_fits(op, 1u << (D1 + D2 - 1)))
+        fa_col_fwd_first<D1, KIND, true, D2>(x, op, e0, n, ninv, w2, pow2);
     else
-        fa_col_fwd_first<D1, KIND, false>(x, op, e0, n, ninv, w2, pow2);
+        fa_col_fwd_first<D1, KIND, false, D2>(x, op, e0, n, ninv, w2, pow2);
     if constexpr (D1 >= 4) {
 #pragma unroll
         for (int j = 1; j < G::NSTAGE; j++) {
@@ -793,11 +806,11 @@ FA_DEV void fa_col_fwd_tile(const fa_operand& op, double* __restrict__ dst, int 
     const int jl = (D1 < 4) ? 0 : G::NSTAGE - 1;
     // rows at or past trows are not read by a truncated product
     const int r0 = G::pos(jl, tc, 0);
-    const uint32_t at = ((uint32_t)r0 * FA_ROW_PITCH + col) * 8u;
+    const uint32_t at = (fa_row_off<D2>(r0) + col) * 8u;
     // (the last stage of a column ends at level D1: consecutive rows)
 #pragma unroll
     for (int k = 0; k < G::NEL; k++)
-        if (r0 + k < trows) fa_st(dst + k * FA_ROW_PITCH, at, x[k]);
+        if (r0 + k < trows) fa_st(dst + fa_row_off<D2>(k), at, x[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -913,19 +926,19 @@ FA_DEV void fa_col_inv_trunc_tile(double* __restrict__ dst, int g, int t, double
     }
 }
 
-template <int D1>
+template <int D1, int D2 = FA_ROW_LG>
 FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int g, double n, double ninv,
                             const double* __restrict__ wi, double* lds)
 {
-    typedef col_geom<D1> G;
+    typedef col_geom<D1, D2> G;
     const int c = threadIdx.x % G::CPW, tc = threadIdx.x / G::CPW;
     const uint32_t col = (uint32_t)(g * G::CPW + c);
     double* my = lds + c;   // column c of the interleaved LDS rows
     double x[16], tw[15];
     const int jl = (D1 < 4) ? 0 : G::NSTAGE - 1;
-    const uint32_t in = ((uint32_t)G::pos(jl, tc, 0) * FA_ROW_PITCH + col) * 8u;
+    const uint32_t in = (fa_row_off<D2>(G::pos(jl, tc, 0)) + col) * 8u;
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++) x[k] = fa_ld<double>(dst + k * FA_ROW_PITCH, in);
+    for (int k = 0; k < G::NEL; k++) x[k] = fa_ld<double>(dst + fa_row_off<D2>(k), in);
     if constexpr (D1 < 4) {
         fa_inv_small_col<D1>(x, wi, n, ninv);
     } else {
@@ -948,10 +961,10 @@ FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int g, double n, double ni
             }
         }
     }
-    const uint32_t out = ((uint32_t)G::pos(0, tc, 0) * FA_ROW_PITCH + col) * 8u;
-    constexpr uint32_t rs = (D1 < 4 ? 1u : 1u << (D1 - 4)) * FA_ROW_PITCH;
+    const uint32_t out = (fa_row_off<D2>(G::pos(0, tc, 0)) + col) * 8u;
+    constexpr uint32_t rs = 1u << (D1 < 4 ? 0 : D1 - 4);   // rows between elements
 #pragma unroll
-    for (int k = 0; k < G::NEL; k++) fa_st(dst + k * rs, out, x[k]);
+    for (int k = 0; k < G::NEL; k++) fa_st(dst + fa_row_off<D2>(k * rs), out, x[k]);
 }
 
 // Work order of the column passes: blocks of `lines` adjacent column groups
@@ -1019,6 +1032,140 @@ fa_k_col_inv16(double* __restrict__ A, uint64_t stride, fa_prime_set S, int np, 
                                   S.w2inv[i], lds);
     else
         fa_col_inv_tile<D1>(A + (uint64_t)i * stride, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
+}
+
+// ---------------------------------------------------------------------------
+// Short rows.  A single product of up to 2^18 points has too few rows of 4096
+// to fill the GPU: 2^13 points modulo four primes are eight row workgroups,
+// each 13 us of dependent work.  There the transform is split into columns of
+// 2^D1 points and rows of 2^D2 = 256 or 1024: a row is radix-4 stages of four
+// elements per thread, and all twiddles are read from the tables (2^(depth-1)
+// entries, in L2) instead of formed.  Residue arrays keep their layout, so
+// the import, the CRT and the exports are unchanged.  Each kernel is latency
+// bound (a dependent chain of loads, some 500 vector instructions and LDS
+// exchanges); measured with rows of 4096 and now: the row kernel of 6000 x
+// 5000 limbs 13.1 -> 4.3 us, of a 65,536-limb square 11.7 -> 7.2 us (columns
+// 8.0 + 4.8 -> 6.6 + 4.5).  Rows of 16 elements per thread took 7.0 us at 2^13
+// points.
+// ---------------------------------------------------------------------------
+template <int D1, int D2>
+constexpr int fa_short_nt() { return col_geom<D1, D2>::NT; }
+
+template <int D1, int D2, int KIND>
+__global__ void __launch_bounds__((fa_short_nt<D1, D2>()))
+fa_k_col_fwd_s(fa_operand a, fa_operand b, double* __restrict__ A, double* __restrict__ B,
+               uint64_t stride, fa_prime_set S, int np, int nops)
+{
+    typedef col_geom<D1, D2> G;
+    constexpr int NG = (1 << D2) / G::CPW;
+    __shared__ double lds[G::LDS];
+    int i, g, z;
+    fa_col_split<G::CPW, (1 << D2)>(fa_xcd_linear(), np, NG, &i, &g, &z);
+    if (z >= nops) return;
+    fa_col_fwd_tile<D1, KIND, D2>(z ? b : a, (z ? B : A) + (uint64_t)i * stride, g, S.p[i],
+                                  S.pinv[i], S.w2[i], S.pow2[i], lds, 1 << D1);
+}
+
+template <int D1, int D2>
+__global__ void __launch_bounds__((fa_short_nt<D1, D2>()))
+fa_k_col_inv_s(double* __restrict__ A, uint64_t stride, fa_prime_set S, int np)
+{
+    typedef col_geom<D1, D2> G;
+    constexpr int NG = (1 << D2) / G::CPW;
+    __shared__ double lds[G::LDS];
+    int i, g, z;
+    fa_col_split<G::CPW, (1 << D2)>(fa_xcd_linear(), np, NG, &i, &g, &z);
+    if (z >= 1) return;
+    fa_col_inv_tile<D1, D2>(A + (uint64_t)i * stride, g, S.p[i], S.pinv[i], S.w2inv[i], lds);
+}
+
+// A row of 2^D2 points by 2^(D2-2) threads: D2 / 2 radix-4 stages.  At stage st
+// thread t owns, in block b of level 2 st, the positions
+// (b << (D2 - 2 st)) + i0 + (k << (D2 - 2 - 2 st)), k < 4.
+template <int D2>
+FA_DEV int fa_srow_pos(int st, int t, int k)
+{
+    const int sh = D2 - 2 - 2 * st;
+    const int p = ((t >> sh) << (sh + 2)) + (t & ((1 << sh) - 1)) + (k << sh);
+    return PADX(p);
+}
+
+template <int D2>
+FA_DEV void fa_srow_swap(double* x, double* s, int t, int from, int to)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++) s[fa_srow_pos<D2>(from, t, k)] = x[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = s[fa_srow_pos<D2>(to, t, k)];
+    __syncthreads();
+}
+
+// the twiddles of each stage: w[Q], w[2Q], w[2Q+1] of block Q = (r << 2 st) + b
+template <int D2>
+FA_DEV void fa_srow_tw(const double* __restrict__ w, uint32_t r, int t, double tw[D2 / 2][3])
+{
+#pragma unroll
+    for (int st = 0; st < D2 / 2; st++) {
+        const uint32_t Q = (r << (2 * st)) + (uint32_t)(t >> (D2 - 2 - 2 * st));
+        tw[st][0] = w[Q];
+        tw[st][1] = w[2 * Q];
+        tw[st][2] = w[2 * Q + 1];
+    }
+}
+
+// MODE 0: forward rows of a and b, pointwise product, inverse rows, in place
+// in A; 1: the same for a square; 2: forward only; 3: inverse only.  The
+// forward transform's element k of thread t is stored at t + 2^(D2-2) k
+// (pointwise operations do not mind the order).  blockIdx.x = row, y = prime
+template <int MODE, int D2>
+__global__ void __launch_bounds__(1 << (D2 - 2)) fa_k_row_s(double* __restrict__ A,
+                                                            const double* __restrict__ B,
+                                                            uint64_t stride, fa_prime_set S)
+{
+    constexpr int NT = 1 << (D2 - 2), LEN = 4 * NT + NT / 4, NS = D2 / 2;
+    __shared__ double sx[LEN], sy[MODE == 0 ? LEN : 1];
+    const int i = blockIdx.y, t = threadIdx.x;
+    const uint32_t r = blockIdx.x;
+    const double n = S.p[i], ninv = S.pinv[i];
+    double* a = A + (uint64_t)i * stride + fa_row_off<D2>(r);
+    const double* b = B + (uint64_t)i * stride + fa_row_off<D2>(r);
+    double x[4], y[4], tw[NS][3], ti[NS][3];
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = fa_ld<double>(a + NT * k, t * 8);
+    if (MODE == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = fa_ld<double>(b + NT * k, t * 8);
+    }
+    if (MODE != 3) fa_srow_tw<D2>(S.w2[i], r, t, tw);
+    if (MODE != 2) fa_srow_tw<D2>(S.w2inv[i], r, t, ti);
+    if (MODE != 3) {
+#pragma unroll
+        for (int st = 0; st < NS; st++) {
+            fa_fwd4(x[0], x[1], x[2], x[3], tw[st][0], tw[st][1], tw[st][2], n, ninv);
+            if (MODE == 0)
+                fa_fwd4(y[0], y[1], y[2], y[3], tw[st][0], tw[st][1], tw[st][2], n, ninv);
+            if (st < NS - 1) {
+                fa_srow_swap<D2>(x, sx, t, st, st + 1);
+                if (MODE == 0) fa_srow_swap<D2>(y, sy, t, st, st + 1);
+            }
+        }
+        if (MODE != 2) {
+            const double m = S.norm[i];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                x[k] = fa_mulmod(fa_mulmod(x[k], m, n, ninv), MODE == 0 ? y[k] : x[k], n, ninv);
+        }
+    }
+    if (MODE != 2) {
+#pragma unroll
+        for (int st = NS - 1; st >= 0; st--) {
+            fa_inv4(x[0], x[1], x[2], x[3], ti[st][0], ti[st][1], ti[st][2], n, ninv);
+            if (st > 0) fa_srow_swap<D2>(x, sx, t, st, st - 1);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) fa_st(a + NT * k, t * 8, x[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1750,6 +1897,86 @@ static int launch_forward_any(const fa_operand& oa, int np, double* A, uint64_t 
     }
 }
 
+// Single products of 2^11 .. 2^18 points take short rows.  Whole products, the
+// other path and this one, us: 2^11 points 21.9 and 20.4 (one workgroup per
+// prime in LDS; at 2^10 that path is level, 19.5), 2^12 32.1 and 20.5, 2^14
+// 25.1 and 20.7, 2^16 31.1 and 26.3, 2^17 39.3 and 35.3 (products mod a 61-bit
+// n); 2^18 63.8 and 58.8 (integers); at 2^19 points the rows of 4096 fill
+// the GPU.  The lengths of the rows are the faster ones: at 2^16 and 2^17
+// points 1024 (26.4, 35.3) against 256 (29.7, 37.8).
+#define FA_SHORT_MAX 18
+#define FA_SHORT_MIN 11
+
+template <int D1, int D2, int KIND>
+static void launch_short_fwd(const fa_operand& oa, const fa_operand& ob, int nops, int np,
+                             double* A, double* B, uint64_t stride, const fa_prime_set& S,
+                             hipStream_t s)
+{
+    typedef col_geom<D1, D2> G;
+    const unsigned grid = ((unsigned)(np * ((1 << D2) / G::CPW) * nops) + 7) & ~7u;
+    FA_LAUNCH("fa_k_col_fwd_s", (fa_k_col_fwd_s<D1, D2, KIND>), dim3(grid), dim3(G::NT), 0, s, oa,
+              ob, A, B, stride, S, np, nops);
+}
+
+template <int MODE, int D2>
+static void launch_short_row(int depth, int np, double* A, const double* B, uint64_t stride,
+                             const fa_prime_set& S, hipStream_t s)
+{
+    FA_LAUNCH("fa_k_row_s", (fa_k_row_s<MODE, D2>), dim3(1u << (depth - D2), np),
+              dim3(1 << (D2 - 2)), 0, s, A, B, stride, S);
+}
+
+// what: 0 product, 1 square, 2 forward transform, 3 inverse transform
+template <int D1, int D2>
+static int launch_short(int what, const fa_operand& oa, const fa_operand& ob, int np, double* A,
+                        double* B, uint64_t stride, const fa_prime_set& S, hipStream_t s)
+{
+    const int nops = what == 0 ? 2 : 1;
+    if (what != 3) {
+        switch (fa_pack_kind(oa, ob)) {
+        case FA_PACK_MPN8:
+            launch_short_fwd<D1, D2, FA_PACK_MPN8>(oa, ob, nops, np, A, B, stride, S, s); break;
+        case FA_PACK_U64:
+            launch_short_fwd<D1, D2, FA_PACK_U64>(oa, ob, nops, np, A, B, stride, S, s); break;
+        case FA_PACK_S64W:
+            launch_short_fwd<D1, D2, FA_PACK_S64W>(oa, ob, nops, np, A, B, stride, S, s); break;
+        default:
+            launch_short_fwd<D1, D2, FA_PACK_ANY>(oa, ob, nops, np, A, B, stride, S, s); break;
+        }
+    }
+    switch (what) {
+    case 0: launch_short_row<0, D2>(D1 + D2, np, A, B, stride, S, s); break;
+    case 1: launch_short_row<1, D2>(D1 + D2, np, A, A, stride, S, s); break;
+    case 2: launch_short_row<2, D2>(D1 + D2, np, A, A, stride, S, s); break;
+    default: launch_short_row<3, D2>(D1 + D2, np, A, A, stride, S, s); break;
+    }
+    if (what != 2) {
+        typedef col_geom<D1, D2> G;
+        const unsigned grid = ((unsigned)(np * ((1 << D2) / G::CPW)) + 7) & ~7u;
+        FA_LAUNCH("fa_k_col_inv_s", (fa_k_col_inv_s<D1, D2>), dim3(grid), dim3(G::NT), 0, s, A,
+                  stride, S, np);
+    }
+    return 1;
+}
+
+// 1 when launched, 0 for other depths
+static int fa_short(int depth, int what, const fa_operand& oa, const fa_operand& ob, int np,
+                    double* A, double* B, uint64_t stride, const fa_prime_set& S, hipStream_t s)
+{
+    if (depth < FA_SHORT_MIN || depth > FA_SHORT_MAX) return 0;
+    switch (depth) {
+    case 11: return launch_short<3, 8>(what, oa, ob, np, A, B, stride, S, s);
+    case 12: return launch_short<4, 8>(what, oa, ob, np, A, B, stride, S, s);
+    case 13: return launch_short<5, 8>(what, oa, ob, np, A, B, stride, S, s);
+    case 14: return launch_short<6, 8>(what, oa, ob, np, A, B, stride, S, s);
+    case 15: return launch_short<7, 8>(what, oa, ob, np, A, B, stride, S, s);
+    case 16: return launch_short<6, 10>(what, oa, ob, np, A, B, stride, S, s);
+    case 17: return launch_short<7, 10>(what, oa, ob, np, A, B, stride, S, s);
+    case 18: return launch_short<8, 10>(what, oa, ob, np, A, B, stride, S, s);
+    default: return 0;
+    }
+}
+
 #define FA_D1_SWITCH(d1, F)                                                                \
     switch (d1) {                                                                          \
     case 1: return F(1); case 2: return F(2); case 3: return F(3); case 4: return F(4);    \
@@ -1763,6 +1990,7 @@ static int launch_forward_any(const fa_operand& oa, int np, double* A, uint64_t 
 int fa_forward_fast(int depth, const fa_operand& oa, int np, double* A, uint64_t stride,
                     const fa_prime_set& S, hipStream_t s)
 {
+    if (fa_short(depth, 2, oa, oa, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_forward_any<D>(oa, np, A, stride, S, s)
     FA_D1_SWITCH(depth - FA_ROW_LG, FA_F)
 #undef FA_F
@@ -1771,6 +1999,7 @@ int fa_forward_fast(int depth, const fa_operand& oa, int np, double* A, uint64_t
 int fa_inverse_fast(int depth, int np, double* A, uint64_t stride, const fa_prime_set& S,
                     hipStream_t s)
 {
+    if (fa_short(depth, 3, fa_operand{}, fa_operand{}, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_inverse<D>(np, A, stride, S, s)
     FA_D1_SWITCH(depth - FA_ROW_LG, FA_F)
 #undef FA_F
@@ -1791,6 +2020,9 @@ int fa_convolve_fast(int depth, const fa_operand& oa, const fa_operand& ob, int 
         const int t = (int)((zlen + (1u << FA_ROW_LG) - 1) >> FA_ROW_LG);
         if (fa_trunc_enabled == 2 || fa_trunc_rule(d1, t)) trows = t;
     }
+    if (trows == (d1 >= 1 ? 1 << d1 : 0) &&
+        fa_short(depth, sqr ? 1 : 0, oa, ob, np, A, B, stride, S, s))
+        return 1;
 #define FA_F(D) launch_fast_any<D>(oa, ob, nops, np, A, B, stride, S, s, trows)
     FA_D1_SWITCH(d1, FA_F)
 #undef FA_F

@@ -1091,16 +1091,16 @@ int fa_convolve(fa_thread_state* st, const fa_tables* T, int np, int offset, int
     // transform per prime
     const int sqr = fa_sqr_enabled && a->kind == b->kind && a->src == b->src && a->n == b->n &&
                     a->bits == b->bits && a->width == b->width;
+    const uint64_t la = desc_len(a), lb = desc_len(b);
+    const uint64_t zlen = la && lb ? la + lb - 1 : 0;
+    if (fa_fast_enabled && fa_convolve_fast(depth, oa, ob, np, A, B, stride, S, stream, sqr, zlen)) {
+        LAUNCH_CHECK();
+        return FA_OK;
+    }
     if (depth <= FA_ROW_LG) {
         size_t lds = (sqr ? 1 : 2) * stride * sizeof(double);
         FA_LAUNCH("fa_k_small_conv", fa_k_small_conv, dim3(np), dim3(256), lds, stream, oa, ob,
                   depth, A, stride, S, sqr);
-        LAUNCH_CHECK();
-        return FA_OK;
-    }
-    const uint64_t la = desc_len(a), lb = desc_len(b);
-    const uint64_t zlen = la && lb ? la + lb - 1 : 0;
-    if (fa_fast_enabled && fa_convolve_fast(depth, oa, ob, np, A, B, stride, S, stream, sqr, zlen)) {
         LAUNCH_CHECK();
         return FA_OK;
     }

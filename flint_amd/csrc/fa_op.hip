@@ -418,11 +418,13 @@ static int forward(fa_op_struct* X, const fa_operand& op, const fa_plan_struct* 
     hipStream_t s = stream_of(stream);
     fa_prime_set S;
     fa_prime_set_init(&S, T, P->np, P->depth, P->offset, 1);
-    if (P->depth <= FA_ROW_LG) {
+    if (fa_forward_fast(P->depth, op, P->np, X->data, X->stride, S, s)) {
+        // launched
+    } else if (P->depth <= FA_ROW_LG) {
         FA_LAUNCH("fa_k_op_small_fwd", fa_k_op_small_fwd, dim3(P->np), dim3(256),
                   ((size_t)1 << P->depth) * sizeof(double), s, op, P->depth, X->data, X->stride,
                   S);
-    } else if (!fa_forward_fast(P->depth, op, P->np, X->data, X->stride, S, s)) {
+    } else {
         return fa_set_error(FA_E_RANGE, "forward transform: depth %d", P->depth);
     }
     X->domain = FA_OP_PRIMAL;
@@ -536,10 +538,12 @@ extern "C" int fa_ifft(fa_op_struct* X, const fa_plan_struct* P, void* stream)
     hipStream_t s = stream_of(stream);
     fa_prime_set S;
     fa_prime_set_init(&S, T, P->np, P->depth, P->offset, 1);
-    if (P->depth <= FA_ROW_LG) {
+    if (fa_inverse_fast(P->depth, P->np, X->data, X->stride, S, s)) {
+        // launched
+    } else if (P->depth <= FA_ROW_LG) {
         FA_LAUNCH("fa_k_op_small_inv", fa_k_op_small_inv, dim3(P->np), dim3(256),
                   ((size_t)1 << P->depth) * sizeof(double), s, X->data, P->depth, X->stride, S);
-    } else if (!fa_inverse_fast(P->depth, P->np, X->data, X->stride, S, s)) {
+    } else {
         return fa_set_error(FA_E_RANGE, "inverse transform: depth %d", P->depth);
     }
     X->domain = FA_OP_COEFF;

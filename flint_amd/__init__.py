@@ -330,7 +330,7 @@ def set_fast_kernels(on=True):
 
 
 def set_row_variant(v):
-    """row pass of the two-level transforms: 1 = three workgroups per CU,
+    """row pass of the two-level transforms: 1 = four workgroups per CU,
     last-stage twiddles formed per layer (default); 0 = two, all held"""
     lib().fa_set_row_variant(int(v))
 

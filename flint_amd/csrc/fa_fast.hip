@@ -226,6 +226,7 @@ FA_DEV void fa_row_tw_last(const double* rho, const double* __restrict__ w, int 
 
 // radix-16 stage j < 2 of block bq with each radix-4 layer's twiddles read
 // from the LDS table just before the layer
+template <bool R2 = true>
 FA_DEV void fa_fwd16_rowtab(double* x, const double* tab, int j, int bq, double n, double ninv)
 {
     const int m = 4 * j;
@@ -242,7 +243,10 @@ FA_DEV void fa_fwd16_rowtab(double* x, const double* tab, int j, int bq, double 
         const double T0 = tab[(4 << m) - 1 + Qp];
         const double T1 = tab[(8 << m) - 1 + 2 * Qp];
         const double T2 = tab[(8 << m) - 1 + 2 * Qp + 1];
-        fa_fwd4(x[4 * jj], x[4 * jj + 1], x[4 * jj + 2], x[4 * jj + 3], T0, T1, T2, n, ninv);
+        if (R2)
+            fa_fwd4(x[4 * jj], x[4 * jj + 1], x[4 * jj + 2], x[4 * jj + 3], T0, T1, T2, n, ninv);
+        else
+            fa_fwd4_nr(x[4 * jj], x[4 * jj + 1], x[4 * jj + 2], x[4 * jj + 3], T0, T1, T2, n, ninv);
     }
 }
 
@@ -266,7 +270,7 @@ FA_DEV void fa_inv16_rowtab(double* x, const double* tab, int j, int bq, double 
 
 // the last radix-16 stage (levels 8..11 of block t) with its twiddles formed
 // just before each radix-4 layer: fewer registers live across the row
-// transforms than with all 15 held (three workgroups share a CU)
+// transforms than with all 15 held (the row passes share a CU four or three at a time)
 FA_DEV void fa_fwd16_rowlast(double* x, const double* rho, const double* __restrict__ w, int t,
                              double n, double ninv)
 {
@@ -321,18 +325,18 @@ FA_DEV void fa_fwd4096_row(double* x, double* xch, const double* tab, const doub
     fa_row_tw(tab, 0, 0, tw);
     fa_fwd16(x, tw, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(t + 256 * k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[t + (t >> 4) + 272 * k] = x[k];
     __syncthreads();
     const int b = t >> 4, i0 = t & 15;
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(256 * b + i0 + 16 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[272 * b + i0 + 17 * k];
     fa_row_tw(tab, 1, b, tw);
     fa_fwd16(x, tw, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(16 * t + k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[17 * t + k];
     fa_fwd16(x, twl, n, ninv);
     __syncthreads();
 }
@@ -344,18 +348,18 @@ FA_DEV void fa_inv4096_row(double* x, double* xch, const double* tab, const doub
     double tw[15];
     fa_inv16(x, twl, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(16 * t + k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[17 * t + k] = x[k];
     __syncthreads();
     const int b = t >> 4, i0 = t & 15;
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(256 * b + i0 + 16 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[272 * b + i0 + 17 * k];
     fa_row_tw(tab, 1, b, tw);
     fa_inv16(x, tw, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(t + 256 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[t + (t >> 4) + 272 * k];
     fa_row_tw(tab, 0, 0, tw);
     fa_inv16(x, tw, n, ninv);
 }
@@ -387,9 +391,25 @@ FA_DEV void fa_row_conv_tile(double* __restrict__ arow, const double* __restrict
     for (int k = 0; k < 16; k++) arow[t + 256 * k] = x[k];
 }
 
-// fa_row_conv_tile with the last-stage twiddles formed on the fly.
-// SQR: a square (brow unused): one forward transform, pointwise x^2
-// (mpn_mul.c:1425-1452, sd_fft_ctx_point_sqr)
+// fa_row_conv_tile with the last-stage twiddles formed on the fly, once for
+// both operands: a and b go through stages 0 and 1 one after the other, then
+// each radix-4 layer of the last stage takes both, and its second layer runs
+// into the pointwise product and the first inverse layer four points at a
+// time.  SQR: a square (brow unused): one forward transform, pointwise x^2
+// (mpn_mul.c:1425-1452, sd_fft_ctx_point_sqr).
+//
+// Bound by FP64 issue (97% of its vector instructions; VALU busy 74% before).
+// 2,978 vector instructions per wave instead of 3,364, and 128 registers
+// instead of 158, so four workgroups share a CU instead of three: three primes
+// of the 2^24-point product (12,288 rows) 440 -> 382 us.  LDS addresses are a
+// lane base plus constants: computed per element they held registers that
+// spilled.  Ranges in units of n
+// (mulmod: P n^2 -> 1/2 + P'/4, see fa_fwd16): stages 0 and 1 reduce in their
+// first layer only and end at 6; the last stage's second layer reduces and
+// takes 3.5 to 3 with twiddles that are not reduced after their product (at
+// most 1/2 + 1/16: 3.5 * 0.5625 < 2, 4.5 * 0.5625 < 4); m a b lands below 1.5,
+// so the first inverse layer may use such twiddles too (6 * 0.5625 < 4) and
+// ends below 2, the range of the inverse.
 template <bool SQR = false>
 FA_DEV void fa_row_conv_tile_lr(double* __restrict__ arow, const double* __restrict__ brow,
                                 uint64_t r, double n, double ninv, double m,
@@ -399,65 +419,112 @@ FA_DEV void fa_row_conv_tile_lr(double* __restrict__ arow, const double* __restr
     const int t = threadIdx.x;
     const int b = t >> 4, i0 = t & 15;
     double x[16], y[16];
+    // both rows are requested before the table is built
+    if (!SQR) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) y[k] = fa_ld<double>(brow + 256 * k, t * 8);
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = fa_ld<double>(arow + 256 * k, t * 8);
+    if (t >= 16 && t < 28) rho[t] = w2inv[r << (t - 16)];
     fa_build_row_table(tab, w2, r, rho, n, ninv);
 #pragma unroll
     for (int z = SQR ? 1 : 0; z < 2; z++) {
         double* v = z ? x : y;
-        const double* src = z ? arow : brow;
-        __builtin_amdgcn_sched_barrier(0);
+        fa_fwd16_rowtab<false>(v, tab, 0, 0, n, ninv);
 #pragma unroll
-        for (int k = 0; k < 16; k++) v[k] = fa_ld<double>(src + 256 * k, t * 8);
-        fa_fwd16_rowtab(v, tab, 0, 0, n, ninv);
-#pragma unroll
-        for (int k = 0; k < 16; k++) xch[PADX(t + 256 * k)] = v[k];
+        for (int k = 0; k < 16; k++) xch[t + (t >> 4) + 272 * k] = v[k];
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 16; k++) v[k] = xch[PADX(256 * b + i0 + 16 * k)];
-        fa_fwd16_rowtab(v, tab, 1, b, n, ninv);
+        for (int k = 0; k < 16; k++) v[k] = xch[272 * b + i0 + 17 * k];
+        fa_fwd16_rowtab<false>(v, tab, 1, b, n, ninv);
 #pragma unroll
-        for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = v[k];
+        for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = v[k];
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 16; k++) v[k] = xch[PADX(16 * t + k)];
-        __builtin_amdgcn_sched_barrier(0);
-        fa_fwd16_rowlast(v, rho, w2, t, n, ninv);
-        // the finished row is materialized here, not next to its use
-#pragma unroll
-        for (int k = 0; k < 16; k++) asm volatile("" : "+v"(v[k]));
+        for (int k = 0; k < 16; k++) v[k] = xch[17 * t + k];
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     }
+    // the table loads depend on this opaque copy of t, so that they are
+    // issued here rather than at the kernel's start
+    int q = t;
+    asm volatile("" : "+v"(q));
+    {
+        const double T0 = fa_row_entry(rho[8], w2, q, n, ninv);
+        const double T1 = fa_row_entry(rho[9], w2, 2 * q, n, ninv);
+        const double T2 = fa_row_entry(rho[9], w2, 2 * q + 1, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++)
-        x[k] = fa_mulmod(fa_mulmod(x[k], m, n, ninv), SQR ? x[k] : y[k], n, ninv);
-    fa_build_row_table(tab, w2inv, r, rho, n, ninv);
-    __builtin_amdgcn_sched_barrier(0);
-    fa_inv16_rowlast(x, rho, w2inv, t, n, ninv);
-    __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0; k < 4; k++) {
+            fa_fwd4(x[k], x[k + 4], x[k + 8], x[k + 12], T0, T1, T2, n, ninv);
+            if (!SQR) fa_fwd4(y[k], y[k + 4], y[k + 8], y[k + 12], T0, T1, T2, n, ninv);
+        }
+    }
+    const double* rhoi = rho + 16;
+    // the twiddles of a group of four are requested when the group before it
+    // is done (the empty asm ties the index to its result): all at once they
+    // would not fit the registers of four workgroups per CU
+    int Q = 4 * q;
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(16 * t + k)] = x[k];
+    for (int j = 0; j < 4; j++) {
+        if (j > 0) {
+            Q += 1;
+            asm volatile("" : "+v"(Q) : "v"(x[4 * j - 1]));
+        } else {
+            asm volatile("" : "+v"(Q) : "v"(x[15]));
+        }
+        const double T0 = fa_mulmod(rho[10], w2[Q], n, ninv);
+        const double T1 = fa_mulmod(rho[11], w2[2 * Q], n, ninv);
+        const double T2 = fa_mulmod(rho[11], w2[2 * Q + 1], n, ninv);
+        double* u = x + 4 * j;
+        double* v = y + 4 * j;
+        fa_fwd4(u[0], u[1], u[2], u[3], T0, T1, T2, n, ninv);
+        if (!SQR) fa_fwd4(v[0], v[1], v[2], v[3], T0, T1, T2, n, ninv);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            u[k] = fa_mulmod(fa_mulmod(u[k], m, n, ninv), SQR ? u[k] : v[k], n, ninv);
+        const double V0 = fa_mulmod(rhoi[10], w2inv[Q], n, ninv);
+        const double V1 = fa_mulmod(rhoi[11], w2inv[2 * Q], n, ninv);
+        const double V2 = fa_mulmod(rhoi[11], w2inv[2 * Q + 1], n, ninv);
+        fa_inv4(u[0], u[1], u[2], u[3], V0, V1, V2, n, ninv);
+    }
+    {
+        const double T0 = fa_row_entry(rhoi[8], w2inv, q, n, ninv);
+        const double T1 = fa_row_entry(rhoi[9], w2inv, 2 * q, n, ninv);
+        const double T2 = fa_row_entry(rhoi[9], w2inv, 2 * q + 1, n, ninv);
+#pragma unroll
+        for (int k = 0; k < 4; k++) fa_inv4(x[k], x[k + 4], x[k + 8], x[k + 12], T0, T1, T2, n, ninv);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the forward table was last read two barriers ago
+    if (t < 255) {
+        const int l = 31 - __builtin_clz(t + 1);
+        tab[t] = fa_row_entry(rhoi[l], w2inv, t + 1 - (1 << l), n, ninv);
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++) xch[17 * t + k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(256 * b + i0 + 16 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[272 * b + i0 + 17 * k];
     fa_inv16_rowtab(x, tab, 1, b, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(t + 256 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[t + (t >> 4) + 272 * k];
     fa_inv16_rowtab(x, tab, 0, 0, n, ninv);
 #pragma unroll
     for (int k = 0; k < 16; k++) fa_st(arow + 256 * k, t * 8, x[k]);
 }
 
 template <bool SQR>
-__global__ void __launch_bounds__(256, 3) fa_k_row_conv16lr(double* __restrict__ A,
+__global__ void __launch_bounds__(256, 4) fa_k_row_conv16lr(double* __restrict__ A,
                                                              const double* __restrict__ B,
                                                              uint64_t stride, fa_prime_set S)
 {
     __shared__ double xch[4352];
     __shared__ double tab[256];
-    __shared__ double rho[16];
+    __shared__ double rho[32];
     const int i = blockIdx.y;
     const uint64_t r = blockIdx.x;
     fa_row_conv_tile_lr<SQR>(A + (uint64_t)i * stride + r * FA_ROW_PITCH,
@@ -487,24 +554,24 @@ __global__ void __launch_bounds__(256) fa_k_row_fwd16(double* __restrict__ A, ui
     for (int k = 0; k < 16; k++) v[k] = row[t + 256 * k];
     fa_fwd16_rowtab(v, tab, 0, 0, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(t + 256 * k)] = v[k];
+    for (int k = 0; k < 16; k++) xch[t + (t >> 4) + 272 * k] = v[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) v[k] = xch[PADX(256 * b + i0 + 16 * k)];
+    for (int k = 0; k < 16; k++) v[k] = xch[272 * b + i0 + 17 * k];
     fa_fwd16_rowtab(v, tab, 1, b, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = v[k];
+    for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = v[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) v[k] = xch[PADX(16 * t + k)];
+    for (int k = 0; k < 16; k++) v[k] = xch[17 * t + k];
     fa_fwd16_rowlast(v, rho, S.w2[i], t, n, ninv);
     __syncthreads();
     // through LDS so that the stores are coalesced
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(16 * t + k)] = v[k];
+    for (int k = 0; k < 16; k++) xch[17 * t + k] = v[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) row[t + 256 * k] = xch[PADX(t + 256 * k)];
+    for (int k = 0; k < 16; k++) row[t + 256 * k] = xch[t + (t >> 4) + 272 * k];
 }
 
 __global__ void __launch_bounds__(256) fa_k_row_inv16(double* __restrict__ A, uint64_t stride,
@@ -522,23 +589,23 @@ __global__ void __launch_bounds__(256) fa_k_row_inv16(double* __restrict__ A, ui
     double x[16];
     fa_build_row_table(tab, S.w2inv[i], r, rho, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(t + 256 * k)] = row[t + 256 * k];
+    for (int k = 0; k < 16; k++) xch[t + (t >> 4) + 272 * k] = row[t + 256 * k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(16 * t + k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[17 * t + k];
     fa_inv16_rowlast(x, rho, S.w2inv[i], t, n, ninv);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(16 * t + k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[17 * t + k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(256 * b + i0 + 16 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[272 * b + i0 + 17 * k];
     fa_inv16_rowtab(x, tab, 1, b, n, ninv);
 #pragma unroll
-    for (int k = 0; k < 16; k++) xch[PADX(256 * b + i0 + 16 * k)] = x[k];
+    for (int k = 0; k < 16; k++) xch[272 * b + i0 + 17 * k] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = xch[PADX(t + 256 * k)];
+    for (int k = 0; k < 16; k++) x[k] = xch[t + (t >> 4) + 272 * k];
     fa_inv16_rowtab(x, tab, 0, 0, n, ninv);
 #pragma unroll
     for (int k = 0; k < 16; k++) row[t + 256 * k] = x[k];
@@ -1035,7 +1102,7 @@ fa_k_col_inv16(double* __restrict__ A, uint64_t stride, fa_prime_set S, int np, 
 }
 
 // ---------------------------------------------------------------------------
-// Short rows.  A single product of up to 2^18 points has too few rows of 4096
+// Short rows.  A single product of up to 2^19 points has too few rows of 4096
 // to fill the GPU: 2^13 points modulo four primes are eight row workgroups,
 // each 13 us of dependent work.  There the transform is split into columns of
 // 2^D1 points and rows of 2^D2 = 256 or 1024: a row is radix-4 stages of four
@@ -1191,11 +1258,12 @@ __global__ void __launch_bounds__(1 << (D2 - 2)) fa_k_row_s(double* __restrict__
 #define FA_CW_LDS(C) ((C) * 2176)
 #define FA_C8_LDS FA_CW_LDS(8)
 
-template <int C>
-FA_DEV int fa_cw_addr(int c, int row) { return C * PADX(row & 2047) + c; }
-
-// stage-1 row of group tc, element k
-FA_DEV int fa_c8_row1(int tc, int k) { return ((tc >> 4) << 8) + (tc & 15) + 16 * k; }
+// PADX of the rows of a half, each a lane base plus a constant per element:
+// stage 0, u + 256 k (and 128 rows on); stage 1, (u >> 4) 256 + (u & 15) + 16 k;
+// stage 2, 16 u + k
+FA_DEV int fa_cw_row0(int u, int k) { return u + (u >> 4) + 272 * k; }
+FA_DEV int fa_cw_row1(int u, int k) { return 272 * (u >> 4) + (u & 15) + 17 * k; }
+FA_DEV int fa_cw_row2(int u, int k) { return 17 * u + k; }
 
 // stages 1 and 2 of a C-column tile after stage 0 (x0, x1 in the stage-0
 // layout), and the stores of the stage-2 layout
@@ -1212,14 +1280,13 @@ FA_DEV void fa_col_fwdw_rest(double* x0, double* x1, double* __restrict__ dst, i
     for (int H = 0; H < 2; H++) {
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            lds[fa_cw_addr<C>(c, u + 256 * (8 * H + k))] = x0[8 * H + k];
-            lds[fa_cw_addr<C>(c, u + 128 + 256 * (8 * H + k))] = x1[8 * H + k];
+            lds[C * fa_cw_row0(u, k) + c] = x0[8 * H + k];
+            lds[C * (fa_cw_row0(u, k) + 136) + c] = x1[8 * H + k];
         }
         __syncthreads();
-        const int tc = 128 * H + u;
 #pragma unroll
         for (int k = 0; k < 16; k++) {
-            const double v = lds[fa_cw_addr<C>(c, fa_c8_row1(tc, k))];
+            const double v = lds[C * fa_cw_row1(u, k) + c];
             if (H == 0) y0[k] = v; else y1[k] = v;
         }
         __syncthreads();
@@ -1232,14 +1299,13 @@ FA_DEV void fa_col_fwdw_rest(double* x0, double* x1, double* __restrict__ dst, i
     // exchange 1 -> 2, half H holds y_H entirely
 #pragma unroll
     for (int H = 0; H < 2; H++) {
-        const int tc = 128 * H + u;
 #pragma unroll
         for (int k = 0; k < 16; k++)
-            lds[fa_cw_addr<C>(c, fa_c8_row1(tc, k))] = H == 0 ? y0[k] : y1[k];
+            lds[C * fa_cw_row1(u, k) + c] = H == 0 ? y0[k] : y1[k];
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < 16; k++) {
-            const double v = lds[fa_cw_addr<C>(c, 16 * tc + k)];
+            const double v = lds[C * fa_cw_row2(u, k) + c];
             if (H == 0) x0[k] = v; else x1[k] = v;
         }
         if (H == 0) __syncthreads();
@@ -1317,13 +1383,12 @@ FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int g, double n, double n
     double y0[16], y1[16];
 #pragma unroll
     for (int H = 0; H < 2; H++) {
-        const int tc = 128 * H + u;
 #pragma unroll
-        for (int k = 0; k < 16; k++) lds[fa_cw_addr<C>(c, 16 * tc + k)] = H == 0 ? x0[k] : x1[k];
+        for (int k = 0; k < 16; k++) lds[C * fa_cw_row2(u, k) + c] = H == 0 ? x0[k] : x1[k];
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < 16; k++) {
-            const double v = lds[fa_cw_addr<C>(c, fa_c8_row1(tc, k))];
+            const double v = lds[C * fa_cw_row1(u, k) + c];
             if (H == 0) y0[k] = v; else y1[k] = v;
         }
         __syncthreads();
@@ -1337,15 +1402,14 @@ FA_DEV void fa_col_invw_tile(double* __restrict__ dst, int g, double n, double n
     // elements 8H .. 8H+7 of both stage-0 groups
 #pragma unroll
     for (int H = 0; H < 2; H++) {
-        const int tc = 128 * H + u;
 #pragma unroll
         for (int k = 0; k < 16; k++)
-            lds[fa_cw_addr<C>(c, fa_c8_row1(tc, k))] = H == 0 ? y0[k] : y1[k];
+            lds[C * fa_cw_row1(u, k) + c] = H == 0 ? y0[k] : y1[k];
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            x0[8 * H + k] = lds[fa_cw_addr<C>(c, u + 256 * (8 * H + k))];
-            x1[8 * H + k] = lds[fa_cw_addr<C>(c, u + 128 + 256 * (8 * H + k))];
+            x0[8 * H + k] = lds[C * fa_cw_row0(u, k) + c];
+            x1[8 * H + k] = lds[C * (fa_cw_row0(u, k) + 136) + c];
         }
         if (H == 0) __syncthreads();
     }
@@ -1476,13 +1540,13 @@ fa_kb_col_inv(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, 
         fa_col_inv_tile<D1>(dst, w.tile, S.p[pi], S.pinv[pi], S.w2inv[pi], lds);
 }
 
-__global__ void __launch_bounds__(256, 3) fa_kb_row_conv(const fa_bjob* __restrict__ J,
+__global__ void __launch_bounds__(256, 4) fa_kb_row_conv(const fa_bjob* __restrict__ J,
                                                          const uint64_t* __restrict__ work,
                                                          unsigned nwork, fa_prime_set S)
 {
     __shared__ double xch[4352];
     __shared__ double tab[256];
-    __shared__ double rho[16];
+    __shared__ double rho[32];
     const unsigned L = fa_xcd_linear();
     if (L >= nwork) return;
     const fa_witem w = fa_decode(work[L]);
@@ -1653,7 +1717,7 @@ int fa_trunc_rule(int d1, int t)
 // threads, half-column LDS; 0 = 4 columns, 1024 threads, whole-column LDS
 int fa_col_variant = 1;
 extern "C" FA_API void fa_set_col_variant(int v) { fa_col_variant = v; }
-// row pass: 1 = three workgroups per CU (twiddles of the last stage formed
+// row pass: 1 = four workgroups per CU (twiddles of the last stage formed
 // per layer, 168 registers), 0 = two workgroups per CU (all 15 held)
 int fa_row_variant = 1;
 extern "C" FA_API void fa_set_row_variant(int v) { fa_row_variant = v; }
@@ -1901,10 +1965,10 @@ static int launch_forward_any(const fa_operand& oa, int np, double* A, uint64_t 
 // other path and this one, us: 2^11 points 21.9 and 20.4 (one workgroup per
 // prime in LDS; at 2^10 that path is level, 19.5), 2^12 32.1 and 20.5, 2^14
 // 25.1 and 20.7, 2^16 31.1 and 26.3, 2^17 39.3 and 35.3 (products mod a 61-bit
-// n); 2^18 63.8 and 58.8 (integers); at 2^19 points the rows of 4096 fill
-// the GPU.  The lengths of the rows are the faster ones: at 2^16 and 2^17
+// n); 2^18 63.8 and 58.8 (integers); 2^19 57.6 and 52.4 modulo three primes,
+// but 104 and 110 modulo seven, where 896 rows of 4096 fill the GPU.  The lengths of the rows are the faster ones: at 2^16 and 2^17
 // points 1024 (26.4, 35.3) against 256 (29.7, 37.8).
-#define FA_SHORT_MAX 18
+#define FA_SHORT_MAX 19
 #define FA_SHORT_MIN 11
 
 template <int D1, int D2, int KIND>
@@ -1973,6 +2037,7 @@ static int fa_short(int depth, int what, const fa_operand& oa, const fa_operand&
     case 16: return launch_short<6, 10>(what, oa, ob, np, A, B, stride, S, s);
     case 17: return launch_short<7, 10>(what, oa, ob, np, A, B, stride, S, s);
     case 18: return launch_short<8, 10>(what, oa, ob, np, A, B, stride, S, s);
+    case 19: return np <= 3 ? launch_short<9, 10>(what, oa, ob, np, A, B, stride, S, s) : 0;
     default: return 0;
     }
 }

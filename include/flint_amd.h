@@ -574,7 +574,7 @@ FA_API void fa_set_col_variant(int v);
    Tuning and test switch; outputs are identical. */
 FA_API void fa_set_truncation(int mode);
 /* row pass variant of the two-level transforms: 1 = last-stage twiddles
-   formed per radix-4 layer, three workgroups per CU (default); 0 = all 15
+   formed per radix-4 layer, four workgroups per CU (default); 0 = all 15
    held in registers, two workgroups per CU.  Tuning switch, no counterpart
    in the reference. */
 FA_API void fa_set_row_variant(int v);

@@ -1,4 +1,4 @@
-"""GPU parity of the short-row transforms (single products of 2^11..2^18
+"""GPU parity of the short-row transforms (single products of 2^11..2^19
 points: columns of 2^D1 points by rows of 256 or 1024): products that just
 fit and that just exceed half of the transform, squares, every import, and
 transformed operands.  Words against the oracle."""
@@ -33,7 +33,7 @@ def test_nmod_depths(depth):
                           O.nmod_poly_mul_mid(a, b, N // 2 - 1, N, n))
 
 
-@pytest.mark.parametrize("depth", range(11, 19))
+@pytest.mark.parametrize("depth", range(11, 20))
 @pytest.mark.parametrize("np_,bits", [(2, 40), (4, 88), (8, 184)])
 def test_mpn_depths(depth, np_, bits):
     import flint_amd as fa
@@ -51,7 +51,7 @@ def test_mpn_depths(depth, np_, bits):
         assert np.array_equal(got, O.mpn_mul(a, b)), (an, bn)
 
 
-@pytest.mark.parametrize("depth", range(11, 19))
+@pytest.mark.parametrize("depth", range(11, 20))
 def test_fmpz_depths(depth):
     import flint_amd as fa
     rng = np.random.default_rng(depth)

@@ -92,6 +92,18 @@ FA_DEV uint64_t fa_mulmod_preinv(uint64_t a, uint64_t b, uint64_t n, uint64_t di
     return fa_ll_mod_preinv(__umul64hi(a, b), a * b, n, dinv, norm);
 }
 
+// carries through 64 positions with generate and propagate masks G, P (no
+// position both): the carries into the positions for a carry c into the
+// first, and through cout the carry out of the last
+FA_DEV uint64_t fa_gp_carries(uint64_t G, uint64_t P, uint32_t c, uint32_t* cout)
+{
+    const uint64_t X = G | P;
+    const uint64_t s1 = G + X;
+    const uint64_t s2 = s1 + c;
+    *cout = (uint32_t)(s1 < X) | (uint32_t)(s2 < s1);
+    return s2 ^ X ^ G;
+}
+
 struct fa_prime_dev {
     double p;
     double pinv;

@@ -1718,7 +1718,7 @@ int fa_trunc_rule(int d1, int t)
 int fa_col_variant = 1;
 extern "C" FA_API void fa_set_col_variant(int v) { fa_col_variant = v; }
 // row pass: 1 = four workgroups per CU (twiddles of the last stage formed
-// per layer, 168 registers), 0 = two workgroups per CU (all 15 held)
+// per layer, 128 registers), 0 = two workgroups per CU (all 15 held)
 int fa_row_variant = 1;
 extern "C" FA_API void fa_set_row_variant(int v) { fa_row_variant = v; }
 

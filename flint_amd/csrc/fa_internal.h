@@ -236,12 +236,9 @@ struct fa_bks {                 // one signed-slot KS product of a batch
     const uint64_t* a;
     const uint64_t* b;
     uint64_t* z;
-    uint64_t aw, an, bw, bn, s, La, Lb, nP, zw, zl, cnt, zn, top;
+    uint64_t aw, an, bw, bn, s, La, Lb, nP, zw, zl, cnt, zn;
     int32_t* lowa;
     int32_t* lowb;
-    uint8_t* bra;
-    uint8_t* brb;
-    uint8_t* tk;
     int32_t* sig;
     uint64_t* pa;
     uint64_t* pb;

@@ -141,104 +141,147 @@ __global__ void __launch_bounds__(256) fa_k_ks_combine(const uint64_t* __restric
 // [sigma a_i < 0] and propagate [a_i = 0]: a 1-bit scan over coefficients.
 // The product C = A B = sum_k c_k 2^(s k) with |c_k| < 2^(s-1) (the slot
 // width above) has base-2^s digits e_k, and
-//     c_k = e_k + t_(k-1) - 2^s t_k,  t_k = [e_k + t_(k-1) >= 2^(s-1)],
-// again a 1-bit scan: generate [e_k >= 2^(s-1)], propagate
-// [e_k = 2^(s-1) - 1].  So c_k is the s-bit field e_k + t_(k-1), read as a
-// signed s-bit number, times sigma_a sigma_b.
+//     c_k = e_k + t_(k-1) - 2^s t_k,  t_k = [e_k + t_(k-1) >= 2^(s-1)].
+// t_k is the top bit of e_k: they differ only for e_k = 2^(s-1) - 1 with
+// t_(k-1) = 1, which would make |c_k| = 2^(s-1).  (|c_k| <= m 2^(|b1|+|b2|) for
+// m terms and m < 2^bitcount(m), so the bound holds for |a_i| = 2^|b1| too.)
+// So c_k is the s-bit field e_k + t_(k-1), with t_(k-1) one bit of the product
+// and no scan over the slots, read as a signed s-bit number, times sigma_a
+// sigma_b.
 // ---------------------------------------------------------------------------
 
-// one workgroup per operand: the lowest nonzero limb of each coefficient,
-// the sign sigma of the top nonzero coefficient (+1 for a zero operand) and
-// the borrow into each coefficient's slot.  Each thread keeps one
-// contiguous block of coefficients through both passes.
-FA_DEV void ks_sflags_body(const uint64_t* __restrict__ a, int w, uint64_t n,
-                           int32_t* __restrict__ low, uint8_t* __restrict__ br,
-                           int32_t* __restrict__ sig, int64_t* stop, uint8_t* sg, uint8_t* sp)
+typedef __attribute__((address_space(1))) const uint64_t fa_gcw;   // global words
+
+// The flag word of a coefficient: its lowest nonzero limb (KS_ZERO for zero)
+// and in bit 30 the borrow into its slot.
+#define KS_ZERO 0x3fffffff
+
+// the lowest nonzero limb of a w-limb coefficient whose limb 0 is v0
+FA_DEV int ks_low_limb(fa_gcw* c, int w, uint64_t v0)
 {
-    const int t = threadIdx.x;
-    const uint64_t m = (n + 1023) / 1024;
-    const uint64_t i0 = (uint64_t)t * m < n ? (uint64_t)t * m : n;
-    const uint64_t i1 = i0 + m < n ? i0 + m : n;
-    int64_t top = -1;
-    for (uint64_t i = i0; i < i1; i++) {
-        const uint64_t* c = a + i * (uint64_t)w;
-        int l = 0;
-        while (l < w && c[l] == 0) l++;
-        low[i] = l;
-        if (l < w) top = (int64_t)i;
-    }
-    stop[t] = top;
-    __syncthreads();
-    for (int h = 512; h > 0; h >>= 1) {
-        if (t < h && stop[t + h] > stop[t]) stop[t] = stop[t + h];
-        __syncthreads();
-    }
-    const int64_t ti = stop[0];
-    const int negs = ti >= 0 ? (int)(a[(uint64_t)ti * w + w - 1] >> 63) : 0;
-    if (t == 0) *sig = negs ? -1 : 1;
-    // block aggregates of (generate, propagate), composed left to right
-    uint8_t G = 0, P = 1;
-    for (uint64_t i = i0; i < i1; i++) {
-        const int z = low[i] >= w;
-        const int neg = (int)(a[i * (uint64_t)w + w - 1] >> 63);
-        const uint8_t gi = (uint8_t)(!z && neg != negs), pi = (uint8_t)z;
-        G = (uint8_t)(gi | (pi & G));
-        P = (uint8_t)(P & pi);
-    }
-    sg[t] = G;
-    sp[t] = P;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        uint8_t g = sg[t], q = sp[t];
-        if (t >= d) {
-            g = (uint8_t)(g | (q & sg[t - d]));
-            q = (uint8_t)(q & sp[t - d]);
+    if (v0) return 0;
+    int l = 1;
+    while (l < w && c[l] == 0) l++;
+    return l < w ? l : KS_ZERO;
+}
+
+// the carries into the 64 wave masks of a round (64 positions each, in order)
+// as a mask: lane l of every wave reads mask l, whose carry-out depends on its
+// carry-in only if it propagates throughout.  *c: the carry into the round, on
+// return the one out of it
+FA_DEV uint64_t ks_round_carries(const uint64_t* sG, const uint64_t* sP, int lane, uint32_t* c)
+{
+    const uint64_t g = sG[lane], p = sP[lane];
+    uint32_t o, on;
+    (void)fa_gp_carries(g, p, 0, &o);
+    const uint64_t cin = fa_gp_carries(__ballot(o != 0), __ballot(p == ~UINT64_C(0)), *c, &on);
+    *c = on;
+    return cin;
+}
+
+// one workgroup per operand: the sign sigma of the top nonzero coefficient (+1
+// for a zero operand), then the flag words, 4 x 1024 coefficients a round with
+// the loads of a round issued together and the borrows from the ballots of its
+// waves.  sG, sP: 64 words each.  Bound by the latency of one workgroup's
+// loads; a run of coefficients per thread, walked limb by limb, took 159 us for
+// the operands of 64 batched products (561 MB packed), the rounds 85.
+FA_DEV void ks_sflags_body(const uint64_t* __restrict__ ap, int w, uint64_t n,
+                           int32_t* __restrict__ low, int32_t* __restrict__ sig, uint64_t* sG,
+                           uint64_t* sP)
+{
+    fa_gcw* a = (fa_gcw*)ap;
+    typedef __attribute__((address_space(1))) int32_t gI;
+    gI* lowg = (gI*)low;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int negs = 0;
+    for (int64_t hi = (int64_t)n; hi > 0; hi -= 1024) {
+        const int64_t i = hi - 1024 + t;
+        bool nz = false, neg = false;
+        if (i >= 0) {
+            fa_gcw* c = a + (uint64_t)i * w;
+            const uint64_t top = c[w - 1];
+            neg = top >> 63;
+            nz = top != 0 || ks_low_limb(c, w, c[0]) != KS_ZERO;
+        }
+        const uint64_t NZ = __ballot(nz), NG = __ballot(neg);
+        if (lane == 0) {
+            sG[wave] = NZ;
+            sP[wave] = NG;
         }
         __syncthreads();
-        sg[t] = g;
-        sp[t] = q;
+        int found = 0;
+        for (int v = 15; v >= 0 && !found; v--) {
+            if (sG[v]) {
+                negs = (int)((sP[v] >> (63 - __builtin_clzll(sG[v]))) & 1);
+                found = 1;
+            }
+        }
         __syncthreads();
+        if (found) break;
     }
-    uint8_t cin = t ? sg[t - 1] : 0;
-    for (uint64_t i = i0; i < i1; i++) {
-        br[i] = cin;
-        const int z = low[i] >= w;
-        const int neg = (int)(a[i * (uint64_t)w + w - 1] >> 63);
-        cin = (uint8_t)((!z && neg != negs) | (z & cin));
+    if (t == 0) *sig = negs ? -1 : 1;
+    uint32_t c = 0;
+    for (uint64_t base = 0; base < n; base += 4096) {
+        uint64_t v0[4], vt[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint64_t i = base + 1024 * k + t;
+            fa_gcw* p = a + (i < n ? i : n - 1) * (uint64_t)w;
+            v0[k] = p[0];
+            vt[k] = p[w - 1];
+        }
+        int l[4];
+        uint64_t G[4], P[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint64_t i = base + 1024 * k + t;
+            const bool in = i < n;
+            l[k] = ks_low_limb(a + (in ? i : n - 1) * (uint64_t)w, w, v0[k]);
+            // generate [sigma c < 0], propagate [c = 0]
+            G[k] = __ballot(in && l[k] != KS_ZERO && (int)(vt[k] >> 63) != negs);
+            P[k] = __ballot(in && l[k] == KS_ZERO);
+            if (lane == 0) {
+                sG[16 * k + wave] = G[k];
+                sP[16 * k + wave] = P[k];
+            }
+        }
+        __syncthreads();
+        const uint64_t cw = ks_round_carries(sG, sP, lane, &c);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            uint32_t o;
+            const uint64_t cin = fa_gp_carries(G[k], P[k], (uint32_t)(cw >> (16 * k + wave)) & 1, &o);
+            const uint64_t i = base + 1024 * k + t;
+            if (i < n) lowg[i] = l[k] | (int)((cin >> lane) & 1) << 30;
+        }
+        __syncthreads();
     }
 }
 
 __global__ void __launch_bounds__(1024) fa_k_ks_sflags(const uint64_t* __restrict__ a, int w,
                                                        uint64_t n, int32_t* __restrict__ low,
-                                                       uint8_t* __restrict__ br,
                                                        int32_t* __restrict__ sig)
 {
-    __shared__ int64_t stop[1024];
-    __shared__ uint8_t sg[1024], sp[1024];
-    ks_sflags_body(a, w, n, low, br, sig, stop, sg, sp);
+    __shared__ uint64_t sG[64], sP[64];
+    ks_sflags_body(a, w, n, low, sig, sG, sP);
 }
 
 // limb m (any m >= 0, sign-extended past w) of v = sigma c - br for a w-limb
-// two's complement coefficient c whose lowest nonzero limb is `low` (w if c
-// is zero); negs: sigma = -1
-FA_DEV uint64_t fa_ks_vlimb(const uint64_t* c, int w, int m, int negs, int br, int low)
+// two's complement coefficient c with flag word f; S = 0 for sigma = +1, all
+// ones for -1.  c - br subtracts br, -c - br = ~c + 1 - br adds 1 - br, in
+// every limb up to the lowest nonzero one (all of them for zero).
+FA_DEV uint64_t fa_ks_vlimb(fa_gcw* c, int w, int m, uint64_t S, int f)
 {
-    const bool zero = low >= w;
-    const uint64_t cs = (c[w - 1] >> 63) ? ~UINT64_C(0) : 0;
-    if (!negs) {
-        if (!br) return m < w ? c[m] : cs;
-        if (zero) return ~UINT64_C(0);                       // 0 - 1
-        return m < w ? c[m] - (m <= low ? 1u : 0u) : cs;     // c - 1, same sign as c
-    }
-    if (br) return m < w ? ~c[m] : ~cs;                      // -c - 1 = ~c
-    if (zero) return 0;
-    return m < w ? ~c[m] + (m <= low ? 1u : 0u) : ~cs;       // -c
+    uint64_t x = c[m < w ? m : w - 1];
+    if (m >= w) x = (uint64_t)((int64_t)x >> 63);
+    const int64_t d = (int64_t)(S & 1) - (f >> 30);
+    return (x ^ S) + (m <= (f & KS_ZERO) ? (uint64_t)d : 0);
 }
 
-// out[j] = limb j of sum_i d_i 2^(s i), d_i = (sigma c_i - br_i) mod 2^s
-FA_DEV uint64_t ks_spack_limb(const uint64_t* __restrict__ a, int w, uint64_t n,
-                              const int32_t* __restrict__ low, const uint8_t* __restrict__ br,
-                              int negs, uint64_t s, uint64_t j)
+// out[j] = limb j of sum_i d_i 2^(s i), d_i = (sigma c_i - br_i) mod 2^s; slots
+// of fewer than 64 bits
+FA_DEV uint64_t ks_spack_limb(fa_gcw* a, int w, uint64_t n, const int32_t* __restrict__ low,
+                              uint64_t S, uint64_t s, uint64_t j)
 {
     const uint64_t bit0 = 64 * j;
     // floor(bit0 / s) from the correctly rounded double quotient (both
@@ -248,16 +291,16 @@ FA_DEV uint64_t ks_spack_limb(const uint64_t* __restrict__ a, int w, uint64_t n,
     if (i0 * s > bit0) i0--;
     uint64_t acc = 0;
     for (uint64_t i = i0; i < n && s * i < bit0 + 64; i++) {
-        const uint64_t* c = a + i * (uint64_t)w;
-        const int lo = low[i], b = br[i];
+        fa_gcw* c = a + i * (uint64_t)w;
+        const int f = low[i];
         const int64_t rel = (int64_t)bit0 - (int64_t)(s * i);   // slot bit at bit0
         uint64_t win;
         if (rel >= 0) {
             const int q = (int)(rel >> 6), r = (int)(rel & 63);
-            win = fa_ks_vlimb(c, w, q, negs, b, lo) >> r;
-            if (r) win |= fa_ks_vlimb(c, w, q + 1, negs, b, lo) << (64 - r);
+            win = fa_ks_vlimb(c, w, q, S, f) >> r;
+            if (r) win |= fa_ks_vlimb(c, w, q + 1, S, f) << (64 - r);
         } else {
-            win = fa_ks_vlimb(c, w, 0, negs, b, lo) << (int)(-rel);
+            win = fa_ks_vlimb(c, w, 0, S, f) << (int)(-rel);
         }
         // keep window positions p with 0 <= rel + p < s
         const int64_t plo = rel < 0 ? -rel : 0;
@@ -270,34 +313,71 @@ FA_DEV uint64_t ks_spack_limb(const uint64_t* __restrict__ a, int w, uint64_t n,
     return acc;
 }
 
-// the same limb for slots of at least 64 bits: the window [64 j, 64 j + 64)
-// meets slot i0 = floor(64 j / s) and at most slot i0 + 1, so both are read
-// with loads that do not wait on each other (the second at a clamped index
-// and used only when that slot starts inside the window)
-FA_DEV uint64_t ks_spack_limb_wide(const uint64_t* __restrict__ a, int w, uint64_t n,
-                                   const int32_t* __restrict__ low, const uint8_t* __restrict__ br,
-                                   int negs, uint64_t s, uint64_t j)
+// the same for K limbs j0 + 256 k + threadIdx.x of slots of at least 64 bits:
+// the window [64 j, 64 j + 64) meets slot i0 = floor(64 j / s) and at most slot
+// i0 + 1.  i0 comes from one reciprocal per thread and a correction by one
+// (64 j < 2^46: the product of the two roundings is within 2^-11 of the
+// quotient); the limbs of i0 are requested for all K windows before any is
+// used, slot i0 + 1 is read only where it starts inside the window.  An
+// emulated division, the limbs of both slots and their flags for every window
+// took 520 us for 64 batched products (561 MB written), this 273.
+template <int K>
+FA_DEV void ks_spack_wide(uint64_t* v, fa_gcw* a, int w, uint64_t n,
+                          const int32_t* __restrict__ lowp, uint64_t S, uint64_t s, uint64_t L,
+                          uint64_t j0)
 {
-    const uint64_t bit0 = 64 * j;
-    uint64_t i0 = (uint64_t)((double)bit0 / (double)s);
-    if (i0 * s > bit0) i0--;
-    if (i0 >= n) return 0;
-    const uint64_t i1 = i0 + 1 < n ? i0 + 1 : i0;
-    const uint64_t rel = bit0 - s * i0;   // slot bit at bit0, in [0, s)
-    const int q = (int)(rel >> 6), r = (int)(rel & 63);
-    const uint64_t* c0 = a + i0 * (uint64_t)w;
-    const uint64_t* c1 = a + i1 * (uint64_t)w;
-    const int lo0 = low[i0], b0 = br[i0], lo1 = low[i1], b1 = br[i1];
-    uint64_t win = fa_ks_vlimb(c0, w, q, negs, b0, lo0) >> r;
-    if (r) win |= fa_ks_vlimb(c0, w, q + 1, negs, b0, lo0) << (64 - r);
-    const uint64_t next = fa_ks_vlimb(c1, w, 0, negs, b1, lo1);
-    // window positions below s - rel belong to slot i0, the rest (when
-    // s - rel < 64) to slot i0 + 1, whose bit 0 sits at position s - rel
-    const uint64_t phi = s - rel;
-    if (phi >= 64) return win;
-    uint64_t acc = win & ((UINT64_C(1) << phi) - 1);
-    if (i0 + 1 < n) acc |= next << phi;
-    return acc;
+    typedef __attribute__((address_space(1))) const int32_t gI;
+    gI* low = (gI*)lowp;
+    const double inv = 1.0 / (double)s;
+    uint64_t i0[K];
+    int64_t rel[K];
+    uint64_t lo[K], hi[K];
+    int f[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        uint64_t j = j0 + 256 * (uint64_t)k + threadIdx.x;
+        if (j >= L) j = L - 1;
+        const uint64_t bit0 = 64 * j;
+        uint64_t i = (uint64_t)((double)bit0 * inv);
+        int64_t d = (int64_t)(bit0 - i * s);
+        if (d < 0) {
+            i--;
+            d += (int64_t)s;
+        } else if (d >= (int64_t)s) {
+            i++;
+            d -= (int64_t)s;
+        }
+        i0[k] = i;
+        rel[k] = d;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const uint64_t i = i0[k] < n ? i0[k] : n - 1;
+        const int q = (int)(rel[k] >> 6);
+        fa_gcw* c = a + i * (uint64_t)w;
+        f[k] = low[i];
+        lo[k] = c[q < w ? q : w - 1];
+        hi[k] = c[q + 1 < w ? q + 1 : w - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int q = (int)(rel[k] >> 6), r = (int)(rel[k] & 63);
+        const int64_t d = (int64_t)(S & 1) - (f[k] >> 30);
+        const int lw = f[k] & KS_ZERO;
+        uint64_t x = q < w ? lo[k] : (uint64_t)((int64_t)lo[k] >> 63);
+        uint64_t y = q + 1 < w ? hi[k] : (uint64_t)((int64_t)hi[k] >> 63);
+        x = (x ^ S) + (q <= lw ? (uint64_t)d : 0);
+        y = (y ^ S) + (q + 1 <= lw ? (uint64_t)d : 0);
+        uint64_t win = r ? (x >> r) | (y << (64 - r)) : x;
+        const uint64_t phi = s - (uint64_t)rel[k];
+        if (phi < 64) {
+            // positions below phi belong to slot i0, the rest to slot i0 + 1
+            win &= (UINT64_C(1) << phi) - 1;
+            if (i0[k] + 1 < n)
+                win |= fa_ks_vlimb(a + (i0[k] + 1) * (uint64_t)w, w, 0, S, low[i0[k] + 1]) << phi;
+        }
+        v[k] = i0[k] < n ? win : 0;
+    }
 }
 
 // packed limbs j0 + 256 k + threadIdx.x (k < K) below L: all computed
@@ -305,100 +385,36 @@ FA_DEV uint64_t ks_spack_limb_wide(const uint64_t* __restrict__ a, int w, uint64
 // takes K = FA_KS_PACK_BLK / 256; one product alone takes K = 1, which
 // leaves more waves per CU to hide the loads of a small grid.
 template <int K>
-FA_DEV void ks_spack_block(const uint64_t* __restrict__ a, int w, uint64_t n,
-                           const int32_t* __restrict__ low, const uint8_t* __restrict__ br,
-                           int negs, uint64_t s, uint64_t* __restrict__ out, uint64_t L,
-                           uint64_t j0)
+FA_DEV void ks_spack_block(const uint64_t* __restrict__ ap, int w, uint64_t n,
+                           const int32_t* __restrict__ low, int negs, uint64_t s,
+                           uint64_t* __restrict__ out, uint64_t L, uint64_t j0)
 {
+    typedef __attribute__((address_space(1))) uint64_t gT;
+    fa_gcw* a = (fa_gcw*)ap;
+    const uint64_t S = negs ? ~UINT64_C(0) : 0;
     uint64_t v[K];
+    if (s >= 64) {
+        ks_spack_wide<K>(v, a, w, n, low, S, s, L, j0);
+    } else {
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const uint64_t j = j0 + 256 * (uint64_t)k + threadIdx.x;
-        v[k] = 0;
-        if (j < L)
-            v[k] = s >= 64 ? ks_spack_limb_wide(a, w, n, low, br, negs, s, j)
-                           : ks_spack_limb(a, w, n, low, br, negs, s, j);
+        for (int k = 0; k < K; k++) {
+            const uint64_t j = j0 + 256 * (uint64_t)k + threadIdx.x;
+            v[k] = j < L ? ks_spack_limb(a, w, n, low, S, s, j) : 0;
+        }
     }
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const uint64_t j = j0 + 256 * (uint64_t)k + threadIdx.x;
-        if (j < L) out[j] = v[k];
+        if (j < L) ((gT*)out)[j] = v[k];
     }
 }
 
 __global__ void __launch_bounds__(256) fa_k_ks_spack(const uint64_t* __restrict__ a, int w,
                                                      uint64_t n, const int32_t* __restrict__ low,
-                                                     const uint8_t* __restrict__ br,
                                                      const int32_t* __restrict__ sig, uint64_t s,
                                                      uint64_t* __restrict__ out, uint64_t L)
 {
-    ks_spack_block<1>(a, w, n, low, br, *sig < 0, s, out, L, (uint64_t)blockIdx.x * 256);
-}
-
-// generate and propagate of slot k of the product: the slot's top bit, and
-// whether its other s - 1 bits are all ones with the top bit clear
-FA_DEV void fa_ks_slot_gp(const uint64_t* __restrict__ C, uint64_t nP, uint64_t s, uint64_t k,
-                          uint8_t* g, uint8_t* p)
-{
-    const uint64_t tb = s * k + s - 1;
-    const uint64_t q = tb >> 6;
-    const uint8_t top = q < nP ? (uint8_t)((C[q] >> (tb & 63)) & 1) : 0;
-    *g = top;
-    uint8_t ones = !top;
-    for (uint64_t lb = 0; ones && lb < s - 1; lb += 64) {
-        const uint64_t nb = s - 1 - lb < 64 ? s - 1 - lb : 64;
-        const uint64_t want = nb == 64 ? ~UINT64_C(0) : ((UINT64_C(1) << nb) - 1);
-        const uint64_t v = fa_ks_slot(C, nP, s, k, (int)(lb >> 6));
-        if ((v & want) != want) ones = 0;
-    }
-    *p = ones;
-}
-
-// one workgroup: t_k for the slots k < K of the product (the borrow each
-// slot passes up), as bytes
-FA_DEV void ks_uscan_body(const uint64_t* __restrict__ C, uint64_t nP, uint64_t s, uint64_t K,
-                          uint8_t* __restrict__ tk, uint8_t* sg, uint8_t* sp)
-{
-    const int t = threadIdx.x;
-    const uint64_t m = (K + 1023) / 1024;
-    const uint64_t k0 = (uint64_t)t * m < K ? (uint64_t)t * m : K;
-    const uint64_t k1 = k0 + m < K ? k0 + m : K;
-    uint8_t G = 0, P = 1;
-    for (uint64_t k = k0; k < k1; k++) {
-        uint8_t g, p;
-        fa_ks_slot_gp(C, nP, s, k, &g, &p);
-        tk[k] = (uint8_t)(g | (p << 1));
-        G = (uint8_t)(g | (p & G));
-        P = (uint8_t)(P & p);
-    }
-    sg[t] = G;
-    sp[t] = P;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        uint8_t g = sg[t], q = sp[t];
-        if (t >= d) {
-            g = (uint8_t)(g | (q & sg[t - d]));
-            q = (uint8_t)(q & sp[t - d]);
-        }
-        __syncthreads();
-        sg[t] = g;
-        sp[t] = q;
-        __syncthreads();
-    }
-    uint8_t cin = t ? sg[t - 1] : 0;
-    for (uint64_t k = k0; k < k1; k++) {
-        const uint8_t f = tk[k];
-        cin = (uint8_t)((f & 1) | ((f >> 1) & cin));
-        tk[k] = cin;
-    }
-}
-
-__global__ void __launch_bounds__(1024) fa_k_ks_uscan(const uint64_t* __restrict__ C,
-                                                      uint64_t nP, uint64_t s, uint64_t K,
-                                                      uint8_t* __restrict__ tk)
-{
-    __shared__ uint8_t sg[1024], sp[1024];
-    ks_uscan_body(C, nP, s, K, tk, sg, sp);
+    ks_spack_block<1>(a, w, n, low, *sig < 0, s, out, L, (uint64_t)blockIdx.x * 256);
 }
 
 // limbs of each coefficient staged through LDS per step of the unpack
@@ -414,8 +430,7 @@ static_assert(FA_KS_UC + 1 < 64, "unpack staging width");
 // consecutive limbs, so neither side accesses memory one limb per
 // coefficient at a stride of zw limbs.  buf: 256 * (FA_KS_UC + 1) words.
 FA_DEV void ks_unpack_tile(const uint64_t* __restrict__ C, uint64_t nP, uint64_t s,
-                           const uint8_t* __restrict__ tk, const int32_t* __restrict__ sig,
-                           uint64_t zl, uint64_t zn, uint64_t cnt, int zw,
+                           const int32_t* __restrict__ sig, uint64_t zl, uint64_t zn, uint64_t cnt, int zw,
                            uint64_t* __restrict__ z, uint64_t t0, uint64_t* __restrict__ buf)
 {
     constexpr int W = FA_KS_UC + 1;
@@ -426,7 +441,12 @@ FA_DEV void ks_unpack_tile(const uint64_t* __restrict__ C, uint64_t nP, uint64_t
     const bool live = mine && k < zn;
     const int neg = (sig[0] < 0) != (sig[1] < 0);
     const int r = (int)((s * k) & 63);   // bit offset of the slot in its first limb
-    uint64_t carry = (live && k) ? tk[k - 1] : 0;
+    // t_(k-1): the top bit of slot k - 1
+    uint64_t carry = 0;
+    if (live && k) {
+        const uint64_t tb = s * k - 1;
+        if (tb >> 6 < nP) carry = (C[tb >> 6] >> (tb & 63)) & 1;
+    }
     uint64_t fill = 0;
     uint64_t ncarry = 1;   // two's complement negation: ~v + 1
     for (int lc = 0; lc < zw; lc += FA_KS_UC) {
@@ -493,31 +513,29 @@ FA_DEV void ks_unpack_tile(const uint64_t* __restrict__ C, uint64_t nP, uint64_t
 
 __global__ void __launch_bounds__(256) fa_k_ks_unpack(const uint64_t* __restrict__ C,
                                                       uint64_t nP, uint64_t s,
-                                                      const uint8_t* __restrict__ tk,
                                                       const int32_t* __restrict__ sig,
                                                       uint64_t zl, uint64_t cnt, uint64_t zn,
                                                       int zw, uint64_t* __restrict__ z)
 {
     __shared__ uint64_t buf[256 * (FA_KS_UC + 1)];
-    ks_unpack_tile(C, nP, s, tk, sig, zl, zn, cnt, zw, z, (uint64_t)blockIdx.x * 256, buf);
+    ks_unpack_tile(C, nP, s, sig, zl, zn, cnt, zw, z, (uint64_t)blockIdx.x * 256, buf);
 }
 
 // ---------------------------------------------------------------------------
 // batched signed-slot route: every KS product of a batch in one launch per
-// step.  Flags and slot scans take one workgroup per operand or product;
-// packing and unpacking take work items (record | operand << 31 | block of
-// FA_KS_PACK_BLK packed limbs or 256 output coefficients << 32).
+// step.  Flags take one workgroup per operand; packing and unpacking take work
+// items (record | operand << 31 | block of FA_KS_PACK_BLK packed limbs or 256
+// output coefficients << 32).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024) fa_kb_ks_sflags(const fa_bks* __restrict__ R, unsigned nks)
 {
-    __shared__ int64_t stop[1024];
-    __shared__ uint8_t sg[1024], sp[1024];
+    __shared__ uint64_t sG[64], sP[64];
     if (blockIdx.x >= 2 * nks) return;
     const fa_bks& r = R[blockIdx.x >> 1];
     if (blockIdx.x & 1)
-        ks_sflags_body(r.b, (int)r.bw, r.bn, r.lowb, r.brb, r.sig + 1, stop, sg, sp);
+        ks_sflags_body(r.b, (int)r.bw, r.bn, r.lowb, r.sig + 1, sG, sP);
     else
-        ks_sflags_body(r.a, (int)r.aw, r.an, r.lowa, r.bra, r.sig, stop, sg, sp);
+        ks_sflags_body(r.a, (int)r.aw, r.an, r.lowa, r.sig, sG, sP);
 }
 
 __global__ void __launch_bounds__(256) fa_kb_ks_spack(const fa_bks* __restrict__ R,
@@ -530,17 +548,9 @@ __global__ void __launch_bounds__(256) fa_kb_ks_spack(const fa_bks* __restrict__
     const int op = (int)((wi >> 31) & 1);
     const uint64_t j0 = (wi >> 32) * FA_KS_PACK_BLK;
     if (op)
-        ks_spack_block<FA_KS_PACK_BLK / 256>(r.b, (int)r.bw, r.bn, r.lowb, r.brb, r.sig[1] < 0, r.s, r.pb, r.Lb, j0);
+        ks_spack_block<FA_KS_PACK_BLK / 256>(r.b, (int)r.bw, r.bn, r.lowb, r.sig[1] < 0, r.s, r.pb, r.Lb, j0);
     else
-        ks_spack_block<FA_KS_PACK_BLK / 256>(r.a, (int)r.aw, r.an, r.lowa, r.bra, r.sig[0] < 0, r.s, r.pa, r.La, j0);
-}
-
-__global__ void __launch_bounds__(1024) fa_kb_ks_uscan(const fa_bks* __restrict__ R, unsigned nks)
-{
-    __shared__ uint8_t sg[1024], sp[1024];
-    if (blockIdx.x >= nks) return;
-    const fa_bks& r = R[blockIdx.x];
-    if (r.top > 0) ks_uscan_body(r.pr, r.nP, r.s, r.top, r.tk, sg, sp);
+        ks_spack_block<FA_KS_PACK_BLK / 256>(r.a, (int)r.aw, r.an, r.lowa, r.sig[0] < 0, r.s, r.pa, r.La, j0);
 }
 
 __global__ void __launch_bounds__(256) fa_kb_ks_unpack(const fa_bks* __restrict__ R,
@@ -552,7 +562,7 @@ __global__ void __launch_bounds__(256) fa_kb_ks_unpack(const fa_bks* __restrict_
     const uint64_t wi = work[blockIdx.x];
     const fa_bks& r = R[(unsigned)(wi & 0x7fffffffu)];
     const uint64_t t0 = (wi >> 32) * 256;
-    if (t0 < r.cnt) ks_unpack_tile(r.pr, r.nP, r.s, r.tk, r.sig, r.zl, r.zn, r.cnt, (int)r.zw, r.z, t0, buf);
+    if (t0 < r.cnt) ks_unpack_tile(r.pr, r.nP, r.s, r.sig, r.zl, r.zn, r.cnt, (int)r.zw, r.z, t0, buf);
 }
 
 int fa_batch_ks_pre(const fa_bks* R, unsigned nks, const uint64_t* work, unsigned nwork,
@@ -569,7 +579,6 @@ int fa_batch_ks_post(const fa_bks* R, unsigned nks, const uint64_t* work, unsign
                      hipStream_t s)
 {
     if (!nks) return FA_OK;
-    FA_LAUNCH("fa_kb_ks_uscan", fa_kb_ks_uscan, dim3(nks), dim3(1024), 0, s, R, nks);
     if (nwork)
         FA_LAUNCH("fa_kb_ks_unpack", fa_kb_ks_unpack, dim3(nwork), dim3(256), 0, s, R, work, nwork);
     return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "batch ks unpack launch");
@@ -593,8 +602,7 @@ int fa_ks_current_variant() { return fa_ks_variant; }
 int fa_ks_nprod(int variant) { return variant ? 1 : 3; }
 
 // scratch layout of one KS product: the packed operands, the products, the
-// low-limb indices; for signed slots also the borrows, the product's slot
-// borrows and the two signs
+// low-limb indices (signed slots: the flag words and the two signs)
 struct ks_layout {
     uint64_t La, Lb, nP;
     uint64_t* pa[3];
@@ -602,9 +610,6 @@ struct ks_layout {
     uint64_t* pr[3];
     int32_t* lowa;
     int32_t* lowb;
-    uint8_t* bra;
-    uint8_t* brb;
-    uint8_t* tk;
     int32_t* sig;
 };
 
@@ -622,12 +627,7 @@ static ks_layout ks_lay(int variant, uint64_t sb, uint64_t an, uint64_t bn, uint
     for (int k = 0; k < np; k++) { K.pr[k] = w; w += K.nP; }
     K.lowa = (int32_t*)w;
     K.lowb = K.lowa + an;
-    if (variant) {
-        K.sig = K.lowb + bn;                  // two int32
-        K.bra = (uint8_t*)(K.sig + 2);
-        K.brb = K.bra + an;
-        K.tk = K.brb + bn;                    // an + bn slots
-    }
+    if (variant) K.sig = K.lowb + bn;         // two int32
     return K;
 }
 
@@ -638,7 +638,7 @@ uint64_t fa_ks_scratch_words_v(int variant, int64_t b1, int64_t b2, uint64_t an,
     const uint64_t La = cdiv(an * sb, 64), Lb = cdiv(bn * sb, 64);
     const uint64_t np = (uint64_t)fa_ks_nprod(variant);
     uint64_t w = np * (La + Lb) + np * (La + Lb) + cdiv(an + bn, 2) + 8;
-    if (variant) w += 1 + cdiv(2 * (an + bn), 8);
+    if (variant) w += 1;
     return w;
 }
 
@@ -687,12 +687,8 @@ void fa_ks_record(uint64_t sb, const uint64_t* a, uint64_t aw, uint64_t an, cons
     r->zl = zl;
     r->cnt = cnt;
     r->zn = an + bn - 1;
-    r->top = zl + cnt < r->zn ? zl + cnt : r->zn;
     r->lowa = K.lowa;
     r->lowb = K.lowb;
-    r->bra = K.bra;
-    r->brb = K.brb;
-    r->tk = K.tk;
     r->sig = K.sig;
     r->pa = K.pa[0];
     r->pb = K.pb[0];
@@ -706,13 +702,13 @@ int fa_ks_pre_v(int variant, const uint64_t* a, uint64_t aw, uint64_t an, const 
     ks_layout K = ks_lay(variant, sb, an, bn, scratch);
     if (variant) {
         FA_LAUNCH("fa_k_ks_sflags", fa_k_ks_sflags, dim3(1), dim3(1024), 0, s, a, (int)aw, an,
-                  K.lowa, K.bra, K.sig);
+                  K.lowa, K.sig);
         FA_LAUNCH("fa_k_ks_sflags", fa_k_ks_sflags, dim3(1), dim3(1024), 0, s, b, (int)bw, bn,
-                  K.lowb, K.brb, K.sig + 1);
+                  K.lowb, K.sig + 1);
         FA_LAUNCH("fa_k_ks_spack", fa_k_ks_spack, dim3((unsigned)cdiv(K.La, 256)), dim3(256), 0, s,
-                  a, (int)aw, an, K.lowa, K.bra, K.sig, sb, K.pa[0], K.La);
+                  a, (int)aw, an, K.lowa, K.sig, sb, K.pa[0], K.La);
         FA_LAUNCH("fa_k_ks_spack", fa_k_ks_spack, dim3((unsigned)cdiv(K.Lb, 256)), dim3(256), 0, s,
-                  b, (int)bw, bn, K.lowb, K.brb, K.sig + 1, sb, K.pb[0], K.Lb);
+                  b, (int)bw, bn, K.lowb, K.sig + 1, sb, K.pb[0], K.Lb);
         return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "ks pack launch");
     }
     FA_LAUNCH("fa_k_ks_low", fa_k_ks_low, dim3((unsigned)cdiv(an, 256)), dim3(256), 0, s, a,
@@ -736,12 +732,8 @@ int fa_ks_post_v(int variant, uint64_t sb, uint64_t an, uint64_t bn, uint64_t* s
     ks_layout K = ks_lay(variant, sb, an, bn, scratch);
     const uint64_t zn = an + bn - 1;
     if (variant) {
-        const uint64_t top = zl + cnt < zn ? zl + cnt : zn;   // slots the window reads up to
-        if (top > 0)
-            FA_LAUNCH("fa_k_ks_uscan", fa_k_ks_uscan, dim3(1), dim3(1024), 0, s, K.pr[0], K.nP, sb,
-                      top, K.tk);
         FA_LAUNCH("fa_k_ks_unpack", fa_k_ks_unpack, dim3((unsigned)cdiv(cnt, 256)), dim3(256), 0, s,
-                  K.pr[0], K.nP, sb, K.tk, K.sig, zl, cnt, zn, (int)zw, z);
+                  K.pr[0], K.nP, sb, K.sig, zl, cnt, zn, (int)zw, z);
         return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "ks unpack launch");
     }
     FA_LAUNCH("fa_k_ks_combine", fa_k_ks_combine, dim3((unsigned)cdiv(cnt, 256)), dim3(256), 0, s,

@@ -639,18 +639,6 @@ FA_DEV void fa_add_one(uint64_t* __restrict__ pz, int n)
     }
 }
 
-// carries through 64 positions with generate and propagate masks G, P (no
-// position both): the carries into the positions for a carry c into the
-// first, and through cout the carry out of the last
-FA_DEV uint64_t fa_gp_carries(uint64_t G, uint64_t P, uint32_t c, uint32_t* cout)
-{
-    const uint64_t X = G | P;
-    const uint64_t s1 = G + X;
-    const uint64_t s2 = s1 + c;
-    *cout = (uint32_t)(s1 < X) | (uint32_t)(s2 < s1);
-    return s2 ^ X ^ G;
-}
-
 // carries between CRT workgroups ("blocks" of bl limbs), for the blocks
 // [b0, b1).  A block's aggregate holds bit 0: carry out with no carry in, bit
 // 1: all its limbs are ones.

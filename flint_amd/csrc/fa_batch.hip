@@ -10,7 +10,8 @@
 //     transform, binned by (depth, import kind), every workgroup taking one
 //     (product, prime, operand, tile) item of its bin's work list;
 //   - CRT: integer products binned by prime count (then one carry
-//     workgroup per product), nmod and fmpz windows in 256-coefficient chunks.
+//     workgroup per product), nmod windows in chunks of FA_NMOD_BLK coefficients,
+//     fmpz windows in chunks of 256.
 // The launch sequence is captured once into a hipGraph (FA_BATCH_GRAPH) and
 // replayed by fa_batch_launch.  No memset node is recorded: every output
 // word is written by a kernel (outputs past the product are written as 0).
@@ -536,7 +537,9 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             }
             prec.push_back(b);
             auto& w = q.kind == FA_REQ_NMOD ? nmod_w : fmpz_w;
-            for (uint64_t c = 0; c < (p.cnt + 255) / 256; c++) w.push_back((uint64_t)pid | (c << 32));
+            const uint64_t blk = q.kind == FA_REQ_NMOD ? FA_NMOD_BLK : 256;
+            for (uint64_t c = 0; c < (p.cnt + blk - 1) / blk; c++)
+                w.push_back((uint64_t)pid | (c << 32));
         }
     }
     B->jobs = L.take(jobs.size() * sizeof(fa_bjob) + 8);

@@ -210,6 +210,7 @@ struct fa_bmpn {               // integer product
     uint8_t* agg;              // their carry aggregates
     int bits, np;
 };
+#define FA_NMOD_BLK 1024          // outputs per workgroup of the batched nmod CRT
 struct fa_bpoly {              // nmod or fmpz polynomial product
     const double* Q;           // residue rows; null: the zero product (n = 1)
     uint64_t stride;

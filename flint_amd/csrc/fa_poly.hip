@@ -110,47 +110,56 @@ FA_DEV void fa_crt_coeff_poly(const double* __restrict__ Q, uint64_t stride, uin
 // in FP64 mulmods, then c mod n by Horner's rule over the digits with
 // 128-bit products.  c is the same integer in [0, M) as the limb-by-limb
 // recombination gives, found without its rounded quotient: every step is
-// exact.  Bounds: each mulmod sees |a b| < 2 p_k^2 (primes within a factor
-// 2 of each other, the running value reduced to [-p_k/2, p_k/2] first), and
-// v (p_k mod n) + t_k < n 2^64 keeps the high word below n.
+// exact.  A mulmod of |a b| < P p^2, P < 4, gives at most (1/2 + P'/4) p with
+// P' the power of two from P on; the primes are within a factor 2 of each
+// other, so a digit t_i is below 2 p_k.  Values are reduced only where these
+// bounds ask for it (in units of p = p_k):
+//   x = Q in [-1/2, 1/2]; r = x gcm: 3/4, so t_0 = r or r + p;
+//   u = t_(k-1) < 2, then u gpm + t_i: 1 + 2 = 3, then 3/2 + 2 = 7/2 for good;
+//   (r - u) ginv: 11/4 for k = 1, 15/4 for k = 2, else u is reduced first;
+//   t_k by one reduction to [0, 1).
+// Horner: v pk + t < 2^64 n for v < 2^50 or v < n keeps the high word below
+// n, so the top digit needs no reduction of its own.
 // p_k mod n for the primes of C, computed once per workgroup into pm
 // (threads 0..7; the caller puts a barrier after it)
-FA_DEV void fa_crt_nmod_pm(const fa_crt_consts& C, uint64_t n, uint64_t dinv, int norm,
-                           uint64_t* pm)
+template <class CC>
+FA_DEV void fa_crt_nmod_pm(const CC& C, uint64_t n, uint64_t dinv, int norm, uint64_t* pm)
 {
     const int k = threadIdx.x;
     if (k < FA_NPRIMES) pm[k] = k < C.np ? fa_ll_mod_preinv(0, (uint64_t)C.p[k], n, dinv, norm) : 0;
 }
 
-template <int NP>
-FA_DEV uint64_t fa_crt_nmod_one(const double* __restrict__ Q, uint64_t stride, uint64_t j,
-                                const fa_crt_consts& C, uint64_t n, uint64_t dinv, int norm,
-                                const uint64_t* pm)
+// an integer in [0, 2^52) held in a double, as a 64-bit word
+FA_DEV uint64_t fa_u52(double x)
 {
-    const uint64_t pos = fa_res_pos(j, stride);
+    return (uint64_t)__double_as_longlong(x + 4503599627370496.0) & 0xfffffffffffffu;
+}
+
+template <int NP, class CC>
+FA_DEV uint64_t fa_crt_nmod_value(const double* q, const CC& C, uint64_t n, uint64_t dinv,
+                                  int norm, const uint64_t* pm)
+{
     double t[NP];
-    {
-        const double p = C.p[0], pinv = C.pinv[0];
-        const double x = (double)fa_reduce_0n_u64(Q[pos], p, pinv);
-        t[0] = (double)fa_reduce_0n_u64(fa_mulmod(x, C.gcm[0], p, pinv), p, pinv);
-    }
 #pragma unroll
-    for (int k = 1; k < NP; k++) {
+    for (int k = 0; k < NP; k++) {
         const double p = C.p[k], pinv = C.pinv[k];
-        const double x = (double)fa_reduce_0n_u64(Q[(uint64_t)k * stride + pos], p, pinv);
-        const double r = fa_mulmod(x, C.gcm[k], p, pinv);   // c mod p_k, in (-p_k, p_k)
-        double u = t[k - 1];
+        const double r = fa_mulmod(fa_reduce_pm1n(q[k], p, pinv), C.gcm[k], p, pinv);
+        double y = r;                                       // c mod p_k
+        if (k > 0) {
+            double u = t[k - 1];
 #pragma unroll
-        for (int i = k - 2; i >= 0; i--)
-            u = fa_reduce_pm1n(fa_mulmod(u, C.gpm[k][i], p, pinv) + t[i], p, pinv);
-        u = fa_reduce_pm1n(u, p, pinv);
-        t[k] = (double)fa_reduce_0n_u64(fa_mulmod(r - u, C.ginv[k], p, pinv), p, pinv);
+            for (int i = k - 2; i >= 0; i--) u = fa_mulmod(u, C.gpm[k][i], p, pinv) + t[i];
+            if (k > 2) u = fa_reduce_pm1n(u, p, pinv);
+            y = fa_reduce_pm1n(fa_mulmod(r - u, C.ginv[k], p, pinv), p, pinv);
+        }
+        t[k] = y < 0.0 ? y + p : y;
     }
-    uint64_t v = fa_ll_mod_preinv(0, (uint64_t)t[NP - 1], n, dinv, norm);
+    uint64_t v = fa_u52(t[NP - 1]);
+    if (NP == 1) return fa_ll_mod_preinv(0, v, n, dinv, norm);
 #pragma unroll
     for (int k = NP - 2; k >= 0; k--) {
         const uint64_t pk = pm[k];
-        const uint64_t tk = (uint64_t)t[k];
+        const uint64_t tk = fa_u52(t[k]);
         uint64_t lo = v * pk;
         uint64_t hi = __umul64hi(v, pk);
         lo += tk;
@@ -160,6 +169,33 @@ FA_DEV uint64_t fa_crt_nmod_one(const double* __restrict__ Q, uint64_t stride, u
     return v;
 }
 
+// coefficients [j0, j0 + cnt) into z, cnt <= 256 K, K per thread; the
+// residues are requested before the workgroup's pm is formed
+template <int NP, int K, class CC>
+FA_DEV void fa_crt_nmod_block(const double* Q, uint64_t stride, uint64_t j0, uint64_t cnt,
+                              const CC& C, uint64_t n, uint64_t dinv, int norm, uint64_t* z,
+                              uint64_t* pm)
+{
+    typedef __attribute__((address_space(1))) uint64_t gT;
+    double q[K][NP];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        uint64_t t = 256 * (uint64_t)k + threadIdx.x;
+        if (t >= cnt) t = cnt - 1;
+        const uint32_t at = (uint32_t)fa_res_pos(j0 + t, stride) * 8u;
+#pragma unroll
+        for (int i = 0; i < NP; i++) q[k][i] = fa_ld<double>(Q + (uint64_t)i * stride, at);
+    }
+    fa_crt_nmod_pm(C, n, dinv, norm, pm);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const uint64_t t = 256 * (uint64_t)k + threadIdx.x;
+        const uint64_t v = fa_crt_nmod_value<NP>(q[k], C, n, dinv, norm, pm);
+        if (t < cnt) ((gT*)z)[t] = v;
+    }
+}
+
 template <int NP>
 __global__ void __launch_bounds__(256) fa_k_crt_nmod(const double* __restrict__ Q, uint64_t stride,
                                                      fa_crt_consts C, uint64_t zl, uint64_t cnt,
@@ -167,11 +203,9 @@ __global__ void __launch_bounds__(256) fa_k_crt_nmod(const double* __restrict__ 
                                                      uint64_t* __restrict__ z)
 {
     __shared__ uint64_t pm[FA_NPRIMES];
-    fa_crt_nmod_pm(C, n, dinv, norm, pm);
-    __syncthreads();
-    uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    z[t] = fa_crt_nmod_one<NP>(Q, stride, zl + t, C, n, dinv, norm, pm);
+    const uint64_t t0 = (uint64_t)blockIdx.x * 256;
+    fa_crt_nmod_block<NP, 1>(Q, stride, zl + t0, cnt - t0 < 256 ? cnt - t0 : 256, C, n, dinv, norm,
+                             z + t0, pm);
 }
 
 // NP = C.np (1 .. 8) as a template argument
@@ -251,10 +285,9 @@ __global__ void __launch_bounds__(256) fa_k_crt_fmpz(const double* __restrict__ 
     default: F(8); break;       \
     }
 
-// batched nmod / fmpz CRT: work item = job | chunk << 32, 256 outputs per
-// chunk; outputs at or beyond the product length are zero
-template <int FMPZ>
-__global__ void __launch_bounds__(256) fa_kb_crt_poly(const fa_bpoly* __restrict__ P,
+// batched fmpz CRT: work item = job | chunk << 32, 256 outputs per chunk;
+// outputs at or beyond the product length are zero
+__global__ void __launch_bounds__(256) fa_kb_crt_fmpz(const fa_bpoly* __restrict__ P,
                                                       const uint64_t* __restrict__ work,
                                                       unsigned nwork)
 {
@@ -263,36 +296,57 @@ __global__ void __launch_bounds__(256) fa_kb_crt_poly(const fa_bpoly* __restrict
     if (L >= nwork) return;
     const uint64_t w = work[L];
     const fa_bpoly& j = P[(unsigned)(w & 0xffffffffu)];
-    __shared__ uint64_t pm[FA_NPRIMES];
-    if (!FMPZ && j.Q) {         // the same job for the whole workgroup
-        fa_crt_nmod_pm(*(const fa_crt_consts*)j.C, j.n, j.dinv, j.norm, pm);
-        __syncthreads();
-    }
     const uint64_t t = (w >> 32) * 256 + threadIdx.x;
     if (t >= j.cnt) return;
     const uint64_t idx = j.zl + t;
-    if (FMPZ) {
-        uint64_t* o = j.z + t * (uint64_t)j.zw;
-        if (idx >= j.zn || !j.Q) {
-            for (int l = 0; l < j.zw; l++) o[l] = 0;
-            return;
-        }
-        const fa_crt_consts& C = *(const fa_crt_consts*)j.C;
-#define FA_KB_FMPZ(NL) fa_crt_fmpz_one<NL>(j.Q, j.stride, idx, C, o, (uint64_t)j.zw)
-        FA_CRT_NL_SWITCH(fa_crt_poly_limbs(C), FA_KB_FMPZ)
-#undef FA_KB_FMPZ
-    } else {
-        if (idx >= j.zn || !j.Q) {
-            j.z[t] = 0;
-            return;
-        }
-        const fa_crt_consts& C = *(const fa_crt_consts*)j.C;
-        uint64_t r = 0;
-#define FA_KB_NMOD(NP) r = fa_crt_nmod_one<NP>(j.Q, j.stride, idx, C, j.n, j.dinv, j.norm, pm)
-        FA_CRT_NP_SWITCH(C.np, FA_KB_NMOD)
-#undef FA_KB_NMOD
-        j.z[t] = r;
+    uint64_t* o = j.z + t * (uint64_t)j.zw;
+    if (idx >= j.zn || !j.Q) {
+        for (int l = 0; l < j.zw; l++) o[l] = 0;
+        return;
     }
+    const fa_crt_consts& C = *(const fa_crt_consts*)j.C;
+#define FA_KB_FMPZ(NL) fa_crt_fmpz_one<NL>(j.Q, j.stride, idx, C, o, (uint64_t)j.zw)
+    FA_CRT_NL_SWITCH(fa_crt_poly_limbs(C), FA_KB_FMPZ)
+#undef FA_KB_FMPZ
+}
+
+// batched nmod CRT: work item = job | chunk << 32, FA_NMOD_BLK outputs per
+// chunk.  A workgroup goes through five dependent steps (work item, record,
+// constants, p_k mod n, residues) before it computes, so each takes four
+// outputs per thread; the constants are read through the scalar cache.
+// (A batch of about 79 million outputs: 1050 us with one output per thread and
+// every value reduced, 427 now.)  A modulus below 2^64 and a length below 2^40
+// need at most 2^168 < p_0 p_1 p_2 p_3.
+__global__ void __launch_bounds__(256) fa_kb_crt_nmod(const fa_bpoly* __restrict__ P,
+                                                      const uint64_t* __restrict__ work,
+                                                      unsigned nwork)
+{
+    typedef __attribute__((address_space(4))) const fa_crt_consts cC;
+    const unsigned nb = gridDim.x, bid = blockIdx.x;
+    const unsigned L = (bid & 7) * (nb >> 3) + (bid >> 3);
+    if (L >= nwork) return;
+    const uint64_t w = work[L];
+    const fa_bpoly& j = P[(unsigned)(w & 0xffffffffu)];
+    __shared__ uint64_t pm[FA_NPRIMES];
+    const uint64_t t0 = (w >> 32) * FA_NMOD_BLK;
+    if (t0 >= j.cnt) return;
+    uint64_t cnt = j.cnt - t0 < FA_NMOD_BLK ? j.cnt - t0 : FA_NMOD_BLK;
+    const uint64_t j0 = j.zl + t0;
+    // the outputs of this chunk below the product's length
+    const uint64_t live = !j.Q || j0 >= j.zn ? 0 : j.zn - j0 < cnt ? j.zn - j0 : cnt;
+    for (uint64_t t = live + threadIdx.x; t < cnt; t += 256) j.z[t0 + t] = 0;
+    if (!live) return;
+    cC& C = *(cC*)j.C;
+#define FA_KB_NMOD(NP)                                                                          \
+    fa_crt_nmod_block<NP, FA_NMOD_BLK / 256>(j.Q, j.stride, j0, live, C, j.n, j.dinv, j.norm,   \
+                                             j.z + t0, pm)
+    switch (C.np) {
+    case 1: FA_KB_NMOD(1); break;
+    case 2: FA_KB_NMOD(2); break;
+    case 3: FA_KB_NMOD(3); break;
+    default: FA_KB_NMOD(4); break;
+    }
+#undef FA_KB_NMOD
 }
 
 int fa_batch_crt_poly(int fmpz, const fa_bpoly* P, const uint64_t* work, unsigned nwork,
@@ -301,9 +355,9 @@ int fa_batch_crt_poly(int fmpz, const fa_bpoly* P, const uint64_t* work, unsigne
     if (!nwork) return FA_OK;
     const unsigned grid = (nwork + 7) & ~7u;
     if (fmpz)
-        FA_LAUNCH("fa_kb_crt_fmpz", fa_kb_crt_poly<1>, dim3(grid), dim3(256), 0, s, P, work, nwork);
+        FA_LAUNCH("fa_kb_crt_fmpz", fa_kb_crt_fmpz, dim3(grid), dim3(256), 0, s, P, work, nwork);
     else
-        FA_LAUNCH("fa_kb_crt_nmod", fa_kb_crt_poly<0>, dim3(grid), dim3(256), 0, s, P, work, nwork);
+        FA_LAUNCH("fa_kb_crt_nmod", fa_kb_crt_nmod, dim3(grid), dim3(256), 0, s, P, work, nwork);
     return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "batch crt launch");
 }
 

@@ -35,17 +35,35 @@ __global__ void __launch_bounds__(256) fa_k_small_conv(fa_operand a, fa_operand 
     const double n = S.p[i], ninv = S.pinv[i];
     const int N = 1 << depth;
     double* sa = lds;
-    double* sb = sqr ? lds : lds + N;
-    for (int x = threadIdx.x; x < N; x += blockDim.x) {
-        sa[x] = fa_operand_value(a, (uint64_t)x, S.pow2[i], n, ninv);
-        if (!sqr) sb[x] = fa_operand_value(b, (uint64_t)x, S.pow2[i], n, ninv);
-    }
-    __syncthreads();
-    fa_lds_fwd(sa, depth, 0, 0, S.w2[i], n, ninv);
-    if (!sqr) fa_lds_fwd(sb, depth, 0, 0, S.w2[i], n, ninv);
     const double m = S.norm[i];
-    for (int x = threadIdx.x; x < N; x += blockDim.x)
-        sa[x] = fa_mulmod(fa_mulmod(sa[x], m, n, ninv), sb[x], n, ninv);
+    if (!sqr && N <= 256) {
+        // up to one point per thread the two operands go through the import
+        // and the forward passes together, as two interleaved columns: these
+        // are chains of latencies (7.2 -> 4.9 us for 24 x 17 limbs).  Above, the
+        // passes are long enough to fill the workgroup one after the other.
+        for (int u = threadIdx.x; u < 2 * N; u += blockDim.x) {
+            const int sel = u >> depth, x = u & (N - 1);
+            lds[2 * x + sel] = fa_operand_value(sel ? b : a, (uint64_t)x, S.pow2[i], n, ninv);
+        }
+        __syncthreads();
+        fa_lds_fwd(lds, depth, 1, 0, S.w2[i], n, ninv);
+        const int x = threadIdx.x;
+        double v = 0.0;
+        if (x < N) v = fa_mulmod(fa_mulmod(lds[2 * x], m, n, ninv), lds[2 * x + 1], n, ninv);
+        __syncthreads();
+        if (x < N) sa[x] = v;
+    } else {
+        double* sb = sqr ? lds : lds + N;
+        for (int x = threadIdx.x; x < N; x += blockDim.x) {
+            sa[x] = fa_operand_value(a, (uint64_t)x, S.pow2[i], n, ninv);
+            if (!sqr) sb[x] = fa_operand_value(b, (uint64_t)x, S.pow2[i], n, ninv);
+        }
+        __syncthreads();
+        fa_lds_fwd(sa, depth, 0, 0, S.w2[i], n, ninv);
+        if (!sqr) fa_lds_fwd(sb, depth, 0, 0, S.w2[i], n, ninv);
+        for (int x = threadIdx.x; x < N; x += blockDim.x)
+            sa[x] = fa_mulmod(fa_mulmod(sa[x], m, n, ninv), sb[x], n, ninv);
+    }
     __syncthreads();
     fa_lds_inv(sa, depth, 0, 0, S.w2inv[i], n, ninv);
     double* o = out + (uint64_t)i * stride;

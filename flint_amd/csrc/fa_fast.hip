@@ -1045,9 +1045,7 @@ FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int g, double n, double ni
 // L2 beside the tiles, so the blocks there are 64 columns (the whole product
 // 2.33 ms; 2.48 with 512).
 #define FA_COL_BLOCK 512
-#ifndef FA_COLW_BLOCK
 #define FA_COLW_BLOCK 64
-#endif
 template <int CPW, int BLOCK>
 constexpr int fa_col_block() { return BLOCK / CPW < 2 ? 2 : BLOCK / CPW; }
 

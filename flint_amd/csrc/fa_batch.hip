@@ -9,9 +9,9 @@
 //   - depth 13..24: the column / row / column passes of the two-level
 //     transform, binned by (depth, import kind), every workgroup taking one
 //     (product, prime, operand, tile) item of its bin's work list;
-//   - CRT: integer products binned by prime count (then one carry
-//     workgroup per product), nmod windows in chunks of FA_NMOD_BLK coefficients,
-//     fmpz windows in chunks of 256.
+//   - CRT: integer products binned by prime count (then the carries between
+//     their workgroups, FA_CARRY_SEG per wave), nmod windows in chunks of
+//     FA_NMOD_BLK coefficients, fmpz windows in chunks of 256.
 // The launch sequence is captured once into a hipGraph (FA_BATCH_GRAPH) and
 // replayed by fa_batch_launch.  No memset node is recorded: every output
 // word is written by a kernel (outputs past the product are written as 0).
@@ -137,7 +137,7 @@ struct fa_batch_s {
     size_t jobs;                                  // fa_bjob[]
     size_t mpn_rec, fp_consts[FA_NPRIMES + 1];    // fa_bmpn[], fa_crt_fp_consts per np
     std::vector<std::pair<int, std::pair<size_t, unsigned>>> crt_mpn;     // np -> (work, n)
-    size_t carry_jobs;
+    size_t carry_work;
     unsigned ncarry;
     size_t poly_rec;
     size_t nmod_work, fmpz_work;
@@ -188,7 +188,7 @@ static int batch_record(fa_batch_s* B, hipStream_t s)
                               d + B->fp_consts[c.first], s);
         if (rc) return rc;
     }
-    rc = fa_batch_carry(M, (const unsigned*)(d + B->carry_jobs), B->ncarry, s);
+    rc = fa_batch_carry(M, (const uint64_t*)(d + B->carry_work), B->ncarry, s);
     if (rc) return rc;
     const fa_bpoly* P = (const fa_bpoly*)(d + B->poly_rec);
     rc = fa_batch_crt_poly(0, P, (const uint64_t*)(d + B->nmod_work), B->nnmod, s);
@@ -430,7 +430,7 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
     std::map<bin_key, std::vector<uint64_t>> small_bins;
     std::map<bin_key, tbin> trans_bins;
     std::map<int, std::vector<uint64_t>> crt_bins;
-    std::vector<unsigned> carry;
+    std::vector<uint64_t> carry;
     std::vector<uint64_t> nmod_w, fmpz_w;
     for (int64_t r = 0; r < ntot; r++) {
         fa_request& q = req(r);
@@ -516,7 +516,9 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             mrec.push_back(m);
             auto& w = crt_bins[p.np];
             for (uint64_t blk = 0; blk < p.nblk; blk++) w.push_back((uint64_t)mid | (blk << 32));
-            if (p.nblk > 1) carry.push_back(mid);   // one workgroup resolves its own
+            if (p.nblk > 1)   // one workgroup resolves its own
+                for (uint64_t seg = 0; seg * FA_CARRY_SEG < p.nblk; seg += FA_CARRY_WG)
+                    carry.push_back((uint64_t)mid | (seg << 32));
         } else {
             const unsigned pid = (unsigned)prec.size();
             rec_of[(size_t)r] = (int)pid;
@@ -562,7 +564,7 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
     }
     for (auto& e : crt_bins) B->crt_mpn.push_back({e.first, {L.take(e.second.size() * 8),
                                                              (unsigned)e.second.size()}});
-    B->carry_jobs = L.take(carry.size() * 4 + 8);
+    B->carry_work = L.take(carry.size() * 8 + 8);
     B->ncarry = (unsigned)carry.size();
     // signed-slot KS products: record index k of ks_live, work items in
     // blocks of FA_KS_PACK_BLK packed limbs (per operand) and 256 output
@@ -708,7 +710,7 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
         k = 0;
         for (auto& e : crt_bins) { put(B->crt_mpn[k].second.first, e.second.data(), e.second.size() * 8); k++; }
     }
-    put(B->carry_jobs, carry.data(), carry.size() * 4);
+    put(B->carry_work, carry.data(), carry.size() * 8);
     {
         std::vector<fa_bks> recs(ks_live.size());
         for (size_t i = 0; i < ks_live.size(); i++) {

@@ -210,6 +210,8 @@ struct fa_bmpn {               // integer product
     uint8_t* agg;              // their carry aggregates
     int bits, np;
 };
+#define FA_CARRY_SEG 16           // CRT workgroups per wave of the carry kernels
+#define FA_CARRY_WG 4             // waves per workgroup of these
 #define FA_NMOD_BLK 1024          // outputs per workgroup of the batched nmod CRT
 struct fa_bpoly {              // nmod or fmpz polynomial product
     const double* Q;           // residue rows; null: the zero product (n = 1)
@@ -224,7 +226,7 @@ struct fa_bpoly {              // nmod or fmpz polynomial product
 extern "C++" {
 int fa_batch_crt_mpn(int np, const fa_bmpn* M, const uint64_t* work, unsigned nwork,
                      const void* F, hipStream_t s);
-int fa_batch_carry(const fa_bmpn* M, const unsigned* jobs, unsigned njobs, hipStream_t s);
+int fa_batch_carry(const fa_bmpn* M, const uint64_t* work, unsigned nwork, hipStream_t s);
 int fa_nmod_primes(const fa_tables* T, uint64_t len, uint64_t n, int* np, int* offset);
 // transform depth of the window [zl, zh) of a zn-coefficient product, with
 // the wraparound of plan.c:47-89 when it leaves the window exact

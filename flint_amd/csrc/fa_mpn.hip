@@ -634,110 +634,145 @@ __global__ void __launch_bounds__(256) fa_k_crt_mpn16(const double* __restrict__
     }
 }
 
-// adds 1 to the n limbs at p with carry (stops at the first limb that does
-// not wrap); eight loads in flight at a time
-FA_DEV void fa_add_one(uint64_t* __restrict__ pz, int n)
+typedef __attribute__((address_space(1))) uint64_t fa_gw;   // global words
+
+// adds 1 to the n <= 8 limbs at p, all loaded together; whether the carry
+// leaves the last of them
+FA_DEV bool fa_add_one(fa_gw* p, int n)
 {
-    typedef __attribute__((address_space(1))) uint64_t gT;
-    gT* p = (gT*)pz;
-    for (int l0 = 0; l0 < n; l0 += 8) {
-        const int m = n - l0 < 8 ? n - l0 : 8;
-        uint64_t v[8];
+    uint64_t v[8];
 #pragma unroll
-        for (int l = 0; l < 8; l++)
-            if (l < m) v[l] = p[l0 + l];
+    for (int l = 0; l < 8; l++)
+        if (l < n) v[l] = p[l];
 #pragma unroll
-        for (int l = 0; l < 8; l++) {
-            if (l < m) {
-                v[l] += 1;
-                p[l0 + l] = v[l];
-                if (v[l] != 0) return;
+    for (int l = 0; l < 8; l++) {
+        if (l < n) {
+            v[l] += 1;
+            p[l] = v[l];
+            if (v[l] != 0) return false;
+        }
+    }
+    return true;
+}
+
+// bit 0 of each byte of w as a mask of eight bits
+FA_DEV uint32_t fa_byte_bits(uint64_t w)
+{
+    return (uint32_t)(((w & UINT64_C(0x0101010101010101)) * UINT64_C(0x0102040810204080)) >> 56);
+}
+
+// carries between CRT workgroups ("blocks" of bl limbs), for the FA_CARRY_SEG
+// blocks from b0 (a multiple of it) by one wave.  A block's aggregate holds
+// bit 0: carry out with no carry in, bit 1: all its limbs are ones.
+//  1. the carry into b0: the 64 blocks before it, one per lane; while all of
+//     a step's blocks propagate, the 2048 before them, 32 per lane;
+//  2. the carries into the segment's blocks, from its ballots;
+//  3. a block with a carry-in adds it to its limbs.  The addition leaves the
+//     block only if all its limbs are ones, which the propagate bit has
+//     already told the next block, so blocks are independent.  A run of blocks
+//     of ones becomes zeros by the whole wave's stores, with no loads.  In any
+//     other block one lane adds to the first eight limbs; where the carry runs
+//     on, the wave takes 256 limbs at a time.
+// Latency bound on random operands: 4 us for the 63,671 blocks of 2^24 x 2^24
+// limbs, 2 to 3 us for a 65,536-limb square (529 blocks).  (2^(64 n) - 1)^2
+// makes every block of the product's lower half a block of ones with a
+// carry-in: 5 us at n = 2^16 and 22 us at 2^24, where one lane walking each
+// block, its loads and stores a block away from the next lane's, took 80 us
+// and 1.4 ms.
+FA_DEV void fa_carry_resolve(const uint8_t* __restrict__ aggp, uint64_t* __restrict__ zp,
+                             uint64_t zn, uint32_t bl, uint64_t nblk, uint64_t b0)
+{
+    typedef __attribute__((address_space(1))) const uint8_t gB;
+    typedef __attribute__((address_space(1))) const uint64_t gC;
+    gB* agg = (gB*)aggp;
+    fa_gw* z = (fa_gw*)zp;
+    const int lane = threadIdx.x & 63;
+    if (b0 >= nblk) return;
+    const uint64_t b = b0 + lane;
+    const bool mine = lane < FA_CARRY_SEG && b < nblk;
+    const uint8_t f = mine ? agg[b] : 0;
+    // 1.
+    uint32_t c = 0;
+    int64_t hi = (int64_t)b0;
+    if (hi > 0) {
+        const uint8_t before = hi - 64 + lane >= 0 ? agg[hi - 64 + lane] : 0;
+        uint64_t all = __ballot(before & 2);
+        (void)fa_gp_carries(__ballot(before & 1), all, 0, &c);
+        for (hi -= 64; hi > 0 && !~all; hi -= 2048) {
+            const int64_t at = hi - 2048 + 32 * lane;   // a multiple of 16
+            uint32_t G = 0, P = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint64_t w = at + 8 * k >= 0 ? *(gC*)(agg + at + 8 * k) : 0;
+                G |= fa_byte_bits(w) << (8 * k);
+                P |= fa_byte_bits(w >> 1) << (8 * k);
+            }
+            all = __ballot(P == ~0u);
+            (void)fa_gp_carries(__ballot(((uint64_t)G + (G | P)) >> 32), all, 0, &c);
+        }
+    }
+    // 2.
+    uint32_t o;
+    const uint64_t cin = fa_gp_carries(__ballot(f & 1), __ballot(f & 2), c, &o);
+    // 3.
+    const uint64_t zb = b * bl;
+    const bool in = mine && ((cin >> lane) & 1) && zb < zn;
+    bool on = false;
+    if (in && !(f & 2)) {
+        const uint64_t n = zn - zb < bl ? zn - zb : bl;
+        on = fa_add_one(z + zb, n < 8 ? (int)n : 8);
+    }
+    uint32_t ones = (uint32_t)__ballot(in && (f & 2));
+    while (ones) {
+        typedef uint64_t u64x2 __attribute__((ext_vector_type(2), aligned(8)));
+        typedef __attribute__((address_space(1))) u64x2 g2;
+        const int l = __builtin_ctz(ones), run = __builtin_ctz(~(ones >> l));
+        const uint64_t i0 = (b0 + l) * bl, e = (b0 + l + run) * bl;
+        const uint64_t i1 = e < zn ? e : zn;
+        ones &= ~(((1u << run) - 1) << l);
+        for (uint64_t i = i0 + 2 * lane; i + 1 < i1; i += 128) *(g2*)(z + i) = u64x2{0, 0};
+        if (lane == 0 && ((i1 - i0) & 1)) z[i1 - 1] = 0;
+    }
+    uint32_t rest = (uint32_t)__ballot(on);
+    while (rest) {
+        const int l = __builtin_ctz(rest);
+        rest &= rest - 1;
+        const uint64_t i0 = (b0 + l) * bl, i1 = i0 + bl < zn ? i0 + bl : zn;
+        bool done = false;
+        for (uint64_t i = i0 + 8 + lane; !done && i - lane < i1; i += 256) {
+            uint64_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = i + 64 * k < i1 ? z[i + 64 * k] : ~UINT64_C(0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (!done) {
+                    const uint64_t m = __ballot(v[k] != ~UINT64_C(0));
+                    const int stop = m ? __builtin_ctzll(m) : 64;
+                    if (lane <= stop && i + 64 * k < i1) z[i + 64 * k] = v[k] + 1;
+                    done = m != 0;
+                }
             }
         }
     }
 }
 
-// carries between CRT workgroups ("blocks" of bl limbs), for the blocks
-// [b0, b1).  A block's aggregate holds bit 0: carry out with no carry in, bit
-// 1: all its limbs are ones.
-//  1. the carry into b0: the blocks before it, blockDim at a time from the
-//     nearest, until some block does not propagate (the first chunk, unless
-//     the product holds long runs of ones);
-//  2. tiles of blockDim blocks, one per thread: the carries into the blocks
-//     of a wave come from its ballots and the waves' masks in LDS;
-//  3. a block with a carry-in adds it to its limbs.  The addition leaves the
-//     block only if all its limbs are ones, which the propagate bit has
-//     already told the next block, so blocks are independent.
-// Latency bound: 25 -> 6 us for the 63,671 blocks of 2^24 x 2^24 limbs and 6
-// -> 1.5..2 us for a few blocks, against LDS scans of flag bytes by 1024
-// threads in 20 steps and one wave per block.
-FA_DEV void fa_carry_resolve(const uint8_t* __restrict__ agg, uint64_t* __restrict__ z,
-                             uint64_t zn, uint32_t bl, uint64_t nblk, uint64_t b0, uint64_t b1)
+__global__ void __launch_bounds__(64 * FA_CARRY_WG) fa_k_carry_fused(
+    const uint8_t* __restrict__ agg, uint64_t* __restrict__ z, uint64_t zn, uint32_t bl,
+    uint64_t nblk)
 {
-    __shared__ uint64_t sG[16], sP[16];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nt = blockDim.x, nw = nt >> 6;
-    uint32_t c = 0;
-    for (int64_t hi = (int64_t)b0; hi > 0; hi -= nt) {
-        const int64_t b = hi - nt + t;
-        const uint8_t a = b >= 0 ? agg[b] : 0;
-        const uint64_t G = __ballot(a & 1), P = __ballot(a & 2);
-        if (lane == 0) {
-            sG[wave] = G;
-            sP[wave] = P;
-        }
-        __syncthreads();
-        uint64_t all = ~UINT64_C(0);
-        c = 0;
-        for (int w = 0; w < nw; w++) {
-            uint32_t o;
-            (void)fa_gp_carries(sG[w], sP[w], c, &o);
-            c = o;
-            all &= sP[w];
-        }
-        __syncthreads();
-        if (~all) break;     // the same for every thread
-    }
-    for (uint64_t tb = b0; tb < b1; tb += nt) {
-        const uint64_t b = tb + (uint64_t)t;
-        const uint8_t a = b < b1 ? agg[b] : 0;
-        const uint64_t G = __ballot(a & 1), P = __ballot(a & 2);
-        if (lane == 0) {
-            sG[wave] = G;
-            sP[wave] = P;
-        }
-        __syncthreads();
-        uint32_t cw = 0;
-        for (int w = 0; w < nw; w++) {
-            if (w == wave) cw = c;
-            uint32_t o;
-            (void)fa_gp_carries(sG[w], sP[w], c, &o);
-            c = o;
-        }
-        uint32_t o;
-        const uint64_t cin = fa_gp_carries(G, P, cw, &o);
-        const uint64_t zb = b * bl;
-        if (b < b1 && ((cin >> lane) & 1) && zb < zn)
-            fa_add_one(z + zb, zn - zb < bl ? (int)(zn - zb) : (int)bl);
-        __syncthreads();
-    }
+    const uint64_t seg = (uint64_t)blockIdx.x * FA_CARRY_WG + (threadIdx.x >> 6);
+    fa_carry_resolve(agg, z, zn, bl, nblk, seg * FA_CARRY_SEG);
 }
 
-__global__ void __launch_bounds__(1024) fa_k_carry_fused(const uint8_t* __restrict__ agg,
-                                                         uint64_t* __restrict__ z, uint64_t zn,
-                                                         uint32_t bl, uint64_t nblk)
-{
-    const uint64_t b0 = (uint64_t)blockIdx.x * blockDim.x;
-    fa_carry_resolve(agg, z, zn, bl, nblk, b0, b0 + blockDim.x < nblk ? b0 + blockDim.x : nblk);
-}
-
-// one block per thread; a single block has no carry to receive
+// a single block has no carry to receive
 static void launch_carry(const uint8_t* agg, uint64_t* z, uint64_t zn, int own, uint64_t nblk,
                          hipStream_t s)
 {
     if (nblk < 2) return;
-    const unsigned nt = nblk < 1024 ? (unsigned)((nblk + 63) & ~UINT64_C(63)) : 1024u;
-    FA_LAUNCH("fa_k_carry_fused", fa_k_carry_fused, dim3((unsigned)((nblk + nt - 1) / nt)),
-              dim3(nt), 0, s, agg, z, zn, (uint32_t)(FA_CRT16_GROUPS - 1) * (uint32_t)own, nblk);
+    constexpr uint64_t per = FA_CARRY_SEG * FA_CARRY_WG;
+    FA_LAUNCH("fa_k_carry_fused", fa_k_carry_fused, dim3((unsigned)((nblk + per - 1) / per)),
+              dim3(64 * FA_CARRY_WG), 0, s, agg, z, zn,
+              (uint32_t)(FA_CRT16_GROUPS - 1) * (uint32_t)own, nblk);
 }
 
 // ------------------------------------------------------------------------
@@ -934,14 +969,16 @@ __global__ void __launch_bounds__(256) fa_kb_crt_fp(const fa_bmpn* __restrict__ 
     fa_crt_fp_block<NP>(m.Q, m.stride, *F, m.zlen, m.bits, m.z, m.zn, m.agg, w >> 32);
 }
 
-__global__ void __launch_bounds__(1024) fa_kb_carry(const fa_bmpn* __restrict__ M,
-                                                    const unsigned* __restrict__ jobs,
-                                                    unsigned njobs)
+// batched carries: work item = job | first segment << 32
+__global__ void __launch_bounds__(64 * FA_CARRY_WG) fa_kb_carry(const fa_bmpn* __restrict__ M,
+                                                                const uint64_t* __restrict__ work,
+                                                                unsigned nwork)
 {
-    if (blockIdx.x >= njobs) return;
-    const fa_bmpn& m = M[jobs[blockIdx.x]];
+    if (blockIdx.x >= nwork) return;
+    const uint64_t w = work[blockIdx.x];
+    const fa_bmpn& m = M[(unsigned)(w & 0xffffffffu)];
     fa_carry_resolve(m.agg, m.z, m.zn, (uint32_t)(FA_CRT16_GROUPS - 1) * (uint32_t)(m.bits / 8),
-                     m.nblk, 0, m.nblk);
+                     m.nblk, ((w >> 32) + (threadIdx.x >> 6)) * FA_CARRY_SEG);
 }
 
 int fa_batch_crt_mpn(int np, const fa_bmpn* M, const uint64_t* work, unsigned nwork,
@@ -963,10 +1000,10 @@ int fa_batch_crt_mpn(int np, const fa_bmpn* M, const uint64_t* work, unsigned nw
     return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "batch crt launch");
 }
 
-int fa_batch_carry(const fa_bmpn* M, const unsigned* jobs, unsigned njobs, hipStream_t s)
+int fa_batch_carry(const fa_bmpn* M, const uint64_t* work, unsigned nwork, hipStream_t s)
 {
-    if (!njobs) return FA_OK;
-    FA_LAUNCH("fa_kb_carry", fa_kb_carry, dim3(njobs), dim3(1024), 0, s, M, jobs, njobs);
+    if (!nwork) return FA_OK;
+    FA_LAUNCH("fa_kb_carry", fa_kb_carry, dim3(nwork), dim3(64 * FA_CARRY_WG), 0, s, M, work, nwork);
     return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "batch carry launch");
 }
 

@@ -6,7 +6,8 @@ that fall on a chunk, passes the excess to the next chunk, resolves the
 remaining single-bit carries from generate / propagate masks, and joins the
 chunks into words; the carry kernel then adds one to every block that receives
 a carry.  The model replays these steps (32-bit words, 64-lane masks, blocks
-of 248 chunks behind a halo of 8) and compares the limbs with the integer."""
+of 248 chunks behind a halo of 8, segments of 16 blocks) and compares the limbs
+with the integer."""
 import random
 from fractions import Fraction
 
@@ -81,20 +82,80 @@ def crt_blocks(coeffs, np_, own, zn):
         for w in range(4):
             cin, c = carries(G[w], P[w], c)
             out += [(T[64 * w + b] + ((cin >> b) & 1)) & ((1 << bits) - 1) for b in range(64)]
-        agg.append((c, allp))
+        agg.append((c, int(allp)))
         data = b"".join(v.to_bytes(own, "little") for v in out[8:])
         for i in range(31 * own):
             if blk * 31 * own + i < zn:
                 z[blk * 31 * own + i] = int.from_bytes(data[8 * i:8 * i + 8], "little")
-    cin = 0
-    for blk, (g, p) in enumerate(agg):
-        if cin:
-            for i in range(blk * 31 * own, min((blk + 1) * 31 * own, zn)):
+    bl = 31 * own
+    for blk, cin in enumerate(block_carries(agg)):
+        lo, hi = blk * bl, min((blk + 1) * bl, zn)
+        if cin and agg[blk][1]:
+            assert z[lo:hi] == [M64] * max(hi - lo, 0)
+            z[lo:hi] = [0] * max(hi - lo, 0)
+        elif cin:
+            for i in range(lo, hi):
                 z[i] = (z[i] + 1) & M64
                 if z[i]:
                     break
-        cin = g | (p and cin)
     return z
+
+
+def byte_bits(w):
+    return ((w & 0x0101010101010101) * 0x0102040810204080 & M64) >> 56
+
+
+def block_carries(agg):
+    """the carry into every block as fa_carry_resolve finds it: segments of 16
+    blocks, the 64 blocks before one, then 2048 at a time, 32 per lane"""
+    flags = [g | 2 * p for g, p in agg]
+    at = lambda i: flags[i] if 0 <= i < len(flags) else 0
+    out = []
+    for b0 in range(0, len(agg), 16):
+        c, hi = 0, b0
+        if hi > 0:
+            f = [at(hi - 64 + l) for l in range(64)]
+            every = sum((x >> 1) << l for l, x in enumerate(f))
+            _, c = carries(sum((x & 1) << l for l, x in enumerate(f)), every, 0)
+            hi -= 64
+            while hi > 0 and every == M64:
+                G = P = 0
+                for l in range(64):
+                    g = p = 0
+                    for k in range(4):
+                        i = hi - 2048 + 32 * l + 8 * k
+                        assert i % 8 == 0
+                        w = sum(at(i + b) << (8 * b) for b in range(8)) if i >= 0 else 0
+                        g |= byte_bits(w) << (8 * k)
+                        p |= byte_bits(w >> 1) << (8 * k)
+                    G |= ((g + (g | p)) >> 32) << l
+                    P |= (p == 0xFFFFFFFF) << l
+                _, c = carries(G, P, 0)
+                every = P
+                hi -= 2048
+        f = [at(b0 + l) if l < 16 else 0 for l in range(64)]
+        cin, _ = carries(sum((x & 1) << l for l, x in enumerate(f)),
+                         sum((x >> 1) << l for l, x in enumerate(f)), c)
+        out += [(cin >> l) & 1 for l in range(min(16, len(agg) - b0))]
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 80, 2111, 2112, 2113, 2129, 4300])
+def test_carries_between_blocks(n):
+    rng = random.Random(n)
+    for k in range(12):
+        agg = []
+        while len(agg) < n:      # (generate, propagate): runs of ones between them
+            run = int(2 ** rng.uniform(0, 12.5)) if k else n
+            agg += [(rng.getrandbits(1), 0)] + [(0, 1)] * run
+        agg = agg[:n]
+        if k == 1:
+            agg[0] = (0, 1)
+        want, c = [], 0
+        for g, p in agg:
+            want.append(c)
+            c = g | (p & c)
+        assert block_carries(agg) == want
 
 
 @pytest.mark.parametrize("np_,own", [(2, 3), (2, 4), (2, 6), (3, 4), (3, 9), (4, 12), (5, 15),

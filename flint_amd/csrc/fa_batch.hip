@@ -11,7 +11,7 @@
 //     (product, prime, operand, tile) item of its bin's work list;
 //   - CRT: integer products binned by prime count (then the carries between
 //     their workgroups, FA_CARRY_SEG per wave), nmod windows in chunks of
-//     FA_NMOD_BLK coefficients, fmpz windows in chunks of 256.
+//     256 or 1024 coefficients, fmpz windows in chunks of 256.
 // The launch sequence is captured once into a hipGraph (FA_BATCH_GRAPH) and
 // replayed by fa_batch_launch.  No memset node is recorded: every output
 // word is written by a kernel (outputs past the product are written as 0).
@@ -142,6 +142,7 @@ struct fa_batch_s {
     size_t poly_rec;
     size_t nmod_work, fmpz_work;
     unsigned nnmod, nfmpz;
+    int nmod_k;                        // nmod outputs per thread of the CRT
     // fmpz products routed through Kronecker substitution: packing before
     // the transforms, recombination after the integer CRT (device addresses)
     struct ksrec {
@@ -191,9 +192,9 @@ static int batch_record(fa_batch_s* B, hipStream_t s)
     rc = fa_batch_carry(M, (const uint64_t*)(d + B->carry_work), B->ncarry, s);
     if (rc) return rc;
     const fa_bpoly* P = (const fa_bpoly*)(d + B->poly_rec);
-    rc = fa_batch_crt_poly(0, P, (const uint64_t*)(d + B->nmod_work), B->nnmod, s);
+    rc = fa_batch_crt_poly(0, B->nmod_k, P, (const uint64_t*)(d + B->nmod_work), B->nnmod, s);
     if (rc) return rc;
-    rc = fa_batch_crt_poly(1, P, (const uint64_t*)(d + B->fmpz_work), B->nfmpz, s);
+    rc = fa_batch_crt_poly(1, 1, P, (const uint64_t*)(d + B->fmpz_work), B->nfmpz, s);
     if (rc) return rc;
     for (auto& k : B->ks) {
         rc = fa_ks_post_v(k.variant, k.sb, k.an, k.bn, k.scratch, k.z, k.zw, k.zl, k.cnt, s);
@@ -432,6 +433,17 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
     std::map<int, std::vector<uint64_t>> crt_bins;
     std::vector<uint64_t> carry;
     std::vector<uint64_t> nmod_w, fmpz_w;
+    uint64_t nmod_out = 0;
+    for (int64_t r = 0; r < nreq; r++)
+        if (R[r].kind == FA_REQ_NMOD && P[(size_t)r].live && R[r].status == 1)
+            nmod_out += P[(size_t)r].cnt;
+    // From a million outputs on a thread of the nmod CRT takes four.  A smaller
+    // batch does not fill the GPU with one each, and its CRT is a chain of
+    // latencies that three more values would lengthen.  us per batch with one
+    // and with four: 31 outputs 12.6 and 13.0, 999 16.1 and 17.5, 63,984 32.2 and
+    // 33.8, 239,996 35.1 and 36.6 (61-bit n), 1,023,744 43.2 and 42.8 (20-bit),
+    // 68.7 and 69.0 (61-bit), 79 million 4190 and 4100 (20 to 63 bits).
+    B->nmod_k = nmod_out >= (1u << 20) ? 4 : 1;
     for (int64_t r = 0; r < ntot; r++) {
         fa_request& q = req(r);
         plan& p = P[(size_t)r];
@@ -539,7 +551,7 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             }
             prec.push_back(b);
             auto& w = q.kind == FA_REQ_NMOD ? nmod_w : fmpz_w;
-            const uint64_t blk = q.kind == FA_REQ_NMOD ? FA_NMOD_BLK : 256;
+            const uint64_t blk = q.kind == FA_REQ_NMOD ? 256 * (uint64_t)B->nmod_k : 256;
             for (uint64_t c = 0; c < (p.cnt + blk - 1) / blk; c++)
                 w.push_back((uint64_t)pid | (c << 32));
         }

@@ -212,7 +212,6 @@ struct fa_bmpn {               // integer product
 };
 #define FA_CARRY_SEG 16           // CRT workgroups per wave of the carry kernels
 #define FA_CARRY_WG 4             // waves per workgroup of these
-#define FA_NMOD_BLK 1024          // outputs per workgroup of the batched nmod CRT
 struct fa_bpoly {              // nmod or fmpz polynomial product
     const double* Q;           // residue rows; null: the zero product (n = 1)
     uint64_t stride;
@@ -269,7 +268,7 @@ int fa_ks_device(uint64_t* z, uint64_t zw, uint64_t zl, uint64_t cnt, const uint
                  int64_t b1, int64_t b2, uint64_t* scratch, hipStream_t s);
 int fa_fmpz_primes(uint64_t bn, int64_t b1, int64_t b2);
 int64_t fa_vec_max_bits(const uint64_t* v, uint64_t w, int64_t n);
-int fa_batch_crt_poly(int fmpz, const fa_bpoly* P, const uint64_t* work, unsigned nwork,
+int fa_batch_crt_poly(int fmpz, int k, const fa_bpoly* P, const uint64_t* work, unsigned nwork,
                       hipStream_t s);
 // launches of one bin; return FA_OK or an error code
 int fa_batch_small_bin(int depth, int kind, const fa_bjob* J, const uint64_t* work,

@@ -310,17 +310,19 @@ __global__ void __launch_bounds__(256) fa_kb_crt_fmpz(const fa_bpoly* __restrict
 #undef FA_KB_FMPZ
 }
 
-// batched nmod CRT: work item = job | chunk << 32, FA_NMOD_BLK outputs per
-// chunk.  A workgroup goes through five dependent steps (work item, record,
-// constants, p_k mod n, residues) before it computes, so each takes four
-// outputs per thread; the constants are read through the scalar cache.
-// (A batch of about 79 million outputs: 1050 us with one output per thread and
-// every value reduced, 427 now.)  A modulus below 2^64 and a length below 2^40
-// need at most 2^168 < p_0 p_1 p_2 p_3.
+// batched nmod CRT: work item = job | chunk << 32, 256 K outputs per chunk, K
+// per thread.  A workgroup goes through five dependent steps (work item,
+// record, constants, p_k mod n, residues) before it computes, so in a large
+// batch each takes four outputs per thread; the constants are read through the
+// scalar cache.  (A batch of about 79 million outputs: 1050 us with one output
+// per thread and every value reduced, 427 now.)  A modulus below 2^64 and a
+// length below 2^40 need at most 2^168 < p_0 p_1 p_2 p_3.
+template <int K>
 __global__ void __launch_bounds__(256) fa_kb_crt_nmod(const fa_bpoly* __restrict__ P,
                                                       const uint64_t* __restrict__ work,
                                                       unsigned nwork)
 {
+    constexpr uint64_t BLK = 256 * K;
     typedef __attribute__((address_space(4))) const fa_crt_consts cC;
     const unsigned nb = gridDim.x, bid = blockIdx.x;
     const unsigned L = (bid & 7) * (nb >> 3) + (bid >> 3);
@@ -328,18 +330,17 @@ __global__ void __launch_bounds__(256) fa_kb_crt_nmod(const fa_bpoly* __restrict
     const uint64_t w = work[L];
     const fa_bpoly& j = P[(unsigned)(w & 0xffffffffu)];
     __shared__ uint64_t pm[FA_NPRIMES];
-    const uint64_t t0 = (w >> 32) * FA_NMOD_BLK;
+    const uint64_t t0 = (w >> 32) * BLK;
     if (t0 >= j.cnt) return;
-    uint64_t cnt = j.cnt - t0 < FA_NMOD_BLK ? j.cnt - t0 : FA_NMOD_BLK;
+    uint64_t cnt = j.cnt - t0 < BLK ? j.cnt - t0 : BLK;
     const uint64_t j0 = j.zl + t0;
     // the outputs of this chunk below the product's length
     const uint64_t live = !j.Q || j0 >= j.zn ? 0 : j.zn - j0 < cnt ? j.zn - j0 : cnt;
     for (uint64_t t = live + threadIdx.x; t < cnt; t += 256) j.z[t0 + t] = 0;
     if (!live) return;
     cC& C = *(cC*)j.C;
-#define FA_KB_NMOD(NP)                                                                          \
-    fa_crt_nmod_block<NP, FA_NMOD_BLK / 256>(j.Q, j.stride, j0, live, C, j.n, j.dinv, j.norm,   \
-                                             j.z + t0, pm)
+#define FA_KB_NMOD(NP) \
+    fa_crt_nmod_block<NP, K>(j.Q, j.stride, j0, live, C, j.n, j.dinv, j.norm, j.z + t0, pm)
     switch (C.np) {
     case 1: FA_KB_NMOD(1); break;
     case 2: FA_KB_NMOD(2); break;
@@ -349,15 +350,17 @@ __global__ void __launch_bounds__(256) fa_kb_crt_nmod(const fa_bpoly* __restrict
 #undef FA_KB_NMOD
 }
 
-int fa_batch_crt_poly(int fmpz, const fa_bpoly* P, const uint64_t* work, unsigned nwork,
+int fa_batch_crt_poly(int fmpz, int k, const fa_bpoly* P, const uint64_t* work, unsigned nwork,
                       hipStream_t s)
 {
     if (!nwork) return FA_OK;
     const unsigned grid = (nwork + 7) & ~7u;
     if (fmpz)
         FA_LAUNCH("fa_kb_crt_fmpz", fa_kb_crt_fmpz, dim3(grid), dim3(256), 0, s, P, work, nwork);
+    else if (k == 1)
+        FA_LAUNCH("fa_kb_crt_nmod", fa_kb_crt_nmod<1>, dim3(grid), dim3(256), 0, s, P, work, nwork);
     else
-        FA_LAUNCH("fa_kb_crt_nmod", fa_kb_crt_nmod, dim3(grid), dim3(256), 0, s, P, work, nwork);
+        FA_LAUNCH("fa_kb_crt_nmod", fa_kb_crt_nmod<4>, dim3(grid), dim3(256), 0, s, P, work, nwork);
     return hipGetLastError() == hipSuccess ? FA_OK : fa_set_error(FA_E_HIP, "batch crt launch");
 }
 

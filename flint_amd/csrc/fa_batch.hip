@@ -8,7 +8,8 @@
 //     convolution in LDS, binned by (depth, import kind);
 //   - depth 13..24: the column / row / column passes of the two-level
 //     transform, binned by (depth, import kind), every workgroup taking one
-//     (product, prime, operand, tile) item of its bin's work list;
+//     (product, prime, operand, tile) of its bin's work list (an item names a
+//     block of adjacent tiles);
 //   - CRT: integer products binned by prime count (then the carries between
 //     their workgroups, FA_CARRY_SEG per wave), nmod windows in chunks of
 //     256 or 1024 coefficients, fmpz windows in chunks of 256.
@@ -444,6 +445,12 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
     // 33.8, 239,996 35.1 and 36.6 (61-bit n), 1,023,744 43.2 and 42.8 (20-bit),
     // 68.7 and 69.0 (61-bit), 79 million 4190 and 4100 (20 to 63 bits).
     B->nmod_k = nmod_out >= (1u << 20) ? 4 : 1;
+    auto more = [](std::vector<uint64_t>& v, size_t n) {   // room for n more items
+        const size_t k = v.size();
+        if (v.capacity() < k + n) v.reserve(2 * (k + n));
+        v.resize(k + n);
+        return v.data() + k;
+    };
     for (int64_t r = 0; r < ntot; r++) {
         fa_request& q = req(r);
         plan& p = P[(size_t)r];
@@ -495,23 +502,21 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
                 for (int i = 0; i < p.np; i++) w.push_back(FA_WORK(jid, i, 0, 0));
             } else {
                 auto& tb = trans_bins[key];
-                const int ng = fa_batch_col_groups(p.depth);
-                const int nrow = 1 << (p.depth - FA_ROW_LG);
+                int ng;
+                const int gb = fa_batch_col_block(p.depth, &ng);
                 // blocks of adjacent column groups, then the primes (the
                 // order of the single-product kernels)
-                const int gb = fa_batch_col_block(p.depth);
+                uint64_t* w = more(tb.fwd, (size_t)(2 * ng / gb * p.np));
                 for (int z = 0; z < 2; z++)
                     for (int h = 0; h < ng; h += gb)
-                        for (int i = 0; i < p.np; i++)
-                            for (int lo = 0; lo < gb; lo++)
-                                tb.fwd.push_back(FA_WORK(jid, i, z, h + lo));
+                        for (int i = 0; i < p.np; i++) *w++ = FA_WORK(jid, i, z, h);
+                const int rb = fa_batch_row_block(p.depth);
+                w = more(tb.row, (size_t)(p.np * ((j.trows + rb - 1) / rb)));
                 for (int i = 0; i < p.np; i++)
-                    for (int row = 0; row < nrow && row < j.trows; row++)
-                        tb.row.push_back(FA_WORK(jid, i, 0, row));
+                    for (int row = 0; row < j.trows; row += rb) *w++ = FA_WORK(jid, i, 0, row);
+                w = more(tb.inv, (size_t)(ng / gb * p.np));
                 for (int h = 0; h < ng; h += gb)
-                    for (int i = 0; i < p.np; i++)
-                        for (int lo = 0; lo < gb; lo++)
-                            tb.inv.push_back(FA_WORK(jid, i, 0, h + lo));
+                    for (int i = 0; i < p.np; i++) *w++ = FA_WORK(jid, i, 0, h);
             }
         }
         if (q.kind == FA_REQ_MPN) {
@@ -527,7 +532,8 @@ extern "C" int fa_batch_create(fa_batch_s** out, fa_request* R, int64_t nreq, in
             m.np = p.np;
             mrec.push_back(m);
             auto& w = crt_bins[p.np];
-            for (uint64_t blk = 0; blk < p.nblk; blk++) w.push_back((uint64_t)mid | (blk << 32));
+            uint64_t* wb = more(w, (size_t)p.nblk);
+            for (uint64_t blk = 0; blk < p.nblk; blk++) *wb++ = (uint64_t)mid | (blk << 32);
             if (p.nblk > 1)   // one workgroup resolves its own
                 for (uint64_t seg = 0; seg * FA_CARRY_SEG < p.nblk; seg += FA_CARRY_WG)
                     carry.push_back((uint64_t)mid | (seg << 32));

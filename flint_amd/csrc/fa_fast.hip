@@ -1496,15 +1496,31 @@ FA_DEV fa_operand fa_job_operand(const fa_bjob& j, int z)
 template <int D1>
 constexpr int fa_kb_nt() { return D1 == 12 ? 1024 : col_geom<D1>::NT; }
 
+// columns of such a tile, and the adjacent tiles that one work item names by
+// the first of them (a block of the work order, one workgroup per tile)
+template <int D1>
+constexpr unsigned fa_kb_cpw() { return D1 == 12 ? 8 : col_geom<D1>::CPW; }
+// (up to D1 = 4 a block is half of the 4096 columns: items are then as few as
+// the GPU's time allows; 1000 nmod products of 2^14 points 765 us, with blocks
+// of 512 columns 785, 400 of 2^15 points 617 and 615)
+template <int D1>
+constexpr unsigned fa_kb_block()
+{
+    return fa_col_block<fa_kb_cpw<D1>(),
+                        D1 == 12 ? FA_COLW_BLOCK : D1 <= 4 ? 2048 : FA_COL_BLOCK>();
+}
+
 template <int D1, int KIND>
 __global__ void __launch_bounds__(fa_kb_nt<D1>(), 4)
 fa_kb_col_fwd(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, unsigned nwork,
               fa_prime_set S)
 {
     __shared__ double lds[(D1 == 12) ? FA_C8_LDS : col_geom<D1>::LDS];
+    constexpr unsigned GB = fa_kb_block<D1>();
     const unsigned L = fa_xcd_linear();
-    if (L >= nwork) return;
-    const fa_witem w = fa_decode(work[L]);
+    if (L >= nwork * GB) return;
+    fa_witem w = fa_decode(work[L / GB]);
+    w.tile += L % GB;
     const fa_bjob& j = J[w.job];
     const int pi = j.offset + w.prime;
     const fa_operand op = fa_job_operand(j, w.op);
@@ -1523,9 +1539,11 @@ fa_kb_col_inv(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, 
               fa_prime_set S)
 {
     __shared__ double lds[(D1 == 12) ? FA_C8_LDS : fa_col_inv_lds<D1>()];
+    constexpr unsigned GB = fa_kb_block<D1>();
     const unsigned L = fa_xcd_linear();
-    if (L >= nwork) return;
-    const fa_witem w = fa_decode(work[L]);
+    if (L >= nwork * GB) return;
+    fa_witem w = fa_decode(work[L / GB]);
+    w.tile += L % GB;
     const fa_bjob& j = J[w.job];
     const int pi = j.offset + w.prime;
     double* dst = j.A + (uint64_t)w.prime * j.stride;
@@ -1540,17 +1558,18 @@ fa_kb_col_inv(const fa_bjob* __restrict__ J, const uint64_t* __restrict__ work, 
 
 __global__ void __launch_bounds__(256, 4) fa_kb_row_conv(const fa_bjob* __restrict__ J,
                                                          const uint64_t* __restrict__ work,
-                                                         unsigned nwork, fa_prime_set S)
+                                                         unsigned nwork, int lg, fa_prime_set S)
 {
     __shared__ double xch[4352];
     __shared__ double tab[256];
     __shared__ double rho[32];
     const unsigned L = fa_xcd_linear();
-    if (L >= nwork) return;
-    const fa_witem w = fa_decode(work[L]);
+    if (L >> lg >= nwork) return;
+    const fa_witem w = fa_decode(work[L >> lg]);
     const fa_bjob& j = J[w.job];
     const int pi = j.offset + w.prime;
-    const uint64_t r = (uint64_t)w.tile;
+    const uint64_t r = (uint64_t)w.tile + (L & ((1u << lg) - 1));
+    if ((int)r >= j.trows) return;   // the last item of a truncated product
     const uint64_t off = (uint64_t)w.prime * j.stride + r * FA_ROW_PITCH;
     fa_row_conv_tile_lr(j.A + off, j.B + off, r, S.p[pi], S.pinv[pi], j.norm[w.prime], S.w2[pi],
                         S.w2inv[pi], xch, tab, rho);
@@ -1593,31 +1612,29 @@ __global__ void __launch_bounds__(256) fa_kb_small_conv(const fa_bjob* __restric
 
 static unsigned grid8(unsigned n) { return (n + 7) & ~7u; }
 
-static int batch_col_cpw(int depth)
+int fa_batch_col_block(int depth, int* ngroups)
 {
+#define FA_F(D) (*ngroups = 4096 / (int)fa_kb_cpw<D>(), (int)fa_kb_block<D>())
     switch (depth - FA_ROW_LG) {
-    case 1: return col_geom<1>::CPW;
-    case 2: return col_geom<2>::CPW;
-    case 3: return col_geom<3>::CPW;
-    case 4: return col_geom<4>::CPW;
-    case 5: return col_geom<5>::CPW;
-    case 6: return col_geom<6>::CPW;
-    case 7: return col_geom<7>::CPW;
-    case 8: return col_geom<8>::CPW;
-    case 9: return col_geom<9>::CPW;
-    case 10: return col_geom<10>::CPW;
-    case 11: return col_geom<11>::CPW;
-    default: return 8;
+    case 1: return FA_F(1);
+    case 2: return FA_F(2);
+    case 3: return FA_F(3);
+    case 4: return FA_F(4);
+    case 5: return FA_F(5);
+    case 6: return FA_F(6);
+    case 7: return FA_F(7);
+    case 8: return FA_F(8);
+    case 9: return FA_F(9);
+    case 10: return FA_F(10);
+    case 11: return FA_F(11);
+    default: return FA_F(12);
     }
+#undef FA_F
 }
 
-int fa_batch_col_groups(int depth) { return 4096 / batch_col_cpw(depth); }
-
-int fa_batch_col_block(int depth)
-{
-    const int b = (depth == 24 ? FA_COLW_BLOCK : FA_COL_BLOCK) / batch_col_cpw(depth);
-    return b < 2 ? 2 : b;
-}
+// log2 of the adjacent rows of a work item of the row pass
+static constexpr int fa_kb_row_lg(int d1) { return d1 < 3 ? d1 : 3; }
+int fa_batch_row_block(int depth) { return 1 << fa_kb_row_lg(depth - FA_ROW_LG); }
 
 int fa_batch_small_bin(int depth, int kind, const fa_bjob* J, const uint64_t* work,
                        unsigned nwork, const fa_prime_set& S, hipStream_t s)
@@ -1649,14 +1666,14 @@ static void batch_bin(const fa_bjob* J, const uint64_t* wf, unsigned nf, const u
                       hipStream_t s)
 {
     if (nf)
-        FA_LAUNCH("fa_kb_col_fwd", (fa_kb_col_fwd<D1, KIND>), dim3(grid8(nf)),
-                  dim3(fa_kb_nt<D1>()), 0, s, J, wf, nf, S);
+        FA_LAUNCH("fa_kb_col_fwd", (fa_kb_col_fwd<D1, KIND>),
+                  dim3(grid8(nf * fa_kb_block<D1>())), dim3(fa_kb_nt<D1>()), 0, s, J, wf, nf, S);
     if (nr)
-        FA_LAUNCH("fa_kb_row_conv", fa_kb_row_conv, dim3(grid8(nr)), dim3(256), 0, s, J, wr, nr,
-                  S);
+        FA_LAUNCH("fa_kb_row_conv", fa_kb_row_conv, dim3(grid8(nr << fa_kb_row_lg(D1))),
+                  dim3(256), 0, s, J, wr, nr, fa_kb_row_lg(D1), S);
     if (ni)
-        FA_LAUNCH("fa_kb_col_inv", fa_kb_col_inv<D1>, dim3(grid8(ni)),
-                  dim3(fa_kb_nt<D1>()), 0, s, J, wi, ni, S);
+        FA_LAUNCH("fa_kb_col_inv", fa_kb_col_inv<D1>,
+                  dim3(grid8(ni * fa_kb_block<D1>())), dim3(fa_kb_nt<D1>()), 0, s, J, wi, ni, S);
 }
 
 template <int D1>

@@ -277,10 +277,11 @@ int fa_batch_transform_bin(int depth, int kind, const fa_bjob* J, const uint64_t
                            unsigned nfwd, const uint64_t* wrow, unsigned nrow,
                            const uint64_t* winv, unsigned ninv, const fa_prime_set& S,
                            hipStream_t s);
-// column groups per residue array in the batched column passes at depth D
-int fa_batch_col_groups(int depth);
-// adjacent column groups that come before the next prime in a work list
-int fa_batch_col_block(int depth);
+// batched column passes at this depth: the adjacent column groups of a work
+// item, and the groups of a residue array
+int fa_batch_col_block(int depth, int* ngroups);
+// and the adjacent rows of a work item of the row pass
+int fa_batch_row_block(int depth);
 }
 
 // ---------------------------------------------------------------------------

@@ -194,6 +194,7 @@ FA_DEV void ks_sflags_body(const uint64_t* __restrict__ ap, int w, uint64_t n,
     gI* lowg = (gI*)low;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     int negs = 0;
+    int64_t last = -1;     // the top nonzero coefficient: above it, limb 0 tells below
     for (int64_t hi = (int64_t)n; hi > 0; hi -= 1024) {
         const int64_t i = hi - 1024 + t;
         bool nz = false, neg = false;
@@ -212,7 +213,9 @@ FA_DEV void ks_sflags_body(const uint64_t* __restrict__ ap, int w, uint64_t n,
         int found = 0;
         for (int v = 15; v >= 0 && !found; v--) {
             if (sG[v]) {
-                negs = (int)((sP[v] >> (63 - __builtin_clzll(sG[v]))) & 1);
+                const int b = 63 - __builtin_clzll(sG[v]);
+                negs = (int)((sP[v] >> b) & 1);
+                last = hi - 1024 + 64 * v + b;
                 found = 1;
             }
         }
@@ -236,7 +239,7 @@ FA_DEV void ks_sflags_body(const uint64_t* __restrict__ ap, int w, uint64_t n,
         for (int k = 0; k < 4; k++) {
             const uint64_t i = base + 1024 * k + t;
             const bool in = i < n;
-            l[k] = ks_low_limb(a + (in ? i : n - 1) * (uint64_t)w, w, v0[k]);
+            l[k] = ks_low_limb(a + (in ? i : n - 1) * (uint64_t)w, (int64_t)i <= last ? w : 1, v0[k]);
             // generate [sigma c < 0], propagate [c = 0]
             G[k] = __ballot(in && l[k] != KS_ZERO && (int)(vt[k] >> 63) != negs);
             P[k] = __ballot(in && l[k] == KS_ZERO);

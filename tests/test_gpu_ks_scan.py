@@ -3,7 +3,10 @@ can go wrong: lengths around a wave, 1024 and a round of 4096 coefficients,
 runs of zero coefficients that carry a borrow across waves and rounds, the top
 coefficient far below the end, all-zero operands, slots just below, at and
 above 64 bits, coefficients of the largest magnitude.  The expected words are
-those of the exact product, by substitution into Python integers."""
+those of the exact product, by substitution into Python integers.  And the time
+on an operand that is zero above its first coefficient."""
+import time
+
 import numpy as np
 import pytest
 
@@ -53,3 +56,34 @@ def test_flags_and_packing(an, abits, bbits, pattern):
     lo = zn - zn // 3
     z = fa.fmpz_poly_mul_ks(enc(a, aw), aw, enc(b, bw), bw, lo, zn, zw)
     assert dec(z, zw) == want[lo:]
+
+
+def test_time_of_leading_zeros():
+    """the flags of an operand whose coefficients above the first are zero: each
+    zero coefficient's limbs are read once, so the product takes what one with
+    only top limbs set takes (1.28 times that with two walks)"""
+    import torch
+    import flint_amd as fa
+    n, bits = 9000, 3900
+    w, zw = bits // 64 + 1, (2 * bits + 64) // 64 + 1
+    z = torch.empty((2 * n - 1) * zw, dtype=torch.int64, device="cuda")
+    t = []
+    for top in (True, False):
+        a = torch.zeros((n, w), dtype=torch.int64, device="cuda")
+        if top:
+            a[:, -1] = 1
+        else:
+            a[0, 0] = 5
+        torch.cuda.synchronize()
+        best = 1e9
+        for _ in range(12):
+            s = time.perf_counter()
+            for _ in range(3):
+                assert fa.lib().fa_fmpz_poly_mul_mid_device(
+                    z.data_ptr(), zw, 0, 2 * n - 1, a.data_ptr(), w, n, a.data_ptr(), w, n, -bits,
+                    -bits, 1, None) == 1
+            fa.lib().fa_sync()
+            best = min(best, (time.perf_counter() - s) / 3)
+        t.append(best)
+    print("us", [round(1e6 * x) for x in t], flush=True)
+    assert t[1] < 1.15 * t[0]

@@ -1,6 +1,7 @@
 // fa_fast.hip -- register radix-16 kernels for the two-level transforms with
 // a 4096-point row (d2 = 12) and a column of 2^d1 points, d1 = 1..12, i.e.
-// transform lengths 2^13 .. 2^24.
+// transform lengths 2^13 .. 2^24, and with rows of 256 or 1024 points for
+// single products of 2^11 .. 2^19 points ("Short rows" below).
 //
 // A 2^(4s)-point transform is s stages of radix 16: each thread holds 16
 // elements in registers and applies four levels (two radix-4 butterflies,
@@ -638,15 +639,15 @@ __global__ void __launch_bounds__(256) fa_k_row_conv16(double* __restrict__ A,
 
 // A tile is CPW columns of NT threads together: 256 threads up to D1 = 8, so
 // that four tiles of at most 34.8 KB of LDS share a CU and one's loads and
-// stores run beside another's arithmetic, and a product of 2^13..2^20 points
-// gives four times the workgroups of a 1024-thread tile.  CPW never falls
-// below 16 columns (a 128-byte line) there; D1 = 9 keeps 16 with 512 threads,
-// D1 = 10 takes 8 (two tiles per CU), D1 = 11 eight with 1024 threads.
-// Measured against 1024-thread tiles whose import tested every chunk: the
-// column passes of a 65,536-limb square (2^17 points) 13.3 + 8.6 -> 7.8 +
-// 5.1 us; 64 batched fmpz products, 2^20 points, 913 + 389 -> 761 + 346 us (a
-// copy's rate, 5.3 TB/s, in the inverse pass; the forward pass waits on the
-// reads of its limb rows, without which it takes 363 us).
+// stores run beside another's arithmetic, and a product of 2^20 points gives
+// four times the workgroups of a 1024-thread tile.  CPW never falls below 16
+// columns (a 128-byte line) there; D1 = 9 keeps 16 with 512 threads, D1 = 10
+// takes 8 (two tiles per CU), D1 = 11 eight with 1024 threads.
+// Measured against 1024-thread tiles whose import tested every chunk: 64
+// batched fmpz products, 2^20 points, 913 + 389 -> 761 + 346 us (a copy's rate,
+// 5.3 TB/s, in the inverse pass; the forward pass waits on the reads of its
+// limb rows, without which it takes 363 us); the column passes of 2^17 points,
+// three primes, with rows of 4096, 13.3 + 8.6 -> 7.8 + 5.1 us.
 //
 // D2 < 12: shorter rows (the short-row path below).  A tile is then at least
 // one wave, 16 columns wide where that is more.
@@ -1034,16 +1035,17 @@ FA_DEV void fa_col_inv_tile(double* __restrict__ dst, int g, double n, double ni
     for (int k = 0; k < G::NEL; k++) fa_st(dst + fa_row_off<D2>(k * rs), out, x[k]);
 }
 
-// Work order of the column passes: blocks of `lines` adjacent column groups
-// (512 columns), for each block the primes, then the next block, then the
-// other operand.  Concurrent workgroups of an XCD then read long runs of each
-// limb row (row starts are own * 4096 bytes apart, so a narrow block of
-// columns would fall on few HBM channels), and the primes of a block find its
-// limbs in L2.  64 batched fmpz products, 2^20 points, forward: 1015 us with
-// blocks of 64 columns, 906 with 512, 928 with 1024, 954 with all 4096.  At
-// 2^24 points one tile fills a CU and the limb rows of a block no longer fit
-// L2 beside the tiles, so the blocks there are 64 columns (the whole product
-// 2.33 ms; 2.48 with 512).
+// Work order of the column passes: blocks of adjacent column groups (512
+// columns), for each block the primes, then the next block, then the other
+// operand.  Concurrent workgroups of an XCD then read long runs of each limb
+// row (row starts are own * 4096 bytes apart, so a narrow block of columns
+// would fall on few HBM channels), and the primes of a block find its limbs in
+// L2.  64 batched fmpz products, 2^20 points, forward: 1015 us with blocks of
+// 64 columns, 906 with 512, 928 with 1024, 954 with all 4096.
+// At 2^24 points one tile fills a CU, and a wider block asks more of L2 beside
+// the tiles: the forward pass of 2^24 x 2^24 limbs takes 826 us and reads 426
+// MB with blocks of 16 columns, 765 us and 690 MB with 64, 914 us and 1670 MB
+// with 512 (268 MB of limbs).  64 is the faster order although it reads more.
 #define FA_COL_BLOCK 512
 #define FA_COLW_BLOCK 64
 template <int CPW, int BLOCK>
@@ -1976,13 +1978,23 @@ static int launch_forward_any(const fa_operand& oa, int np, double* A, uint64_t 
     }
 }
 
-// Single products of 2^11 .. 2^18 points take short rows.  Whole products, the
-// other path and this one, us: 2^11 points 21.9 and 20.4 (one workgroup per
-// prime in LDS; at 2^10 that path is level, 19.5), 2^12 32.1 and 20.5, 2^14
-// 25.1 and 20.7, 2^16 31.1 and 26.3, 2^17 39.3 and 35.3 (products mod a 61-bit
-// n); 2^18 63.8 and 58.8 (integers); 2^19 57.6 and 52.4 modulo three primes,
-// but 104 and 110 modulo seven, where 896 rows of 4096 fill the GPU.  The lengths of the rows are the faster ones: at 2^16 and 2^17
-// points 1024 (26.4, 35.3) against 256 (29.7, 37.8).
+// Single products of 2^11 .. 2^18 points, and of 2^19 modulo at most three
+// primes, take short rows.  Whole products of integers, us, with the path for
+// other sizes (up to 2^12 points one workgroup per prime in LDS, above rows of
+// 4096), rows of 256 and rows of 1024:
+//            np = 2             np = 4             np = 8
+//   2^10  17.7  17.9    -    19.1  19.0    -    22.3  21.7    -
+//   2^11  24.9  18.1  19.6   26.4  19.1  20.7   30.1  22.2  23.6
+//   2^13  26.9  19.1  20.1   28.1  21.0  21.3   31.2  24.6  24.1
+//   2^15  27.8  24.3  24.7   29.3  25.8  26.8   34.2  31.1  30.8
+//   2^16  29.9  26.5  25.8   33.2  29.0  29.1   40.0  36.4  36.9
+//   2^17  33.7  31.7  27.6   38.3  37.1  33.4   52.5  49.1  46.9
+//   2^18  37.5    -   33.9   49.1    -   44.5   69.0    -   60.3
+// so rows of 256 up to 2^15 points and of 1024 from 2^16.  2^19 points with
+// rows of 4096 and of 1024, np = 2 to 8: 49.1 and 47.3, 61.9 and 56.3, 67.1
+// and 60.5, 75.0 and 73.6, 80.9 and 82.6, 92.9 and 96.2, 99.7 and 104.9.
+// (Products mod n of one prime, 2^11 points: 20.7 and 16.0, but level, 21.6 and
+// 22.6, where a slow host takes 5.5 us per launch.)
 #define FA_SHORT_MAX 19
 #define FA_SHORT_MIN 11
 
@@ -2057,22 +2069,25 @@ static int fa_short(int depth, int what, const fa_operand& oa, const fa_operand&
     }
 }
 
-#define FA_D1_SWITCH(d1, F)                                                                \
-    switch (d1) {                                                                          \
-    case 1: return F(1); case 2: return F(2); case 3: return F(3); case 4: return F(4);    \
-    case 5: return F(5); case 6: return F(6); case 7: return F(7); case 8: return F(8);    \
-    case 9: return F(9); case 10: return F(10); case 11: return F(11);                     \
-    case 12: return F(12);                                                                 \
-    default: return 0;                                                                     \
-    }
+// Transforms on their own: 1 when launched (2^11..2^24 points), 0 for other
+// lengths.  All of 2^11..2^18 points take short rows.
+#define FA_D1_CASES(F)        \
+    case 7: return F(7);      \
+    case 8: return F(8);      \
+    case 9: return F(9);      \
+    case 10: return F(10);    \
+    case 11: return F(11);    \
+    case 12: return F(12);
 
-// depth 13..24: returns 1 when launched, 0 for other depths
 int fa_forward_fast(int depth, const fa_operand& oa, int np, double* A, uint64_t stride,
                     const fa_prime_set& S, hipStream_t s)
 {
     if (fa_short(depth, 2, oa, oa, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_forward_any<D>(oa, np, A, stride, S, s)
-    FA_D1_SWITCH(depth - FA_ROW_LG, FA_F)
+    switch (depth - FA_ROW_LG) {
+    FA_D1_CASES(FA_F)
+    default: return 0;
+    }
 #undef FA_F
 }
 
@@ -2081,7 +2096,10 @@ int fa_inverse_fast(int depth, int np, double* A, uint64_t stride, const fa_prim
 {
     if (fa_short(depth, 3, fa_operand{}, fa_operand{}, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_inverse<D>(np, A, stride, S, s)
-    FA_D1_SWITCH(depth - FA_ROW_LG, FA_F)
+    switch (depth - FA_ROW_LG) {
+    FA_D1_CASES(FA_F)
+    default: return 0;
+    }
 #undef FA_F
 }
 
@@ -2104,6 +2122,16 @@ int fa_convolve_fast(int depth, const fa_operand& oa, const fa_operand& ob, int 
         fa_short(depth, sqr ? 1 : 0, oa, ob, np, A, B, stride, S, s))
         return 1;
 #define FA_F(D) launch_fast_any<D>(oa, ob, nops, np, A, B, stride, S, s, trows)
-    FA_D1_SWITCH(d1, FA_F)
+    // columns below 2^7 points only with fewer rows (fa_set_truncation(2))
+    switch (d1) {
+    case 1: return FA_F(1);
+    case 2: return FA_F(2);
+    case 3: return FA_F(3);
+    case 4: return FA_F(4);
+    case 5: return FA_F(5);
+    case 6: return FA_F(6);
+    FA_D1_CASES(FA_F)
+    default: return 0;
+    }
 #undef FA_F
 }

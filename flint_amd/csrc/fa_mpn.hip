@@ -1440,7 +1440,7 @@ static int mpn_mul_device(uint64_t* z, const uint64_t* a, uint64_t an, const uin
 }
 
 // CRT of zlen coefficients of `bits`-bit chunks into z[0, zn) (the low zn
-// limbs of the sum; zeros above it), carry flags in the thread's scratch
+// limbs of the sum; zeros above it), carry aggregates in the thread's scratch
 int fa_crt_mpn_export(int np, const double* A, uint64_t stride, uint64_t zlen, int bits,
                       uint64_t* z, uint64_t zn, hipStream_t stream, int mode, uint64_t jlo)
 {
@@ -1450,9 +1450,8 @@ int fa_crt_mpn_export(int np, const double* A, uint64_t stride, uint64_t zlen, i
     const uint64_t own = (uint64_t)bits / 8;
     const uint64_t ngroups = (zn + own - 1) / own;
     const uint64_t nblk16 = (ngroups + (FA_CRT16_GROUPS - 2)) / (FA_CRT16_GROUPS - 1);
-    const size_t bytes = ((ngroups + 7) & ~(size_t)7) + 2 * (nblk16 + 8) + 4096;
     void* buf;
-    int rc = fa_scratch_reserve(st, bytes, &buf, stream);
+    int rc = fa_scratch_reserve(st, nblk16, &buf, stream);
     if (rc) return rc;
     uint8_t* agg = (uint8_t*)buf;
     fa_crt_consts C;

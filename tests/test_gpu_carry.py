@@ -1,6 +1,9 @@
-"""Carries between CRT workgroups in products with long runs of ones, where a
-block of ones receives a carry: words against the closed form or the oracle, and
-the time against random operands of the same lengths, single and batched."""
+"""The CRT of integer products at every chunk width a plan may have (a
+coefficient spans up to seven chunks), and the carries between its workgroups in
+products with long runs of ones, where a block of ones receives a carry: words
+against the closed form or the oracle, and the time against random operands of
+the same lengths, single and batched."""
+import math
 import time
 
 import numpy as np
@@ -31,6 +34,29 @@ def test_ones(n, m):
     print(n, m, fa.mpn_plan(n, m), flush=True)
     a = np.full(n, ONES, dtype=np.uint64)
     assert np.array_equal(fa.mpn_mul(a, a[:m]), closed_form(n, m))
+
+
+@pytest.mark.parametrize("np_", range(2, 9))
+def test_chunk_widths(np_):
+    """all widths from the smallest (24 bits for two primes, 64 for eight) to the
+    largest that is exact, random limbs and ones, a few blocks and part of one"""
+    import flint_amd as fa
+    rng = np.random.default_rng(np_)
+    M = math.prod(int(p) for p in O.default_primes()[:np_])
+    tried = 0
+    for bits in range(24, 25 * np_ + 1, 8):
+        if 9 * bits < 64 * -(-M.bit_length() // 64) + 64:
+            continue
+        for an, bn in ((40 * bits // 8 + 3, 23 * bits // 8), (31, 9)):
+            if -(-64 * bn // bits) << 2 * bits > M:
+                continue
+            for a, b in ((rng.integers(0, 2**64, an, dtype=np.uint64),
+                          rng.integers(0, 2**64, bn, dtype=np.uint64)),
+                         (np.full(an, ONES), np.full(bn, ONES))):
+                print(np_, bits, an, bn, flush=True)
+                assert np.array_equal(fa.mpn_mul_plan(a, b, np_, bits), O.mpn_mul(a, b)), (bits, an)
+                tried += 1
+    assert tried >= 4 * (25 * np_ - 24) // 16
 
 
 def runs(rng, n):

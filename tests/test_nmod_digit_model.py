@@ -1,14 +1,45 @@
-"""CPU model of the reductions that the nmod CRT of flint_amd/csrc/fa_poly.hip
-keeps (fa_crt_nmod_value): the double operations replayed exactly, with every
-mulmod's operands below 4 p^2, every running value within the bounds stated at
-the kernel, every digit in [0, p), and the result equal to c mod n, for stored
-residues anywhere in [-8p, 8p] and c at its extremes."""
+"""CPU model of the nmod CRT of flint_amd/csrc/fa_poly.hip (fa_crt_nmod_value).
+
+The kernel finds the mixed-radix digits t_k of the coefficient c in [0, M) with
+FP64 mulmods (h = a b, q = rint(h / p), r = fma(-q, p, h) + fma(a, b, -h)) and
+the reductions that their bounds need, then c mod n by Horner's rule with
+128-bit products.  The double operations are replayed exactly (FMA through
+rationals, rint half-even), with every mulmod's operands below 4 p^2, every
+running value within the bounds stated at the kernel, every digit in [0, p), the
+high word below n at every 128-bit reduction, and the result equal to c mod n:
+for every prime count 1..8 at every offset into the eight default primes, stored
+residues anywhere in [-8p, 8p], c at its extremes and of any length, and moduli
+n from 1 to 2^64 - 59."""
 import random
+from fractions import Fraction
 
 import pytest
 
 from oracle import oracle as O
-from tests.test_nmod_garner_model import _consts, _fma, _pm1n
+
+
+def _fma(a, b, c):
+    return float(Fraction(a) * Fraction(b) + Fraction(c))
+
+
+def _pm1n(a, p, pinv):
+    return _fma(-float(round(a * pinv)), p, a)
+
+
+def _consts(primes):
+    M = 1
+    for p in primes:
+        M *= p
+    gcm = [(M // p) % p for p in primes]
+    ginv, gpm = [], []
+    for k, pk in enumerate(primes):
+        pre, row = 1 % pk, []
+        for j in range(k):
+            row.append(primes[j] % pk)
+            pre = pre * (primes[j] % pk) % pk
+        gpm.append(row)
+        ginv.append(pow(pre, pk - 2, pk))
+    return M, gcm, ginv, gpm
 
 
 def _mulmod(a, b, p, pinv):
@@ -51,10 +82,12 @@ def test_digits_exact(np_):
             M *= p
         for trial in range(60):
             c = (rnd.randrange(M), M - 1 - rnd.randrange(1000), rnd.randrange(1000),
-                 M // 2 + rnd.randrange(-5, 5))[trial % 4]
+                 M // 2 + rnd.randrange(-5, 5),
+                 rnd.randrange(1 << rnd.randint(1, M.bit_length() - 1)))[trial % 5]
             xs = [c * pow((M // p) % p, p - 2, p) % p + p * rnd.randrange(-8, 8) for p in primes]
             t = digits(xs, primes)
-            n = rnd.choice([1, 2, (1 << 64) - 59, (1 << 63) + 29, rnd.randrange(2, 1 << 64)])
+            n = rnd.choice([1, 2, 3, (1 << 64) - 59, (1 << 63) + 29, rnd.randrange(2, 1 << 64),
+                            rnd.randrange(2, 1 << 20)])
             v = t[-1] if np_ > 1 else t[-1] % n
             for k in range(np_ - 2, -1, -1):
                 w = v * (primes[k] % n) + t[k]

@@ -84,8 +84,7 @@ int inv_series_dev(uint64_t* g, const uint64_t* f, uint64_t fn, uint64_t m, fa_n
                    uint64_t* e, uint64_t* t, hipStream_t s)
 {
     uint64_t f0;
-    if (hipMemcpyAsync(&f0, f, 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    if (fa_download(&f0, f, 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "divrem: reading the constant term failed");
     const uint64_t g0 = invmod(f0, mod.n);
     if (!g0 && mod.n != 1)
@@ -165,8 +164,7 @@ extern "C" int fa_nmod_poly_inv_series(uint64_t* g, const uint64_t* f, int64_t f
         return fa_set_error(FA_E_HIP, "upload failed");
     rc = inv_series_dev(dg.p, df.p, (uint64_t)fn, (uint64_t)m, mod, e.p, t.p, s);
     if (rc) return rc;
-    if (hipMemcpyAsync(g, dg.p, (uint64_t)m * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    if (fa_download(g, dg.p, (uint64_t)m * 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return FA_OK;
 }
@@ -194,9 +192,8 @@ extern "C" int fa_nmod_poly_divrem(uint64_t* q, uint64_t* r, const uint64_t* a, 
     if (rc) return rc;
     rc = divrem_dev(dq.p, dr.p, da.p, (uint64_t)an, db.p, (uint64_t)bn, dB.p, Bn, mod, dp.p, s);
     if (rc) return rc;
-    if (hipMemcpyAsync(q, dq.p, qn * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipMemcpyAsync(r, dr.p, (uint64_t)(bn - 1) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    if (fa_download(q, dq.p, qn * 8, s) != hipSuccess ||
+        fa_download(r, dr.p, (uint64_t)(bn - 1) * 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return FA_OK;
 }
@@ -276,9 +273,8 @@ extern "C" int fa_nmod_poly_divrem_precomp(uint64_t* q, uint64_t* r, const uint6
     rc = divrem_dev(dq.p, dr.p, da.p, (uint64_t)an, M->b, M->bn, M->B + (M->Bn - qn), qn, mod,
                     dp.p, s);
     if (rc) return rc;
-    if (hipMemcpyAsync(q, dq.p, qn * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipMemcpyAsync(r, dr.p, (M->bn - 1) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    if (fa_download(q, dq.p, qn * 8, s) != hipSuccess ||
+        fa_download(r, dr.p, (M->bn - 1) * 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return 1;
 }

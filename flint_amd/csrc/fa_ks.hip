@@ -797,7 +797,7 @@ extern "C" int fa_fmpz_poly_mul_ks(uint64_t* z, uint64_t zw, int64_t zl, int64_t
     if (!rc)
         rc = fa_ks_device(dz, zw, (uint64_t)zl, cnt, da, aw, (uint64_t)an, db, bw, (uint64_t)bn,
                           b1, b2, dw, s);
-    if (!rc && hipMemcpyAsync(z, dz, wz * 8, hipMemcpyDeviceToHost, s) != hipSuccess)
+    if (!rc && fa_download(z, dz, wz * 8, s) != hipSuccess)
         rc = fa_set_error(FA_E_HIP, "fa_fmpz_poly_mul_ks: download");
     if (hipStreamSynchronize(s) != hipSuccess && !rc)
         rc = fa_set_error(FA_E_HIP, "fa_fmpz_poly_mul_ks: %s", hipGetErrorString(hipGetLastError()));

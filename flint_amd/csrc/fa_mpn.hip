@@ -1597,10 +1597,8 @@ static int mpn_mul_host(uint64_t* z, const uint64_t* a, int64_t an, const uint64
         (void)hipStreamSynchronize(st->stream);
         return rc;
     }
-    if (hipMemcpyAsync(z, dz, zn * sizeof(uint64_t), hipMemcpyDeviceToHost, st->stream) != hipSuccess)
-        return fa_set_error(FA_E_HIP, "product download failed");
-    if (hipStreamSynchronize(st->stream) != hipSuccess)
-        return fa_set_error(FA_E_HIP, "stream synchronize failed: %s",
+    if (fa_download(z, dz, zn * sizeof(uint64_t), st->stream) != hipSuccess)
+        return fa_set_error(FA_E_HIP, "product download failed: %s",
                             hipGetErrorString(hipGetLastError()));
     return FA_OK;
 }
@@ -1852,8 +1850,7 @@ extern "C" int fa_mpn_mulmod_2expp1(uint64_t* z, const uint64_t* x, const uint64
         (void)hipStreamSynchronize(st->stream);
         return rc;
     }
-    if (hipMemcpyAsync(z, dz, m * 8, hipMemcpyDeviceToHost, st->stream) != hipSuccess ||
-        hipStreamSynchronize(st->stream) != hipSuccess)
+    if (fa_download(z, dz, m * 8, st->stream) != hipSuccess)
         return fa_set_error(FA_E_HIP, "result download failed");
     return FA_OK;
 }
@@ -1922,11 +1919,8 @@ extern "C" int fa_mpn_mul_range_host(uint64_t* z, uint64_t lo, uint64_t hi, cons
         (void)hipStreamSynchronize(st->stream);
         return rc;
     }
-    if (hipMemcpyAsync(z, dz + lo, (hi - lo) * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                       st->stream) != hipSuccess)
-        return fa_set_error(FA_E_HIP, "window download failed");
-    if (hipStreamSynchronize(st->stream) != hipSuccess)
-        return fa_set_error(FA_E_HIP, "stream synchronize failed: %s",
+    if (fa_download(z, dz + lo, (hi - lo) * sizeof(uint64_t), st->stream) != hipSuccess)
+        return fa_set_error(FA_E_HIP, "window download failed: %s",
                             hipGetErrorString(hipGetLastError()));
     return FA_OK;
 }

@@ -672,8 +672,7 @@ static int poly_mul_blocked(int fmpz, uint64_t* z, uint64_t zw, int64_t zl, int6
             HIPTRY(hipGetLastError(), "block launch");
         }
     }
-    HIPTRY(hipMemcpyAsync(z, dz, cnt * zwords * 8, hipMemcpyDeviceToHost, s), "download");
-    HIPTRY(hipStreamSynchronize(s), "synchronize");
+    HIPTRY(fa_download(z, dz, cnt * zwords * 8, s), "download");
     return FA_OK;
 }
 
@@ -747,8 +746,7 @@ extern "C" int fa_nmod_poly_mul_mid(uint64_t* z, int64_t zl, int64_t zh, const u
 #undef FA_L
     HIPTRY(hipGetLastError(), "crt launch");
     if (D.lock.owns_lock()) D.lock.unlock();     // the tables' last reader is enqueued
-    HIPTRY(hipMemcpyAsync(z, dz, cnt * sizeof(uint64_t), hipMemcpyDeviceToHost, s), "download");
-    HIPTRY(hipStreamSynchronize(s), "synchronize");
+    HIPTRY(fa_download(z, dz, cnt * sizeof(uint64_t), s), "download");
     return FA_OK;
 }
 
@@ -1049,8 +1047,6 @@ extern "C" int fa_fmpz_poly_mul_mid(uint64_t* z, uint64_t zw, int64_t zl, int64_
     FA_CRT_NL_SWITCH(fa_crt_poly_limbs(C), FA_L)
 #undef FA_L
     HIPTRY(hipGetLastError(), "crt launch");
-    HIPTRY(hipMemcpyAsync(z, dz, cnt * zw * sizeof(uint64_t), hipMemcpyDeviceToHost, s),
-           "download");
-    HIPTRY(hipStreamSynchronize(s), "synchronize");
+    HIPTRY(fa_download(z, dz, cnt * zw * sizeof(uint64_t), s), "download");
     return 1;
 }

@@ -139,8 +139,7 @@ extern "C" int fa_nmod_poly_mulmid_repack(uint64_t* z, const uint64_t* a, int64_
     hipLaunchKernelGGL(k_unpack, dim3(blocks(cnt)), dim3(256), 0, s, dz, pz, znlo, zn, znlo2, zn2,
                        lgM, n);
     if (hipGetLastError() != hipSuccess) return fa_set_error(FA_E_HIP, "repack launch");
-    if (hipMemcpyAsync(z, dz, cnt * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    if (fa_download(z, dz, cnt * 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "repack: download failed");
     return 1;
 }

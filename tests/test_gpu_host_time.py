@@ -1,0 +1,70 @@
+"""Calls on host memory that run more than a few kernels: what a middle product
+with a kept transform takes against the same product without one, and an integer
+product of 2^11 points against a polynomial one; and that the output is complete
+on return, in pageable and in pinned memory."""
+import time
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _time(f):
+    for _ in range(5):
+        f()
+    best = 1e9
+    for _ in range(9):
+        t = time.perf_counter()
+        for _ in range(30):
+            f()
+        best = min(best, (time.perf_counter() - t) / 30)
+    print("%.1f us" % (1e6 * best), flush=True)
+    return best
+
+
+@pytest.mark.parametrize("an", [700, 1500])
+def test_kept_transform(an):
+    """one upload, six kernels, one download against two, four and one (1.4 and
+    1.6 times while the wait for more than eight commands went through a
+    callback)"""
+    import flint_amd as fa
+    rng = np.random.default_rng(an)
+    n = (1 << 61) - 1
+    a, b = (rng.integers(0, n, an, dtype=np.uint64) for _ in range(2))
+    M = fa.MulPrecomp(b, (2 * an).bit_length(), n)
+    want = fa.nmod_poly_mul_mid(a, b, 0, 2 * an - 1, n)
+    assert np.array_equal(M.mul_mid(a, 0, 2 * an - 1), want)
+    t = [_time(lambda: fa.nmod_poly_mul_mid(a, b, 0, 2 * an - 1, n)),
+         _time(lambda: M.mul_mid(a, 0, 2 * an - 1))]
+    M.close()
+    assert t[1] < 1.2 * t[0]
+
+
+def test_integer_product():
+    """two uploads, five kernels, one download against the same with four (1.35
+    times)"""
+    import flint_amd as fa
+    rng = np.random.default_rng(1)
+    n = (1 << 61) - 1
+    a, b = (rng.integers(0, n, 1000, dtype=np.uint64) for _ in range(2))
+    t = [_time(lambda: fa.nmod_poly_mul_mid(a, b, 0, 1999, n)), _time(lambda: fa.mpn_mul(a, b))]
+    assert t[1] < 1.2 * t[0]
+
+
+@pytest.mark.parametrize("an,bn", [(1, 1), (1000, 1005), (60000, 50000), (700000, 500000)])
+def test_complete_on_return(an, bn):
+    import torch
+    import flint_amd as fa
+    rng = np.random.default_rng(an)
+    pin = torch.zeros(an + bn, dtype=torch.int64, pin_memory=True).numpy().view(np.uint64)
+    page = np.zeros(an + bn, dtype=np.uint64)
+    for k in range(3):
+        a, b = (rng.integers(0, 2**64, n, dtype=np.uint64) for n in (an, bn))
+        want = O.mpn_mul(a, b)
+        for z in (pin, page):
+            z[:] = 0
+            assert fa.lib().fa_mpn_mul(fa._p(z), fa._p(a), an, fa._p(b), bn) == 0
+            assert np.array_equal(z, want)

@@ -477,6 +477,10 @@ int fa_buffers_leave(fa_thread_state* st, hipStream_t s)
     return FA_OK;
 }
 
+// in place of fa_buffers_leave where the call has waited for its own stream: it
+// was the last use, and the ones before it were waited for on entry
+void fa_buffers_idle(fa_thread_state* st) { st->last_stream = NULL; }
+
 // a copy to host memory behind the work of s, complete on return.  A stream
 // synchronization makes the runtime wait for a stream with more than eight
 // commands (uploads, kernels, the copy) by a callback on another thread, 20 to

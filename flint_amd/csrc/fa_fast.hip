@@ -2069,8 +2069,13 @@ static int fa_short(int depth, int what, const fa_operand& oa, const fa_operand&
     }
 }
 
-// Transforms on their own: 1 when launched (2^11..2^24 points), 0 for other
-// lengths.  All of 2^11..2^18 points take short rows.
+// Transforms on their own: 1 when launched (2^12..2^24 points), 0 for other
+// lengths.  Up to 2^18 points they take short rows, but not at 2^11: two kernels
+// for one (8 us) make a chain of forward transform, product, inverse and export
+// eight commands, and the runtime waits for more than eight, with its own, by a
+// callback.  That chain, queued behind others and waited for, us, 1019 limbs: one
+// kernel per transform 28.5 and 34, two 26.1 and 51 to 62; 2^12 points, 2043
+// limbs: 36 and 43, 25.8 and 50 to 63.
 #define FA_D1_CASES(F)        \
     case 7: return F(7);      \
     case 8: return F(8);      \
@@ -2082,7 +2087,7 @@ static int fa_short(int depth, int what, const fa_operand& oa, const fa_operand&
 int fa_forward_fast(int depth, const fa_operand& oa, int np, double* A, uint64_t stride,
                     const fa_prime_set& S, hipStream_t s)
 {
-    if (fa_short(depth, 2, oa, oa, np, A, A, stride, S, s)) return 1;
+    if (depth > FA_SHORT_MIN && fa_short(depth, 2, oa, oa, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_forward_any<D>(oa, np, A, stride, S, s)
     switch (depth - FA_ROW_LG) {
     FA_D1_CASES(FA_F)
@@ -2094,7 +2099,7 @@ int fa_forward_fast(int depth, const fa_operand& oa, int np, double* A, uint64_t
 int fa_inverse_fast(int depth, int np, double* A, uint64_t stride, const fa_prime_set& S,
                     hipStream_t s)
 {
-    if (fa_short(depth, 3, fa_operand{}, fa_operand{}, np, A, A, stride, S, s)) return 1;
+    if (depth > FA_SHORT_MIN && fa_short(depth, 3, fa_operand{}, fa_operand{}, np, A, A, stride, S, s)) return 1;
 #define FA_F(D) launch_inverse<D>(np, A, stride, S, s)
     switch (depth - FA_ROW_LG) {
     FA_D1_CASES(FA_F)

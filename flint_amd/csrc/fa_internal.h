@@ -124,6 +124,7 @@ fa_thread_state* fa_state_swap(fa_thread_state* st);
 // of a call on stream s, leave after its last
 int fa_buffers_enter(fa_thread_state* st, hipStream_t s);
 int fa_buffers_leave(fa_thread_state* st, hipStream_t s);
+void fa_buffers_idle(fa_thread_state* st);
 hipError_t fa_download(void* host, const void* dev, size_t bytes, hipStream_t s);
 // grow-only buffers of a state; s = the stream the caller uses them on
 // (null: the state's own), which first waits for a call on another stream

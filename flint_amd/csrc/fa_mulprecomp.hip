@@ -175,6 +175,6 @@ extern "C" int fa_nmod_poly_mul_mid_precomp(uint64_t* z, uint64_t zl, uint64_t z
     }
     if (fa_download(z, dz, (zh - zl) * 8, s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "fa_nmod_poly_mul_mid_precomp: download failed");
-    rc = fa_buffers_leave(st, s);
-    return rc ? rc : 1;
+    fa_buffers_idle(st);
+    return 1;
 }

@@ -68,3 +68,32 @@ def test_complete_on_return(an, bn):
             z[:] = 0
             assert fa.lib().fa_mpn_mul(fa._p(z), fa._p(a), an, fa._p(b), bn) == 0
             assert np.array_equal(z, want)
+
+
+def test_transform_chain():
+    """forward transform, product with a kept one, inverse, export, 2^11 points,
+    waited for: against the whole product of the same operands (1.3 times; 2 with
+    two kernels per transform)"""
+    import torch
+    import flint_amd as fa
+    n = 1019
+    x, y = (torch.randint(-2**63, 2**63 - 1, (n,), device="cuda") for _ in range(2))
+    z = torch.zeros(2 * n + 1, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    P = fa.Plan.mpn(n, n, 1)
+    assert P.s.depth == 11
+    X, Y, Z = (fa.Op(P) for _ in range(3))
+    Y.fft_mpn(y.data_ptr(), n)
+
+    def chain():
+        X.fft_mpn(x.data_ptr(), n)
+        Z.mul(X, Y)
+        Z.ifft()
+        Z.export_mpn(z.data_ptr(), 2 * n + 1)
+        fa.lib().fa_sync()
+
+    def whole():
+        fa.mpn_mul_device(z.data_ptr(), x.data_ptr(), n, y.data_ptr(), n)
+        fa.lib().fa_sync()
+    t = [_time(whole), _time(chain)]
+    assert t[1] < 1.65 * t[0]

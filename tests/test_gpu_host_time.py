@@ -40,7 +40,7 @@ def test_kept_transform(an):
     t = [_time(lambda: fa.nmod_poly_mul_mid(a, b, 0, 2 * an - 1, n)),
          _time(lambda: M.mul_mid(a, 0, 2 * an - 1))]
     M.close()
-    assert t[1] < 1.2 * t[0]
+    assert t[1] < 1.25 * t[0]
 
 
 def test_integer_product():
@@ -51,7 +51,7 @@ def test_integer_product():
     n = (1 << 61) - 1
     a, b = (rng.integers(0, n, 1000, dtype=np.uint64) for _ in range(2))
     t = [_time(lambda: fa.nmod_poly_mul_mid(a, b, 0, 1999, n)), _time(lambda: fa.mpn_mul(a, b))]
-    assert t[1] < 1.2 * t[0]
+    assert t[1] < 1.25 * t[0]
 
 
 @pytest.mark.parametrize("an,bn", [(1, 1), (1000, 1005), (60000, 50000), (700000, 500000)])

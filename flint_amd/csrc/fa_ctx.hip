@@ -485,9 +485,11 @@ void fa_buffers_idle(fa_thread_state* st) { st->last_stream = NULL; }
 // synchronization makes the runtime wait for a stream with more than eight
 // commands (uploads, kernels, the copy) by a callback on another thread, 20 to
 // 25 us; the synchronous copy waits for the device itself.  us, with an
-// asynchronous copy and a synchronization, and now: 1000 x 1005 limbs from the
-// host (2^11 points, two uploads and five kernels) 70 and 40, 65,536 x 65,536 173
-// and 147, a middle product with a kept transform of 2^12 points 84 and 51.
+// asynchronous copy and a synchronization, and now: 1000 x 1000 limbs from the
+// host (2^11 points, two uploads and five kernels) 68 and 39, 65,536 x 65,536 173
+// and 147, a middle product with a kept transform of 2^12 points 81 and 49;
+// shorter chains gain 10 us while they are small (nmod products of 100
+// coefficients 42 and 33, of 20,000 83 and 82).
 hipError_t fa_download(void* host, const void* dev, size_t bytes, hipStream_t s)
 {
     return bytes ? hipMemcpyWithStream(host, dev, bytes, hipMemcpyDeviceToHost, s)

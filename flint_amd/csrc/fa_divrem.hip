@@ -164,7 +164,10 @@ extern "C" int fa_nmod_poly_inv_series(uint64_t* g, const uint64_t* f, int64_t f
         return fa_set_error(FA_E_HIP, "upload failed");
     rc = inv_series_dev(dg.p, df.p, (uint64_t)fn, (uint64_t)m, mod, e.p, t.p, s);
     if (rc) return rc;
-    if (fa_download(g, dg.p, (uint64_t)m * 8, s) != hipSuccess)
+    // behind some sixty commands the asynchronous copy and a synchronization are
+    // the faster way: 234 us for 100 coefficients, 265 with fa_download
+    if (hipMemcpyAsync(g, dg.p, (uint64_t)m * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return FA_OK;
 }
@@ -192,8 +195,9 @@ extern "C" int fa_nmod_poly_divrem(uint64_t* q, uint64_t* r, const uint64_t* a, 
     if (rc) return rc;
     rc = divrem_dev(dq.p, dr.p, da.p, (uint64_t)an, db.p, (uint64_t)bn, dB.p, Bn, mod, dp.p, s);
     if (rc) return rc;
-    if (fa_download(q, dq.p, qn * 8, s) != hipSuccess ||
-        fa_download(r, dr.p, (uint64_t)(bn - 1) * 8, s) != hipSuccess)
+    if (hipMemcpyAsync(q, dq.p, qn * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipMemcpyAsync(r, dr.p, (uint64_t)(bn - 1) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return FA_OK;
 }
@@ -273,8 +277,9 @@ extern "C" int fa_nmod_poly_divrem_precomp(uint64_t* q, uint64_t* r, const uint6
     rc = divrem_dev(dq.p, dr.p, da.p, (uint64_t)an, M->b, M->bn, M->B + (M->Bn - qn), qn, mod,
                     dp.p, s);
     if (rc) return rc;
-    if (fa_download(q, dq.p, qn * 8, s) != hipSuccess ||
-        fa_download(r, dr.p, (M->bn - 1) * 8, s) != hipSuccess)
+    if (hipMemcpyAsync(q, dq.p, qn * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipMemcpyAsync(r, dr.p, (M->bn - 1) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
         return fa_set_error(FA_E_HIP, "download failed");
     return 1;
 }
